@@ -152,22 +152,119 @@ __global__ void mask_keys_kernel(const uint32_t* __restrict__ masks, int64_t n_o
   rows[p] = row;
 }
 
+// Tile order. A tile costs about its union mask's offsets, 10 to 27 on surfaces, and the
+// convolutions give XCD x the x-th eighth of the tiles (xcd_remap). Tiles that neighbour
+// each other in mask order cost alike, so on a 328k-voxel shell the heaviest eighth held
+// 1.8 times the work of the lightest, and heavy tiles that started last left CUs idle
+// besides. So pairs of tiles (the largest tile of the convolutions) are ranked by cost,
+// heaviest first, and dealt to the eighths in runs of kDealRun. Ranks are in steps of
+// four offsets and pairs of one rank stay in plan order, because neighbours share
+// gathered rows in an XCD's L2: with steps of one the 543k-voxel C128 layer ran 414 us
+// against 401 us in mask order, with steps of four 402 us; runs of 8 / 16 / 32 took
+// 818 / 812 / 794 us on the 328k-voxel res block and 3.06 / 2.97 / 3.09 ms on the fp32
+// C128 VAE block of that set, against 903 us and 3.72 ms in mask order. The C256 block
+// on 4.4M voxels went from 16.0 to 15.0 ms. Tables of few offsets are bound by their
+// rows' traffic and keep the plan order (the 8-slot pair: 135 us, ranked 138 us).
+constexpr int kPairRows = 2 * kTileRows;
+constexpr int kCostStep = 4;
+constexpr int kCosts = 32 / kCostStep + 1;
+constexpr int kOrderThreads = 512;
+constexpr int kDealRun = 16;
+constexpr int kOrderMinKvol = 9;
+constexpr int kOrderMinPairs = 64;  // fewer are all resident at once, in any order
+
+// costs[p] = offsets present in the union of pair p's masks, in steps (keys in plan order;
+// a mask key is a permutation of the mask's bits). One wave per pair.
+template <typename K>
+__global__ __launch_bounds__(256) void pair_cost_kernel(const K* __restrict__ keys, int64_t n_out, int mask_bits,
+                                                        int npairs, uint8_t* __restrict__ costs) {
+  const int pair = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (pair >= npairs) return;
+  uint32_t u = 0;
+#pragma unroll
+  for (int i = 0; i < kPairRows / 64; ++i) {
+    const int64_t p = static_cast<int64_t>(pair) * kPairRows + i * 64 + lane;
+    if (p < n_out) u |= static_cast<uint32_t>(keys[p]);
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) u |= __shfl_xor(u, d, 64);
+  if (mask_bits < 32) u &= (1u << mask_bits) - 1u;
+  if (lane == 0) costs[pair] = static_cast<uint8_t>(__popc(u) / kCostStep);
+}
+
+// position[p] = place of pair p: a stable counting sort by descending cost in one
+// workgroup (each thread a run of consecutive pairs), then the deal.
+__global__ __launch_bounds__(kOrderThreads) void pair_order_kernel(const uint8_t* __restrict__ costs, int npairs,
+                                                                   int32_t* __restrict__ position) {
+  __shared__ int32_t count[kCosts * kOrderThreads];  // [cost, descending][thread]
+  __shared__ int32_t part[kOrderThreads / 64];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int per = (npairs + kOrderThreads - 1) / kOrderThreads;
+  const int lo = min(t * per, npairs), hi = min(lo + per, npairs);
+  for (int c = 0; c < kCosts; ++c) count[c * kOrderThreads + t] = 0;
+  // eight of the run's costs at a time, their loads in flight together
+  auto each = [&](auto&& f) {
+    for (int p0 = lo; p0 < hi; p0 += 8) {
+      int c[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) c[i] = costs[min(p0 + i, hi - 1)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (p0 + i < hi) f(p0 + i, count[(kCosts - 1 - c[i]) * kOrderThreads + t]);
+    }
+  };
+  each([](int, int32_t& n) { ++n; });
+  __syncthreads();
+  // exclusive prefix over the flat counts: thread t sums entries [t * kCosts, + kCosts)
+  int32_t sum = 0;
+  for (int i = 0; i < kCosts; ++i) sum += count[t * kCosts + i];
+  int32_t x = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) part[w] = x;
+  __syncthreads();
+  int32_t run = x - sum;
+  for (int i = 0; i < w; ++i) run += part[i];
+  for (int i = 0; i < kCosts; ++i) {
+    const int32_t v = count[t * kCosts + i];
+    count[t * kCosts + i] = run;
+    run += v;
+  }
+  __syncthreads();
+  const int share = npairs / 8, rem = npairs % 8;
+  const int dealt = npairs - npairs % (8 * kDealRun);  // the rest one by one
+  each([&](int p, int32_t& n) {
+    const int r = n++;
+    const int run_no = r / kDealRun;
+    const int xcd = r < dealt ? run_no % 8 : (r - dealt) % 8;
+    const int at = r < dealt ? run_no / 8 * kDealRun + r % kDealRun : dealt / 8 + (r - dealt) / 8;
+    position[p] = xcd * share + min(xcd, rem) + at;
+  });
+}
+
 // One block of kTileRows threads per tile: output rows, transposed gather indices and
-// the union mask.
+// the union mask, written at the place of its pair (position; null: in plan order).
 __global__ __launch_bounds__(kTileRows) void tile_kernel(const int32_t* __restrict__ table, int64_t n_out,
                                                          int kvol, int64_t n_in,
                                                          const int32_t* __restrict__ order,
+                                                         const int32_t* __restrict__ position, int npairs,
                                                          int32_t* __restrict__ rows,
                                                          int32_t* __restrict__ gidx,
                                                          uint32_t* __restrict__ tile_mask) {
   __shared__ uint32_t wave_mask[kTileRows / 64];
   __shared__ int32_t staged[kTileRows * 32];
   __shared__ int32_t srow[kTileRows];
-  const int64_t tile = blockIdx.x;
   const int r = threadIdx.x;
-  const int64_t p = tile * kTileRows + r;
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * kTileRows + r;
+  const int pair = static_cast<int>(blockIdx.x >> 1);
+  // a last, partial pair stays last
+  const int64_t tile = position != nullptr && pair < npairs
+                           ? static_cast<int64_t>(position[pair]) * 2 + (blockIdx.x & 1) : blockIdx.x;
   const int32_t row = p < n_out ? order[p] : -1;
-  rows[p] = row;
+  rows[tile * kTileRows + r] = row;
   uint32_t mask = 0;
   int32_t* g = gidx + tile * kvol * kTileRows + r;
   const int32_t absent = static_cast<int32_t>(n_in);
@@ -291,19 +388,22 @@ int64_t sort_temp_bytes(int64_t n) { return radix::temp_bytes(std::max<int64_t>(
 // Sorts (keys, rows) on key bits [0, bits) with 32-bit keys when they fit, else 64-bit
 // ones; kbuf0 / kbuf1 hold n 64-bit keys each, rows start in r0. fill(k) launches the
 // kernel that writes the keys into k (uint32_t* or unsigned long long*) and the rows
-// into r0. *sorted receives the sorted rows (r0 or r1).
+// into r0. *sorted receives the sorted rows (r0 or r1), *sorted_keys the sorted keys.
 template <typename Fill>
 hipError_t sort_rows(void* temp, int64_t temp_bytes, unsigned long long* kbuf0, unsigned long long* kbuf1, int32_t* r0,
-                     int32_t* r1, int n, int bits, hipStream_t stream, Fill fill, const int32_t** sorted) {
+                     int32_t* r1, int n, int bits, hipStream_t stream, Fill fill, const int32_t** sorted,
+                     const void** sorted_keys = nullptr) {
   hipError_t e;
   if (bits <= 32) {
     auto* k0 = reinterpret_cast<uint32_t*>(kbuf0);
     auto* k1 = reinterpret_cast<uint32_t*>(kbuf1);
     fill(k0);
     e = radix::sort_pairs(temp, temp_bytes, k0, k1, r0, r1, n, 0, std::max(bits, 1), stream);
+    if (sorted_keys) *sorted_keys = k0;
   } else {
     fill(kbuf0);
     e = radix::sort_pairs(temp, temp_bytes, kbuf0, kbuf1, r0, r1, n, 0, bits, stream);
+    if (sorted_keys) *sorted_keys = kbuf0;
   }
   *sorted = r0;
   return e;
@@ -379,17 +479,33 @@ int hi3d_conv_plan(const int32_t* table, int64_t n_out, int32_t kvol, int64_t n_
     hipLaunchKernelGGL(mask_keys_kernel, dim3(blocks), dim3(256), 0, stream, mk, n_out, mask_bits, ord_in,
                        window_rows, k, ord_alt);
   };
+  const int64_t ntiles = ceil_div(n_out, kTileRows);
+  const int npairs = static_cast<int>(n_out / kPairRows);
+  int32_t* position = nullptr;
   if (mask_bits + window_bits > 0) {
     // mask in bits [0, mask_bits), window above it
+    const void* keys = nullptr;
     HI3D_HIP_CHECK(sort_rows(temp, temp_bytes, k0, k1, ord_alt, ord_in, n, mask_bits + window_bits, stream, fill,
-                             &final_order));
+                             &final_order, &keys));
+    if (mask_bits >= kOrderMinKvol && npairs >= kOrderMinPairs) {
+      // the row masks are used up: their space holds the costs and the positions
+      position = reinterpret_cast<int32_t*>(masks);
+      uint8_t* costs = reinterpret_cast<uint8_t*>(masks + npairs);
+      const dim3 grid(static_cast<unsigned>(ceil_div(npairs, 4)));
+      if (mask_bits + window_bits <= 32)
+        hipLaunchKernelGGL(pair_cost_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<const uint32_t*>(keys),
+                           n_out, mask_bits, npairs, costs);
+      else
+        hipLaunchKernelGGL(pair_cost_kernel<unsigned long long>, grid, dim3(256), 0, stream,
+                           static_cast<const unsigned long long*>(keys), n_out, mask_bits, npairs, costs);
+      hipLaunchKernelGGL(pair_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, costs, npairs, position);
+    }
   } else {
     fill(reinterpret_cast<uint32_t*>(k0));
     final_order = ord_alt;
   }
-  const int64_t ntiles = ceil_div(n_out, kTileRows);
   hipLaunchKernelGGL(tile_kernel, dim3(static_cast<unsigned>(ntiles)), dim3(kTileRows), 0, stream, table, n_out,
-                     kvol, n_in, final_order, rows, gidx, tile_mask);
+                     kvol, n_in, final_order, position, npairs, rows, gidx, tile_mask);
   HI3D_LAUNCH_CHECK();
   return HI3D_OK;
 }

@@ -257,6 +257,8 @@ int hi3d_conv_plan_workspace(int64_t n_out, int64_t* bytes_host);
  * are absent): output rows are ordered by Morton code of coords_dev (NULL = row
  * order), then grouped by their neighbour-presence mask within windows of
  * window_rows rows (0 = one window), and cut into tiles of hi3d_conv_tile_rows() rows.
+ * Pairs of tiles are then placed so that each eighth of the plan (an XCD's share) holds
+ * about the same work, heavy tiles first; a last pair that is not full stays last.
  * coord_bits (<= 19) and batch_bits (<= 7) bound the coordinates and batch indices
  * (< 2^bits) so that the Morton sort runs over 3 * coord_bits + batch_bits key bits;
  * 0 and 0 sort the full 64-bit key. Coordinates beyond the bits still give a valid

@@ -247,6 +247,32 @@ def test_plan_covers_every_row_once(cuda):
         assert np.array_equal(masks, exp)
 
 
+@pytest.mark.parametrize("n", [64 * 256 - 1, 64 * 256, 64 * 256 + 1, 64 * 256 + 129, 65 * 256, 128 * 256 + 255, 40001])
+def test_plan_tile_order(cuda, n):
+    """Around the sizes where pairs of tiles start to be ranked and dealt (64 pairs, whole
+    runs of 8 x 16 pairs, a last pair that is not full): every row once, the rows past the
+    end last, indices and masks of each tile its own rows', and from 64 pairs on no eighth
+    of them (an XCD's share) with more than 1.3 times the mean work."""
+    from hi3d_amd import kmap, workloads
+
+    idx = workloads.sphere_shell(128, 60.0, seed=2)[:n]
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [128] * 3, 1)
+    plan = km.plan()
+    rows = plan.rows.cpu().numpy()
+    assert np.array_equal(np.sort(rows[:n]), np.arange(n)) and (rows[n:] == -1).all()
+    table = km.table.cpu().numpy()
+    t = np.where(rows.reshape(-1, 128)[:, None, :] >= 0,
+                 table[np.maximum(rows, 0)].reshape(plan.ntiles, 128, 27).transpose(0, 2, 1), n)
+    assert np.array_equal(plan.gidx.view(plan.ntiles, 27, 128).cpu().numpy(), t)
+    masks = plan.tile_mask.cpu().numpy().astype(np.uint32)
+    assert np.array_equal(masks, ((t != n).any(2).astype(np.uint64) << np.arange(27, dtype=np.uint64)).sum(1))
+    pairs = masks[: plan.ntiles // 2 * 2].reshape(-1, 2)
+    work = np.array([bin(int(a | b)).count("1") for a, b in pairs])
+    shares = [s.sum() for s in np.array_split(work, 8)]
+    if n >= 64 * 256:  # the shares differ by at most a pair (1 in 8) and a step of cost
+        assert max(shares) <= 1.3 * np.mean(shares), shares
+
+
 def test_plan_work_on_shell_set(cuda):
     """The default plan of the 543k-voxel shell set (one mask-sorting window) runs at
     most 1.052 (row, offset) products per present pair in 128-row tiles: rows sorted by
