@@ -1,0 +1,513 @@
+// fp32 gather convolution on the bf16 matrix cores (gfx950): each fp32 operand as the sum
+// of three bf16 values.
+//
+//   out[o] = act(bias + sum_k in[gidx[o, k]] . W[:, k, :]^T) (+ residual[o])
+//
+// x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2), each
+// rounded to nearest: 24 bits, so the three hold every fp32 bit. Of the nine products
+// the kernel keeps w1 x1, w1 x2, w2 x1, w2 x2, w1 x3 and w3 x1; the others are below
+// 2^-25 of the product, under half an fp32 ulp. Products of two bf16 values are exact in
+// fp32 and the MFMA adds them to fp32 accumulators, as the fp32 MFMA does: the result
+// keeps fp32 accuracy at six 32x32x16 bf16 MFMAs in the place of eight 32x32x2 fp32 ones,
+// 192 cycles against 512. Relative error against 64-bit sums: C128, 327,581 voxels
+// 5.8e-7 (fp32 MFMA 6.7e-7), C64 4.2e-7 (5.0e-7), C256 8.5e-7 (9.8e-7): fewer roundings,
+// since one MFMA sums 16 products. What bounds it: the bf16 matrix rate. At C128 and
+// 327,581 voxels the six products of the 64-row tiles' offsets run at 1.06 PFLOP/s (a
+// large bf16 product of the library: 1.19).
+//
+// Infinities, NaN and values whose bf16 rounding overflows leave a sum that is not
+// finite (a part x2 or x3 of an infinity is NaN); such outputs are summed again in plain
+// fp32 in the epilogue, over the offsets their row has.
+//
+// Reference semantics: subm_conv (src/hi3d_mac/torch_backend/sparse_conv.py:152-195).
+#include <type_traits>
+
+#include "common.h"
+#include "conv_tile.h"
+
+namespace hi3d {
+namespace {
+
+constexpr int kSplitMaxKvol = 27;
+constexpr int kSplitMaxCin = 512;
+constexpr int kGroupThreads = 256;
+// Tables of few offsets (the strided pair, the child projection) are bound by their rows'
+// traffic until the products per row are many: the fp32 MFMA kernels ran the 64 -> 64
+// pair on 100k voxels in 52 us and the 128-channel child step on 200k parents in 897 us
+// against 56 and 934 us here; the 128 <-> 256 pair on 400k voxels took 653 us there and
+// 471 us here, the 256-channel child step 1790 and 1699 us.
+constexpr int kFewOffsets = 8;
+constexpr int64_t kFewOffsetsWork = 128 * 256;
+
+// row that absent neighbours read
+__device__ __attribute__((aligned(16))) const uint32_t g_split_zero_row[kSplitMaxCin] = {};
+
+struct SplitArgs {
+  const float* in;
+  int64_t n_in;
+  int32_t cin;
+  const char* packed;  // [kvol][cin / 16][col_blocks][3 parts][64 lanes][16 bytes]
+  int32_t col_blocks;  // 32-channel blocks of the packed weights (the last may be padding)
+  const float* weight;
+  int64_t wn, wk, wc;  // weight strides: output channel, offset, input channel
+  const float* bias;
+  int32_t cout;
+  int32_t kvol;
+  const int32_t* rows;
+  const int32_t* gidx;
+  int64_t n_out;
+  int32_t ny;  // column tiles
+  const float* residual;
+  int32_t act;
+  float* out;
+};
+
+// The three bf16 parts of 8 fp32 values.
+__device__ __forceinline__ void split8(const f32x4 lo, const f32x4 hi, bf16x8 (&p)[3]) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float a = j < 2 ? lo[2 * j] : hi[2 * j - 4], b = j < 2 ? lo[2 * j + 1] : hi[2 * j - 3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+      uint32_t u = __builtin_bit_cast(uint32_t, v);
+      asm("" : "+v"(u));  // one packed conversion, not another of each value alone
+      p[t][2 * j] = __builtin_bit_cast(bf16x2, u)[0];
+      p[t][2 * j + 1] = __builtin_bit_cast(bf16x2, u)[1];
+      if (t < 2) {
+        a -= __builtin_bit_cast(float, u << 16);
+        b -= __builtin_bit_cast(float, u & 0xffff0000u);
+      }
+    }
+  }
+}
+
+// One thread per 16-byte piece of a part: channel 32 nb + lane % 32, inputs
+// 16 ks + 8 (lane / 32) .. + 7, all three parts. Channels past cout are zero. vec: the
+// inputs of a channel lie next to each other and every 8 of them are 16-byte aligned.
+__global__ __launch_bounds__(256) void split_weight_kernel(const float* __restrict__ w, int64_t wn, int64_t wk,
+                                                           int64_t wc, bool vec, int cout, int cin, int col_blocks,
+                                                           int64_t total, char* __restrict__ packed) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (t >= total) return;
+  const int lane = static_cast<int>(t & 63);
+  const int64_t block = t >> 6;  // (k, ks, nb)
+  const int nb = static_cast<int>(block % col_blocks);
+  const int64_t kks = block / col_blocks;
+  const int ksteps = cin / 16;
+  const int ks = static_cast<int>(kks % ksteps);
+  const int64_t k = kks / ksteps;
+  const int n = nb * 32 + (lane & 31);
+  f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
+  if (n < cout) {
+    const float* src = w + n * wn + k * wk + (ks * 16 + 8 * (lane >> 5)) * wc;
+    if (vec) {
+      lo = *reinterpret_cast<const f32x4*>(src);
+      hi = *reinterpret_cast<const f32x4*>(src + 4);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lo[i] = src[i * wc];
+        hi[i] = src[(i + 4) * wc];
+      }
+    }
+  }
+  bf16x8 p[3];
+  split8(lo, hi, p);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(packed + block * 3072 + i * 1024 + lane * 16) = p[i];
+}
+
+// A workgroup owns BM plan rows and BN channels; its 4 G waves form G groups, each a 2 x 2
+// grid of waves over the whole tile that takes every G-th offset, so that a set of
+// few tiles spreads its chain of offsets over a CU's four SIMDs' worth of waves. The
+// groups' sums are added in order in the epilogue.
+//  * Stages (per group): (present offset, 16 KS inputs): BM gathered fp32 rows of 64 KS
+//    bytes and the packed weights' BN / 32 x KS x 3 KB, by direct-to-LDS 16-byte loads
+//    NS - 1 stages ahead into a ring of NS slots, one barrier a stage.
+//  * The weights' parts are laid out as the fragments are read (1 KB a wave-wide read);
+//    the rows stay fp32 in LDS and each wave splits its fragments in registers (11
+//    vector ops per pair of values).
+//  * The gather indices of all offsets reach LDS once, and with them the offsets that each
+//    32-row block has; a wave skips its blocks' products of the others.
+//  * The MFMAs take the weights as their first operand: a lane ends with four consecutive
+//    channels of one row. The output leaves through LDS as whole row pieces.
+template <int BM, int BN, int KS, int NS, int G>
+__global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitArgs a) {
+  constexpr int KV = kSplitMaxKvol, THREADS = kGroupThreads * G, NWG = kGroupThreads / 64, NW = NWG * G;  // waves of a group, of all
+  constexpr int WM = BM / 2, WN = BN / 2, MB = WM / 32, NB = WN / 32, RB = BM / 32;
+  constexpr int ROWB = 64 * KS;
+  constexpr int A_BYTES = BM * ROWB, B_BYTES = (BN / 32) * KS * 3072, STAGE = A_BYTES + B_BYTES;
+  constexpr int LA = A_BYTES / (1024 * NWG), BKB = B_BYTES / 1024;
+  constexpr int LB = (BKB + NWG - 1) / NWG, LBMIN = BKB / NWG;  // loads of the waves below BKB % NWG, of the others
+  static_assert(LA * 1024 * NWG == A_BYTES && (KS == 1 || KS == 2) && NS >= 2 && NS <= 4, "stage shape");
+  static_assert(BM % 64 == 0 && kTileRows % BM == 0, "a workgroup's rows lie in one plan tile");
+  constexpr int RING = G * NS * STAGE;
+  constexpr int OUTB = BN * 4, CPR = BN / 4;  // staged row: bytes, 16-byte chunks
+  static_assert(G * 64 * OUTB <= RING, "one row block of each wave, staged");
+  __shared__ __attribute__((aligned(16))) char smem[RING + (KV + 1) * BM * 4 + NW * RB * 4];
+  int32_t* const gl = reinterpret_cast<int32_t*>(smem + RING);
+  int32_t* const srow = gl + KV * BM;
+  uint32_t* const smask = reinterpret_cast<uint32_t*>(srow + BM);  // [wave][32-row block]
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave_all / NWG, wave = wave_all % NWG;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int64_t item = xcd_remap(blockIdx.x, static_cast<int64_t>(gridDim.x));
+  const int64_t tile = item / a.ny;
+  const int ct = static_cast<int>(item - tile * a.ny);
+  const int n0 = ct * BN;
+  const int kvol = a.kvol;
+  const uint64_t n_in = static_cast<uint64_t>(a.n_in);
+  const int64_t p0 = tile * BM;  // < ntiles * kTileRows
+  const int32_t* const gsrc = a.gidx + (p0 / kTileRows) * kvol * kTileRows + (p0 % kTileRows);
+
+  // gather indices of all offsets (-1: absent), this wave's offsets wave_all, + NW, ...
+  {
+    constexpr int PER = (KV + NW - 1) / NW;
+    int32_t g[PER][BM / 64];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int k = wave_all + NW * j;
+#pragma unroll
+      for (int h = 0; h < BM / 64; ++h) g[j][h] = gsrc[(k < kvol ? k : 0) * kTileRows + 64 * h + lane];
+    }
+    if (tid < BM) srow[tid] = a.rows[p0 + tid];
+    uint32_t m[RB] = {};
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int k = wave_all + NW * j;
+      if (k >= kvol) continue;
+#pragma unroll
+      for (int h = 0; h < BM / 64; ++h) {
+        const bool ok = static_cast<uint64_t>(static_cast<uint32_t>(g[j][h])) < n_in;
+        const uint64_t b = __builtin_amdgcn_ballot_w64(ok);
+        if (static_cast<uint32_t>(b) != 0) m[2 * h] |= 1u << k;
+        if (static_cast<uint32_t>(b >> 32) != 0) m[2 * h + 1] |= 1u << k;
+        gl[k * BM + 64 * h + lane] = ok ? g[j][h] : -1;
+      }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < RB; ++i) smask[wave_all * RB + i] = m[i];
+    }
+  }
+  __syncthreads();
+  uint32_t mask = 0, bmask[MB];  // offsets of the tile, of this wave's row blocks
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) bmask[mb] = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i) mask |= smask[w * RB + i];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) bmask[mb] |= smask[w * RB + wm * MB + mb];
+  }
+  mask = __builtin_amdgcn_readfirstlane(mask);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) bmask[mb] = __builtin_amdgcn_readfirstlane(bmask[mb]);
+
+  // this group's offsets k = group mod G, whatever the tile: a row's sum does not depend on
+  // the rows it shares a tile with (absent neighbours add zeros)
+  constexpr uint32_t EVERY = G == 4 ? 0x11111111u : 0xffffffffu;
+  static_assert(G == 1 || G == 4, "offset groups");
+  const uint32_t mine = mask & (EVERY << group);
+  int most = 0;
+#pragma unroll
+  for (int g = 0; g < G; ++g) most = max(most, __popc(mask & (EVERY << g)));
+  const int ksteps = a.cin / (16 * KS);  // stages per offset
+  const int S = __popc(mine) * ksteps;
+  const int SMAX = most * ksteps;  // barriers are the workgroup's
+  const int64_t row_bytes = static_cast<int64_t>(a.cin) * 4;
+  char* const ring = smem + group * (NS * STAGE);
+
+  // load u of this wave fills 1 KB of the stage's rows: 16 / KS rows, 4 KS lanes a row
+  constexpr int LPR = 4 * KS;
+  auto a_off = [](int row, int chunk) {
+    return KS == 1 ? row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4) : lds_offset(row, chunk);
+  };
+  int r_ld[LA], c_ld[LA];
+#pragma unroll
+  for (int u = 0; u < LA; ++u) {
+    r_ld[u] = (wave + NWG * u) * (64 / LPR) + lane / LPR;
+    const int c = lane % LPR;
+    c_ld[u] = (KS == 1 ? (c ^ ((r_ld[u] >> 2) & 3)) : (c ^ ((r_ld[u] >> 1) & 7))) * 16;
+  }
+  uint32_t rest = mine;
+  int lks = 0, lslot = 0;
+  const char* src[LA];
+  const char* wsrc = nullptr;
+  const int wstep = a.col_blocks * 3072;  // one 16-input step
+  int woff[LB];                           // KB wave + 4 u of a stage's weights
+#pragma unroll
+  for (int u = 0; u < LB; ++u) {
+    const int i = wave + NWG * u, s = i / (3 * (BN / 32));
+    woff[u] = s * wstep + (i - s * (3 * (BN / 32))) * 1024 + lane * 16;
+  }
+  auto issue = [&]() __attribute__((always_inline)) {
+    if (lks == 0) {
+      const int k = rest ? __builtin_ctz(rest) : 0;
+      rest &= rest - 1u;
+#pragma unroll
+      for (int u = 0; u < LA; ++u) {
+        const int32_t g = gl[k * BM + r_ld[u]];
+        uint64_t pin = reinterpret_cast<uint64_t>(a.in) + static_cast<uint64_t>(g * row_bytes);
+        asm volatile("" : "+v"(pin));  // a select of addresses, not a branch
+        src[u] = (g >= 0 ? reinterpret_cast<const char*>(pin) : reinterpret_cast<const char*>(g_split_zero_row)) + c_ld[u];
+      }
+      wsrc = a.packed + (static_cast<int64_t>(k) * ksteps * KS * a.col_blocks + ct * (BN / 32)) * 3072;
+    }
+    char* st = ring + lslot * STAGE;
+#pragma unroll
+    for (int u = 0; u < LA; ++u) lds_dma16(src[u] + lks * ROWB, st + (wave + NWG * u) * 1024);
+#pragma unroll
+    for (int u = 0; u < LB; ++u)
+      if (u < LBMIN || wave < BKB % NWG) lds_dma16(wsrc + woff[u], st + A_BYTES + (wave + NWG * u) * 1024);
+    wsrc += KS * wstep;
+    lslot = lslot == NS - 1 ? 0 : lslot + 1;
+    if (++lks == ksteps) lks = 0;
+  };
+
+  f32x16 acc[NB][MB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[nb][mb][v] = 0.0f;
+
+  uint32_t crest = mine;
+  int cks = 0, ck = mine ? __builtin_ctz(mine) : 0;  // the offset being multiplied
+  auto compute = [&](int slot) __attribute__((always_inline)) {
+    const char* st = ring + slot * STAGE;
+    uint32_t have = 0;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) have |= ((bmask[mb] >> ck) & 1u) << mb;
+    if (have != 0) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        bf16x8 w[NB][3];
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int t = 0; t < 3; ++t)
+            w[nb][t] = *reinterpret_cast<const bf16x8*>(
+                st + A_BYTES + ((s * (BN / 32) + wn * NB + nb) * 3 + t) * 1024 + lane * 16);
+        auto products = [&](auto first, auto count) __attribute__((always_inline)) {
+          constexpr int M0 = decltype(first)::value, MN = decltype(count)::value;
+          bf16x8 x[MN][3];
+#pragma unroll
+          for (int i = 0; i < MN; ++i) {
+            const int row = wm * WM + (M0 + i) * 32 + (lane & 31), c = 4 * s + 2 * (lane >> 5);
+            split8(*reinterpret_cast<const f32x4*>(st + a_off(row, c)),
+                   *reinterpret_cast<const f32x4*>(st + a_off(row, c + 1)), x[i]);
+          }
+          // small products first
+          constexpr int WP[6] = {2, 0, 1, 1, 0, 0}, XP[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+          for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+              for (int i = 0; i < MN; ++i)
+                acc[nb][M0 + i] =
+                    __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[nb][WP[t]], x[i][XP[t]], acc[nb][M0 + i], 0, 0, 0);
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        if constexpr (MB == 1) {
+          products(I0{}, I1{});
+        } else {
+          static_assert(MB == 2, "row blocks of a wave");
+          if (have == 3) products(I0{}, std::integral_constant<int, 2>{});
+          else if (have == 1) products(I0{}, I1{});
+          else products(I1{}, I1{});
+        }
+      }
+    }
+    if (++cks == ksteps) {
+      cks = 0;
+      crest &= crest - 1u;
+      ck = crest ? __builtin_ctz(crest) : 0;
+    }
+  };
+
+  // At the barrier of stage s every wave has its share of stage s in LDS and has read
+  // the fragments of stage s - 1, whose slot stage s + NS - 1 takes.
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (s < S) issue();
+  int slot = 0;
+  for (int s = 0; s < SMAX; ++s) {
+    constexpr int AHEAD = NS - 2;  // stages that may stay in flight
+    if (s + AHEAD < S) {
+      if (wave < BKB % NWG) wait_vmcnt<AHEAD * (LA + LB)>();
+      else wait_vmcnt<AHEAD * (LA + LBMIN)>();
+    } else {
+      wait_vmcnt<0>();
+    }
+    wait_lgkm0();
+    raw_barrier();
+    if (s + NS - 1 < S) issue();
+    if (s < S) compute(slot);
+    slot = slot == NS - 1 ? 0 : slot + 1;
+  }
+
+  // plain fp32 sum of one output, for sums that are not finite
+  auto plain = [&](int row, int n) {
+    float s = 0.0f;
+    for (int k = 0; k < kvol; ++k) {
+      const int32_t g = gl[k * BM + row];
+      if (g < 0) continue;
+      const float* x = a.in + static_cast<int64_t>(g) * a.cin;
+      const float* w = a.weight + n * a.wn + k * a.wk;
+      for (int c = 0; c < a.cin; ++c) s = fmaf(x[c], w[c * a.wc], s);
+    }
+    return s;
+  };
+  // one 32-row block of each wave at a time: [group][2 x 32 rows][BN], 16-byte chunk c of
+  // row r at c ^ (r % 16)
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) {
+    wait_lgkm0();
+    raw_barrier();
+    char* const stg = smem + (group * 64 + wm * 32 + (lane & 31)) * OUTB;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int chunk = (wn * WN + nb * 32 + 8 * q + 4 * (lane >> 5)) >> 2;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[nb][mb][4 * q + e];
+        *reinterpret_cast<f32x4*>(stg + ((chunk ^ (lane & 15)) << 4)) = v;
+      }
+    }
+    wait_lgkm0();
+    raw_barrier();
+    constexpr int PASS = 64 * CPR / THREADS;
+#pragma unroll
+    for (int i = 0; i < PASS; ++i) {
+      const int r = tid / CPR + (THREADS / CPR) * i, chunk = tid % CPR;
+      const int lrow = (r >> 5) * WM + mb * 32 + (r & 31);  // the tile's row
+      const int32_t orow = srow[lrow];
+      const int n = n0 + chunk * 4;
+      if (orow < 0 || orow >= a.n_out || n >= a.cout) continue;  // cout is a multiple of 4
+      f32x4 v = *reinterpret_cast<const f32x4*>(smem + r * OUTB + ((chunk ^ (r & 15)) << 4));
+#pragma unroll
+      for (int g = 1; g < G; ++g)
+        v += *reinterpret_cast<const f32x4*>(smem + (g * 64 + r) * OUTB + ((chunk ^ (r & 15)) << 4));
+      if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY)) {
+#pragma unroll 1
+        for (int e = 0; e < 4; ++e) {
+          const float y = plain(lrow, n + e);
+          v = f32x4{e == 0 ? y : v[0], e == 1 ? y : v[1], e == 2 ? y : v[2], e == 3 ? y : v[3]};
+        }
+      }
+      if (a.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += a.bias[n + e];
+      }
+      if (a.act == HI3D_ACT_SILU) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = silu_f32(v[e]);
+      }
+      const int64_t off = static_cast<int64_t>(orow) * a.cout + n;
+      if (a.residual != nullptr) v += *reinterpret_cast<const f32x4*>(a.residual + off);
+      *reinterpret_cast<f32x4*>(a.out + off) = v;
+    }
+  }
+}
+
+template <int BM, int BN, int KS, int NS, int G>
+int launch_split(const SplitArgs& base, hipStream_t stream) {
+  SplitArgs a = base;
+  a.ny = static_cast<int32_t>(ceil_div(a.cout, BN));
+  const int64_t blocks = ceil_div(a.n_out, BM) * a.ny;
+  HI3D_REQUIRE(blocks < (int64_t(1) << 31), "too many tiles");
+  hipLaunchKernelGGL((conv_split_kernel<BM, BN, KS, NS, G>), dim3(static_cast<unsigned>(blocks)), dim3(kGroupThreads * G), 0, stream, a);
+  HI3D_LAUNCH_CHECK();
+  return HI3D_OK;
+}
+
+// 32-channel blocks of the packed weights: whole column tiles.
+int col_blocks(int cout) { return cout % 128 == 0 ? cout / 32 : static_cast<int>(ceil_div(cout, 64)) * 2; }
+
+}  // namespace
+}  // namespace hi3d
+
+using namespace hi3d;
+
+extern "C" {
+
+int hi3d_gather_conv_f32_workspace(int32_t cin, int32_t cout, int32_t kvol, int64_t* bytes_host) {
+  HI3D_REQUIRE(bytes_host != nullptr, "null pointer argument");
+  HI3D_REQUIRE(cin > 0 && cout > 0 && kvol > 0, "channels and kvol must be positive");
+  const bool taken = kvol <= kSplitMaxKvol && cin <= kSplitMaxCin && cin % 32 == 0 && cout % 4 == 0 &&
+                     (kvol > kFewOffsets || static_cast<int64_t>(cin) * cout >= kFewOffsetsWork);
+  *bytes_host = taken ? static_cast<int64_t>(kvol) * (cin / 16) * col_blocks(cout) * 3072 : 0;
+  return HI3D_OK;
+}
+
+int hi3d_gather_conv_f32(const float* in, int64_t n_in, int32_t cin, const float* weight, int64_t stride_out,
+                         int64_t stride_offset, int64_t stride_in, const float* bias, int32_t cout, int32_t kvol,
+                         const int32_t* rows, const int32_t* gidx, int64_t n_out, const float* residual, int32_t act,
+                         float* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  int64_t need = 0;
+  if (const int e = hi3d_gather_conv_f32_workspace(cin, cout, kvol, &need)) return e;
+  HI3D_REQUIRE(need > 0, "gather conv f32 takes Cin a multiple of 32 up to %d, Cout a multiple of 4 and at most %d offsets",
+               kSplitMaxCin, kSplitMaxKvol);
+  HI3D_REQUIRE(n_in >= 0 && n_out >= 0, "sizes must be non-negative");
+  HI3D_REQUIRE(act == HI3D_ACT_NONE || act == HI3D_ACT_SILU, "unknown activation %d", act);
+  if (n_out == 0) return HI3D_OK;
+  HI3D_REQUIRE(in && weight && rows && gidx && out, "null pointer argument");
+  HI3D_REQUIRE(workspace != nullptr && workspace_bytes >= need, "workspace of %lld bytes needed", static_cast<long long>(need));
+  const uintptr_t align = reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out) |
+                          reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(workspace);
+  HI3D_REQUIRE((align & 15) == 0, "feature, residual, output and workspace pointers must be 16-byte aligned");
+  HI3D_REQUIRE(stride_out >= 0 && stride_offset >= 0 && stride_in >= 0, "weight strides must be non-negative");
+  const bool dense = stride_in == 1 && stride_offset == cin && stride_out == static_cast<int64_t>(cin) * kvol;
+  HI3D_REQUIRE((reinterpret_cast<uintptr_t>(weight) & (dense ? 15 : 3)) == 0, "the weight must be 16-byte aligned");
+  const bool vec = stride_in == 1 && stride_offset % 4 == 0 && stride_out % 4 == 0 &&
+                   (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
+  HI3D_REQUIRE((reinterpret_cast<uintptr_t>(bias) & 3) == 0, "the bias must be 4-byte aligned");
+  hipStream_t s = as_stream(stream);
+  SplitArgs a{};
+  a.in = in;
+  a.n_in = n_in;
+  a.cin = cin;
+  a.packed = static_cast<const char*>(workspace);
+  a.col_blocks = col_blocks(cout);
+  a.weight = weight;
+  a.wn = stride_out;
+  a.wk = stride_offset;
+  a.wc = stride_in;
+  a.bias = bias;
+  a.cout = cout;
+  a.kvol = kvol;
+  a.rows = rows;
+  a.gidx = gidx;
+  a.n_out = n_out;
+  a.residual = residual;
+  a.act = act;
+  a.out = out;
+  const int64_t total = need / 3 / 16;
+  hipLaunchKernelGGL(split_weight_kernel, dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0, s, weight, stride_out,
+                     stride_offset, stride_in, vec, cout, cin, a.col_blocks, total, static_cast<char*>(workspace));
+  HI3D_LAUNCH_CHECK();
+  // Shapes, against the fp32 MFMA kernels (one box, 3^3 maps): at most one 64 x 64 tile a
+  // CU runs four offset groups a workgroup (3,000 voxels C256: 465 -> 93 us, one group
+  // 141; 8,000 voxels C64: 40 -> 30, one group 43; where a CU has two or three tiles one
+  // group is faster, 20,000 voxels C128: 120 with four, 107 with one). Whole 128-channel
+  // tiles read each gathered row once per 128 channels (327,581 voxels C128: 1307 ->
+  // 805 us, 64-channel tiles 870, 128-row tiles with half the weight reads 808); the
+  // others two stages in 48 KB, so that three workgroups share a CU (45,128 voxels C64:
+  // 78 -> 61 us, three slots and two workgroups 84).
+  if (ceil_div(n_out, 64) * ceil_div(cout, 64) <= compute_units()) return launch_split<64, 64, 1, 2, 4>(a, s);
+  if (cout % 128 == 0) return launch_split<64, 128, 2, 2, 1>(a, s);
+  return launch_split<64, 64, 2, 2, 1>(a, s);
+}
+
+}  // extern "C"

@@ -49,6 +49,9 @@ _SIGNATURES = {
     "hi3d_conv_plan_workspace": [_i64, _p],
     "hi3d_conv_plan": [_p, _i64, _i32, _i64, _p, _i32, _i32, _i64, _p, _i64, _p, _p, _p, _p],
     "hi3d_gather_conv": [_p, _i64, _i32, _p, _p, _i32, _i32, _p, _p, _p, _i64, _p, _i32, _i32, _p, _p],
+    "hi3d_gather_conv_f32_workspace": [_i32, _i32, _i32, _p],
+    "hi3d_gather_conv_f32": [_p, _i64, _i32, _p, _i64, _i64, _i64, _p, _i32, _i32, _p, _p, _i64, _p, _i32, _p, _p,
+                             _i64, _p],
     "hi3d_gather_conv_ln_silu": [_p, _i64, _i32, _p, _p, _i32, _i32, _p, _p, _p, _i64, _p, _i32, _p, _p, _f32, _p,
                                  _p],
     "hi3d_gather_conv_simple": [_p, _i64, _i32, _p, _p, _i32, _i32, _p, _i64, _p, _i32, _i32, _p, _p],

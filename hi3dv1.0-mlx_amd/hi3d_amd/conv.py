@@ -49,12 +49,17 @@ def halo_supported(dtype: torch.dtype, cin: int, cout: int, kvol: int) -> bool:
     return cout % 128 == 0 and rb % 64 == 0 and 256 <= rb <= 512
 
 
-def _flat_weight(weight: torch.Tensor, kvol: int) -> torch.Tensor:
+def _weight_view(weight: torch.Tensor, kvol: int) -> torch.Tensor:
+    """``weight`` as ``[Cout, kvol, Cin]`` (a view where its strides allow one)."""
     cout, cin = int(weight.shape[0]), int(weight.shape[-1])
     w = weight.reshape(cout, -1, cin)
     if w.shape[1] != kvol:
         raise ValueError(f"weight has {w.shape[1]} kernel offsets, the map has {kvol}")
-    return w.contiguous()
+    return w
+
+
+def _flat_weight(weight: torch.Tensor, kvol: int) -> torch.Tensor:
+    return _weight_view(weight, kvol).contiguous()
 
 
 def mfma_supported(dtype: torch.dtype, cin: int, cout: int) -> bool:
@@ -63,6 +68,13 @@ def mfma_supported(dtype: torch.dtype, cin: int, cout: int) -> bool:
         return False
     es = torch.empty((), dtype=dtype).element_size()
     return (cin * es) % 16 == 0 and (cout * es) % 16 == 0
+
+
+@functools.lru_cache(maxsize=1024)
+def split_workspace(cin: int, cout: int, kvol: int) -> int:
+    """Workspace bytes of the fp32 convolution on the bf16 matrix cores
+    (``hi3d_gather_conv_f32``); 0 where it does not take the shape."""
+    return _lib.query("hi3d_gather_conv_f32_workspace", cin, cout, kvol)
 
 
 def gather_conv(
@@ -84,7 +96,7 @@ def gather_conv(
     if features.ndim != 2 or features.shape[0] != plan.n_in:
         raise ValueError(f"expected features [{plan.n_in}, Cin], got {tuple(features.shape)}")
     x = features.contiguous()
-    w = _flat_weight(weight, plan.kvol)
+    w = _weight_view(weight, plan.kvol)
     cin, cout = int(x.shape[1]), int(w.shape[0])
     if int(w.shape[2]) != cin:
         raise ValueError(f"weight expects {int(w.shape[2])} input channels, features have {cin}")
@@ -97,6 +109,7 @@ def gather_conv(
     out = _output(out, plan.n_out, cout, dtype, device)
     hp = plan.halo() if HALO and halo_supported(dtype, cin, cout, plan.kvol) else None
     if hp is not None:
+        w = w.contiguous()
         _lib.call(
             "hi3d_halo_conv",
             _lib.ptr(x), plan.n_in, cin, _lib.ptr(w), _lib.ptr(b), cout, _lib.ptr(hp.rows), _lib.ptr(hp.halo),
@@ -104,6 +117,17 @@ def gather_conv(
             _lib.stream(device),
         )
         return out
+    split = split_workspace(cin, cout, plan.kvol) if dtype == torch.float32 else 0
+    if split:
+        ws = _lib.workspace(split, device)  # the weight's bf16 parts, whatever its strides
+        _lib.call(
+            "hi3d_gather_conv_f32",
+            _lib.ptr(x), plan.n_in, cin, _lib.ptr(w), *w.stride(), _lib.ptr(b), cout, plan.kvol, _lib.ptr(plan.rows),
+            _lib.ptr(plan.gidx), plan.n_out, _lib.ptr(r), ACTIVATIONS[act], _lib.ptr(out), _lib.ptr(ws), split,
+            _lib.stream(device),
+        )
+        return out
+    w = w.contiguous()
     _lib.call(
         "hi3d_gather_conv",
         _lib.ptr(x), plan.n_in, cin, _lib.ptr(w), _lib.ptr(b), cout, plan.kvol, _lib.ptr(plan.rows),

@@ -87,7 +87,7 @@ def conv_gn_swish(x: torch.Tensor, level: Level, norm_weight: torch.Tensor, norm
     wdt = weight_t.dtype
     a = group_norm_swish(x, mean, inv, norm_weight, norm_bias, wdt)
     cin, cout = int(x.shape[1]), int(weight_t.shape[1])
-    w = weight_t.T.reshape(cout, 27, cin).contiguous()
+    w = weight_t.T.reshape(cout, 27, cin)
     if out is None:
         out = torch.float32 if wdt == torch.float32 else wdt
     donated = None

@@ -287,6 +287,23 @@ int hi3d_gather_conv(const void* in_dev, int64_t n_in, int32_t cin, const void* 
                      const void* residual_dev, int32_t act, int32_t dtype, void* out_dev,
                      void* stream);
 
+/* Workspace bytes of hi3d_gather_conv_f32 for these shapes; 0 where it does not take
+ * them (use hi3d_gather_conv): it takes Cin a multiple of 32 up to 512, Cout a multiple
+ * of 4 and at most 27 offsets, with at most 8 offsets only Cin * Cout >= 32768. */
+int hi3d_gather_conv_f32_workspace(int32_t cin, int32_t cout, int32_t kvol, int64_t* bytes_host);
+
+/* hi3d_gather_conv in fp32 on the bf16 matrix cores: each operand as the sum of three
+ * bf16 values, six of the nine products, fp32 accumulation. The error against 64-bit sums
+ * is that of fp32 sums; sums that are not finite are formed in plain fp32. The weight is
+ * read through its element strides (output channel, offset, input channel; a dense one
+ * 16-byte aligned) and its parts are laid out in the workspace, 16-byte aligned and the
+ * call's own until it has run. */
+int hi3d_gather_conv_f32(const float* in_dev, int64_t n_in, int32_t cin, const float* weight_dev,
+                         int64_t stride_out, int64_t stride_offset, int64_t stride_in,
+                         const float* bias_dev, int32_t cout, int32_t kvol, const int32_t* rows_dev,
+                         const int32_t* gidx_dev, int64_t n_out, const float* residual_dev, int32_t act,
+                         float* out_dev, void* workspace_dev, int64_t workspace_bytes, void* stream);
+
 /* hi3d_gather_conv (fp16, no activation, no residual) into 128 output channels with the
  * transformer res block's second norm applied to each output row before it is stored:
  * h = conv row (fp16), then LayerNorm over its 128 channels (fp32 two-pass statistics,

@@ -271,6 +271,82 @@ def test_fp32_block_kernel(cuda, side, density, batch, kvol, act, res):
     assert torch.equal(y, y2)
 
 
+def _rel_rms(y, ref):
+    return float(np.sqrt(((y.astype(np.float64) - ref) ** 2).mean() / (ref ** 2).mean()))
+
+
+@pytest.mark.parametrize("cin,cout,density,side,act,res", [
+    (32, 20, 0.15, 16, None, False),      # 20 of a 64-channel tile's outputs, four offset groups
+    (32, 36, 0.3, 40, "silu", True),      # one group, outputs past Cout in the packed weights
+    (64, 64, 0.2, 48, None, True),        # the 64-channel tiles
+    (96, 160, 0.01, 64, "silu", False),   # few neighbours: groups and blocks without offsets
+    (128, 128, 0.25, 40, None, True),     # the 128-channel tiles
+    (512, 256, 0.2, 24, None, False),     # the longest rows
+])
+def test_fp32_split_kernel(cuda, cin, cout, density, side, act, res):
+    """The fp32 convolution on the bf16 matrix cores, every tile shape of its dispatch:
+    against float64, with no larger error than the fp32 matrix cores' (both entry points
+    on the same inputs; values spread over 2^-20 .. 2^20, so that the low parts count),
+    a strided weight (the transposed layout) bitwise the dense one, and each row's sum
+    independent of the tile order."""
+    from hi3d_amd import _lib, conv, kmap
+
+    rng = np.random.default_rng(cin + 7 * cout)
+    idx = _rand_indices(rng, side, density)
+    n = len(idx)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    x, w, b = _case(rng, n, cin, cout, torch.float32)
+    x *= torch.as_tensor(np.exp2(rng.integers(-20, 21, (1, cin))).astype(np.float32))
+    r = torch.as_tensor(rng.standard_normal((n, cout), dtype=np.float32)) if res else None
+    xd, wd, bd = x.to(cuda), w.to(cuda), b.to(cuda)
+    rd = None if r is None else r.to(cuda)
+    assert conv.split_workspace(cin, cout, 27) > 0
+    plan = km.plan()
+    y = conv.gather_conv(xd, plan, wd, bd, act=act, residual=rd)
+    ref = oconv.gather_conv_f64(x.numpy(), km.table.cpu().numpy(), w.numpy(), b.numpy(), act=act,
+                                residual=None if r is None else r.numpy())
+    z = torch.empty_like(y)
+    _lib.call("hi3d_gather_conv", _lib.ptr(xd), n, cin, _lib.ptr(wd), _lib.ptr(bd), cout, 27, _lib.ptr(plan.rows),
+              _lib.ptr(plan.gidx), _lib.ptr(plan.tile_mask), n, _lib.ptr(rd), conv.ACTIVATIONS[act],
+              _lib.DTYPES[torch.float32], _lib.ptr(z), _lib.stream(xd.device))
+    # 5 %: the two sums' roundings are independent samples over these few outputs
+    assert _rel_rms(y.cpu().numpy(), ref) <= 1.05 * _rel_rms(z.cpu().numpy(), ref)
+    assert oconv.rel_err(y.cpu().numpy(), ref) <= (2e-5 if cin > 256 else GATE[torch.float32])
+    wt = wd.permute(1, 2, 0).contiguous().permute(2, 0, 1)
+    assert torch.equal(conv.gather_conv(xd, plan, wt, bd, act=act, residual=rd), y)
+    y2 = conv.gather_conv(xd, kmap.build_plan(km.table, n, window_rows=64), wd, bd, act=act, residual=rd)
+    assert torch.equal(y, y2)
+
+
+def test_fp32_split_kernel_not_finite(cuda):
+    """Infinities, NaN and values past bf16's largest, in the features and in the weights:
+    where the sum over a row's present neighbours is infinite or NaN so is the output,
+    with the sign, and every other output keeps fp32 accuracy."""
+    from hi3d_amd import conv, kmap
+
+    rng = np.random.default_rng(11)
+    idx = _rand_indices(rng, 24, 0.05)
+    n = len(idx)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [24] * 3, 1)
+    x, w, b = _case(rng, n, 64, 64, torch.float32)
+    x[5, 3], x[17, 0], x[40, 63], x[60, 9] = np.inf, -np.inf, np.nan, 3.4028e38
+    w[7, 13, 5], w[9, 2, 1] = np.inf, 3.4e38
+    y = conv.gather_conv(x.to(cuda), km.plan(), w.to(cuda), b.to(cuda)).cpu().numpy()
+    table = km.table.cpu().numpy()
+    with np.errstate(all="ignore"):
+        ref = b.double().numpy()[None].repeat(n, 0)
+        for k in range(27):
+            to = np.nonzero(table[:, k] < n)[0]
+            # one product at a time: a matrix product may form inf - inf in another order
+            ref[to] += (x.double().numpy()[table[to, k]][:, None] * w.double().numpy()[None, :, k]).sum(2)
+    big = np.isfinite(ref) & (np.abs(ref) > 1e36)  # may overflow in fp32
+    fine = np.isfinite(ref) & (np.abs(ref) < 1e6)
+    assert np.array_equal(np.isnan(ref), np.isnan(y))
+    assert np.array_equal(y[np.isinf(ref)], ref[np.isinf(ref)].astype(np.float32))
+    assert (~np.isnan(y[big])).all() and fine.mean() > 0.9
+    assert np.abs(y[fine] - ref[fine]).max() <= 1e-5 * np.sqrt((ref[fine] ** 2).mean())
+
+
 @pytest.mark.parametrize("dtype,mode", [
     (torch.float16, "one"), (torch.float16, "mixed"), (torch.bfloat16, "mixed"), (torch.float16, "blocks"),
 ])
