@@ -13,8 +13,8 @@ namespace hi3d {
 namespace {
 
 // ------------------------------------------------------------------ quantiser --
-// One wave per row, grid-stride over rows, the next row's fp16 data loaded while the
-// current one is computed. Pass p covers columns [1024p, 1024p + 1024): lane l holds the
+// Up to 2048 columns one wave per row, grid-stride over rows, the next row's fp16 data
+// loaded while the current one is computed. Pass p covers columns [1024p, 1024p + 1024): lane l holds the
 // 16 consecutive columns 1024p + 16l .. +15, i.e. positions 16(l%4) .. +15 of 64-column
 // block 16p + l/4. Hadamard butterflies run over position bits 0..5 in increasing
 // order, the same order as the reference's lane shuffles (bits 0..4) followed by its
@@ -25,19 +25,22 @@ namespace {
 // compiler's own correctly rounded f32 division sequence, its reciprocal refinement
 // hoisted per row (quant_div); rows with a non-finite scale use the full division.
 // The multipliers (signs) sit in LDS, loaded once per workgroup.
+// kBlock (wider rows): a workgroup per row, wave w taking passes w, w + 4, ... (NP of them),
+// so that a row stays in registers and a set of few rows spreads over four times the waves.
 constexpr int kQuantCols = 1024;  // columns per pass
 
-template <int NP, bool kRotate, bool kFull>
+template <int NP, bool kRotate, bool kFull, bool kBlock>
 __global__ __launch_bounds__(256) void quant_kernel(const _Float16* __restrict__ x, int64_t m, int k,
                                                     const float* __restrict__ signs, int8_t* __restrict__ q,
                                                     float* __restrict__ scale) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) float mult[];  // k multipliers when rotating
-  constexpr bool kHold = NP <= 8;      // row held in registers (else recomputed)
-  constexpr bool kPrefetch = NP <= 4;  // and the next row's loads in flight meanwhile
-  const int lane = threadIdx.x & 63;
-  const int64_t first = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 4;
+  static_assert(!kBlock || !kFull, "a wave's last pass may lie past the row");
+  constexpr bool kPrefetch = !kBlock;  // the next row's loads in flight while one is computed
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t first = kBlock ? static_cast<int64_t>(blockIdx.x) : static_cast<int64_t>(blockIdx.x) * 4 + wave;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * (kBlock ? 1 : 4);
+  auto column = [&](int p) { return (kBlock ? wave + 4 * p : p) * kQuantCols + lane * 16; };
   if constexpr (kRotate) {
     for (int i = threadIdx.x * 4; i < k; i += 1024)
       *reinterpret_cast<float4*>(mult + i) = *reinterpret_cast<const float4*>(signs + i);
@@ -49,13 +52,13 @@ __global__ __launch_bounds__(256) void quant_kernel(const _Float16* __restrict__
   using Raw = f16x8[2];
   auto load_raw = [&](int64_t row, int p, Raw& h) {
     const _Float16* xr = x + row * k;
-    const int c0 = p * kQuantCols + lane * 16;
+    const int c0 = column(p);
     h[0] = *reinterpret_cast<const f16x8*>(xr + (kFull || c0 < k ? c0 : 0));
     h[1] = *reinterpret_cast<const f16x8*>(xr + (kFull || c0 + 8 < k ? c0 + 8 : 0));
   };
   // this lane's 16 values of pass p, rotated (unscaled) when kRotate; zeros past k
   auto rotate = [&](int p, const Raw& h, float (&v)[16]) {
-    const int c0 = p * kQuantCols + lane * 16;
+    const int c0 = column(p);
     const bool ok0 = kFull || c0 < k, ok1 = kFull || c0 + 8 < k;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -101,93 +104,77 @@ __global__ __launch_bounds__(256) void quant_kernel(const _Float16* __restrict__
 #pragma unroll
       for (int e = 0; e < 16; ++e) v[e] = v[e] / t;
     }
-    const int c0 = p * kQuantCols + lane * 16;
+    const int c0 = column(p);
     uint32_t w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) w[j] = quant_pack4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
     if (c0 + 8 < k) *reinterpret_cast<uint4*>(qr + c0) = make_uint4(w[0], w[1], w[2], w[3]);
     else if (c0 < k) *reinterpret_cast<uint2*>(qr + c0) = make_uint2(w[0], w[1]);
   };
+  __shared__ float wave_max[kBlock ? 8 : 1];
+  int turn = 0;
   // the row's scale (written out) and the divisor of its values
   auto finish_scale = [&](int64_t row, float maximum, float& t, float& r, bool& fast) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, d, 64));
+    if constexpr (kBlock) {
+      // two sets of slots by turns: a wave writes a set again only after the barrier of
+      // the row between, which follows every wave's reads of it
+      float* const part = wave_max + 4 * (turn & 1);
+      ++turn;
+      if (lane == 0) part[wave] = maximum;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) maximum = fmaxf(maximum, part[i]);
+    }
     float s;
     const QuantDivisor dv = quant_divisor<kRotate>(maximum, s);
-    if (lane == 0) scale[row] = s;
+    if (lane == 0 && (!kBlock || wave == 0)) scale[row] = s;
     t = dv.t;
     r = dv.r;
     fast = dv.fast;
   };
 
-  if constexpr (kHold) {
-    // rows alternate between two register buffers: while one row is computed, the
-    // next one's loads are in flight
-    auto process = [&](int64_t row, Raw (&cur)[NP]) {
-      float v[NP][16];
-      float maximum = 0.0f;
-      // columns past k hold zeros (whole 64-column blocks when rotating), which leave
-      // the maximum of absolute values unchanged
+  // rows alternate between two register buffers: while one row is computed, the
+  // next one's loads are in flight
+  auto process = [&](int64_t row, Raw (&cur)[NP]) {
+    float v[NP][16];
+    float maximum = 0.0f;
+    // columns past k hold zeros (whole 64-column blocks when rotating), which leave
+    // the maximum of absolute values unchanged
 #pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        rotate(p, cur[p], v[p]);
+    for (int p = 0; p < NP; ++p) {
+      rotate(p, cur[p], v[p]);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) maximum = fmaxf(maximum, fabsf(v[p][e]));
-      }
-      float t, r;
-      bool fast;
-      finish_scale(row, maximum, t, r, fast);
-      int8_t* qr = q + row * k;
+      for (int e = 0; e < 16; ++e) maximum = fmaxf(maximum, fabsf(v[p][e]));
+    }
+    float t, r;
+    bool fast;
+    finish_scale(row, maximum, t, r, fast);
+    int8_t* qr = q + row * k;
 #pragma unroll
-      for (int p = 0; p < NP; ++p) store_pass(qr, p, v[p], t, r, fast);
-    };
-    auto load_row = [&](int64_t row, Raw (&buf)[NP]) {  // rows past m load row m - 1
-      const int64_t rr = row < m ? row : m - 1;
+    for (int p = 0; p < NP; ++p) store_pass(qr, p, v[p], t, r, fast);
+  };
+  auto load_row = [&](int64_t row, Raw (&buf)[NP]) {  // rows past m load row m - 1
+    const int64_t rr = row < m ? row : m - 1;
 #pragma unroll
-      for (int p = 0; p < NP; ++p) load_raw(rr, p, buf[p]);
-    };
-    if constexpr (kPrefetch) {
-      Raw a[NP], b[NP];
-      load_row(first, a);
-      for (int64_t row = first; row < m; row += 2 * stride) {
-        load_row(row + stride, b);
-        process(row, a);
-        if (row + stride >= m) break;
-        load_row(row + 2 * stride, a);
-        process(row + stride, b);
-      }
-    } else {
-      for (int64_t row = first; row < m; row += stride) {
-        Raw a[NP];
-        load_row(row, a);
-        process(row, a);
-      }
+    for (int p = 0; p < NP; ++p) load_raw(rr, p, buf[p]);
+  };
+  if constexpr (kPrefetch) {
+    Raw a[NP], b[NP];
+    load_row(first, a);
+    for (int64_t row = first; row < m; row += 2 * stride) {
+      load_row(row + stride, b);
+      process(row, a);
+      if (row + stride >= m) break;
+      load_row(row + 2 * stride, a);
+      process(row + stride, b);
     }
   } else {
-    // wide rows: a first pass for the maximum, a second that recomputes and stores
     for (int64_t row = first; row < m; row += stride) {
-      float maximum = 0.0f;
-#pragma unroll 1
-      for (int p = 0; p < NP; ++p) {
-        Raw h;
-        float v[16];
-        load_raw(row, p, h);
-        rotate(p, h, v);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) maximum = fmaxf(maximum, fabsf(v[e]));
-      }
-      float t, r;
-      bool fast;
-      finish_scale(row, maximum, t, r, fast);
-      int8_t* qr = q + row * k;
-#pragma unroll 1
-      for (int p = 0; p < NP; ++p) {
-        Raw h;
-        float v[16];
-        load_raw(row, p, h);
-        rotate(p, h, v);
-        store_pass(qr, p, v, t, r, fast);
-      }
+      Raw a[NP];
+      load_row(row, a);
+      process(row, a);
     }
   }
 }
@@ -467,6 +454,183 @@ __global__ __launch_bounds__(256, 1) void w8a8_gemm_kernel(const int8_t* __restr
     } else {
       const _Float16* pv = reinterpret_cast<const _Float16*>(&v);
       for (int e = 0; e < 8 && col + e < n; ++e) out[row * n + col + e] = pv[e];
+    }
+  }
+}
+
+// Few tiles: 16 waves share a BM x BN tile in G groups of WM x WN waves, group g taking the
+// K stages s = g mod G, each through its own ring of NS stages of 128 bytes of K; the
+// groups' int32 sums meet in LDS (exact in any order). A launch whose 256 x 256 tiles
+// leave CUs idle spends its time in one tile's chain of K stages: smaller tiles fill the
+// CUs and the groups shorten the chain.
+template <int BM, int BN, int WM, int WN, int NS, int G, int KB>
+__global__ __launch_bounds__(64 * WM * WN * G, 1) void w8a8_gemm_few_kernel(
+    const int8_t* __restrict__ qa, const float* __restrict__ sa, const int8_t* __restrict__ w,
+    const float* __restrict__ sw, const _Float16* __restrict__ bias, int64_t m, int n, int k,
+    _Float16* __restrict__ out, int32_t* __restrict__ acc_out, int ntiles) {
+#pragma clang fp contract(off)
+  constexpr int NWG = WM * WN, THREADS = 64 * NWG * G;
+  constexpr int MB = BM / WM / 32, NB = BN / WN / 32;  // 32 x 32 blocks of a wave
+  constexpr int STAGE = (BM + BN) * KB, CH = KB / 16;  // 16-byte chunks of a stage's row
+  static_assert(KB == 64 || KB == 128, "bytes of K per stage");
+  auto row_off = [](int r, int c) { return KB == 64 ? lds_off64(r, c) : lds_offset(r, c); };
+  auto chunk_of = [](int r, int c) { return KB == 64 ? c ^ ((r >> 2) & 3) : c ^ ((r >> 1) & 7); };
+  constexpr int L = STAGE / 1024 / NWG;  // direct-to-LDS loads per wave and stage
+  static_assert(L * NWG * 1024 == STAGE && NS >= 2, "stage shape");
+  constexpr int RING = G * NS * STAGE;
+  constexpr int ROW = BN * 4 + 16;  // accumulator rows: their lanes' writes spread over the banks
+  constexpr int SMEM = RING > BM * ROW ? RING : BM * ROW;
+  __shared__ __attribute__((aligned(16))) char smem[SMEM];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = wave_all / NWG, wave = wave_all % NWG;
+  const int wm = wave / WN, wn = wave % WN;
+  const int64_t item = xcd_remap(blockIdx.x, static_cast<int64_t>(gridDim.x));
+  const int64_t mt = item / ntiles;
+  const int nt = static_cast<int>(item - mt * ntiles);
+  const int64_t m0 = mt * BM;
+  const int n0 = nt * BN;
+  char* const ring = smem + group * (NS * STAGE);
+
+  // load u fills stage rows (wave + NWG u) * 64 / CH + lane / CH (tokens, then channels); rows
+  // past the matrix re-read its last row (their results are not stored)
+  const int8_t* src[L];
+#pragma unroll
+  for (int u = 0; u < L; ++u) {
+    const int r = (wave + NWG * u) * (64 / CH) + lane / CH;
+    const int c = chunk_of(r, lane % CH) * 16;
+    if (r < BM) {
+      src[u] = qa + (m0 + r < m ? m0 + r : m - 1) * k + c;
+    } else {
+      const int j = n0 + r - BM;
+      src[u] = w + static_cast<int64_t>(j < n ? j : n - 1) * k + c;
+    }
+  }
+  const int stages = (k + KB - 1) / KB;
+  // (with 128-byte stages the second half of the last one is zeros where K = 64 mod 128)
+  const int S = (stages - group + G - 1) / G;  // this group's (may be 0)
+  const int SMAX = (stages + G - 1) / G;
+  auto issue = [&](int i) __attribute__((always_inline)) {
+    char* st = ring + (i % NS) * STAGE;
+    const int off = (i * G + group) * KB;
+    if (KB == 64 || off + KB <= k) {
+#pragma unroll
+      for (int u = 0; u < L; ++u) lds_dma16(src[u] + off, st + (wave + NWG * u) * 1024);
+    } else {
+#pragma unroll
+      for (int u = 0; u < L; ++u) {
+        const int r = (wave + NWG * u) * (64 / CH) + lane / CH;
+        const bool past = chunk_of(r, lane % CH) >= 4;
+        lds_dma16(past ? static_cast<const void*>(g_zero_chunk) : static_cast<const void*>(src[u] + off),
+                  st + (wave + NWG * u) * 1024);
+      }
+    }
+  };
+  i32x16 acc[NB][MB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[nb][mb][v] = 0;
+  // every fragment of a stage is read before its first product, and the next loads are
+  // issued in between, so that neither latency is paid per K-group
+  i32x4 fq[KB / 32][MB], fw[KB / 32][NB];
+  auto frags = [&](int i) __attribute__((always_inline)) {
+    const char* st = ring + (i % NS) * STAGE;
+#pragma unroll
+    for (int g = 0; g < KB / 32; ++g) {
+      const int c = 2 * g + (lane >> 5);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        fq[g][mb] = *reinterpret_cast<const i32x4*>(st + row_off((wm * MB + mb) * 32 + (lane & 31), c));
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        fw[g][nb] = *reinterpret_cast<const i32x4*>(st + row_off(BM + (wn * NB + nb) * 32 + (lane & 31), c));
+    }
+  };
+  auto products = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < KB / 32; ++g)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          acc[nb][mb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw[g][nb], fq[g][mb], acc[nb][mb], 0, 0, 0);
+  };
+  // at the barrier of stage i every wave has its share of stage i in LDS and has read the
+  // fragments of stage i - 1, whose slot stage i + NS - 1 takes
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (i < S) issue(i);
+  for (int i = 0; i < SMAX; ++i) {
+    if (i + NS - 2 < S) wait_vmcnt<(NS - 2) * L>();
+    else wait_vmcnt<0>();
+    wait_lgkm0();
+    raw_barrier();
+    if (i < S) frags(i);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + NS - 1 < S) issue(i + NS - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i < S) products();
+  }
+  wait_lgkm0();
+  raw_barrier();
+  // the tile's sums: group 0 writes, the others add
+  auto cell = [&](int nb, int mb, int q) {
+    return reinterpret_cast<int32_t*>(smem + ((wm * MB + mb) * 32 + (lane & 31)) * ROW) + (wn * NB + nb) * 32 + 8 * q +
+           4 * (lane >> 5);
+  };
+  if (group == 0) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const i32x4 v = {acc[nb][mb][4 * q], acc[nb][mb][4 * q + 1], acc[nb][mb][4 * q + 2], acc[nb][mb][4 * q + 3]};
+          *reinterpret_cast<i32x4*>(cell(nb, mb, q)) = v;
+        }
+  }
+  __syncthreads();
+  if (group != 0) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) atomicAdd(cell(nb, mb, q) + e, acc[nb][mb][4 * q + e]);
+  }
+  __syncthreads();
+  constexpr int CPR = BN / 8;  // 8-channel pieces of a row (n % 8 == 0)
+#pragma unroll
+  for (int p = 0; p < (BM * CPR + THREADS - 1) / THREADS; ++p) {
+    const int i = (tid + p * THREADS) / CPR, c = (tid + p * THREADS) % CPR * 8;
+    const int64_t row = m0 + i;
+    if (i >= BM || row >= m || n0 + c >= n) continue;
+    const float sar = sa[row];
+    float scw[8], bf[8] = {};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) scw[e] = sw[n0 + c + e];
+    if (bias != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bf[e] = static_cast<float>(bias[n0 + c + e]);
+    }
+    int32_t a[8];
+    __builtin_memcpy(a, __builtin_assume_aligned(smem + i * ROW + c * 4, 16), sizeof(a));
+    f16x8 h;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float prod = static_cast<float>(a[e]) * sar;
+      h[e] = static_cast<_Float16>(prod * scw[e] + bf[e]);
+    }
+    *reinterpret_cast<f16x8*>(out + row * n + n0 + c) = h;
+    if (acc_out != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc_out[row * n + n0 + c + e] = a[e];
     }
   }
 }
@@ -1424,17 +1588,52 @@ int pp_groups(int64_t mt, int nt, int k) {
   return best;
 }
 
+// Which tile a GEMM of few 256 x 256 tiles takes, by its estimated time in microseconds:
+// rounds of workgroups over the CUs times a + b K per round. The constants were fitted to
+// K 1024..8448, N 1024..8448 and 16..4000 tokens on one GPU (per round at K 2112 / 8448:
+// 64 x 64 8.5 / 22.6, 128 x 64 11.2 / 29.5, 128 x 128 17 / 42 us; the 256 x 256 kernels of
+// one round 71 us at K 8448 (K a multiple of 256) and 28 us, up to 54 as the CUs fill, at
+// K 2112). With them 1030 x 8448 x 2112 went 71 -> 42 us, 16 x 8448 x 2112 66 -> 16,
+// 500 x 2112 x 6336 36 -> 18, 2500 x 2112 x 2112 38 -> 31.
+// What bounds the 128 x 128 tile: LDS traffic, 80 KB per 128 bytes of K against 512
+// cycles of MFMA.
+enum class FewTile { kNone, k64, k128x64, k128 };
+
+FewTile few_tile(int64_t m, int n, int k, int64_t tiles256) {
+  const int64_t cus = compute_units();
+  if (cus <= 0 || tiles256 > cus) return FewTile::kNone;
+  auto time = [&](int bm, int bn, double a, double b) {
+    return static_cast<double>(ceil_div(ceil_div(m, bm) * ceil_div(n, bn), cus)) * (a + b * k);
+  };
+  const double t64 = time(64, 64, 3.8, 2.2e-3), t128x64 = time(128, 64, 5.0, 2.9e-3), t128 = time(128, 128, 8.6, 3.95e-3);
+  const double load = static_cast<double>(tiles256) / static_cast<double>(cus);
+  const double t256 = k % 256 == 0 ? 9.0 + 7.4e-3 * k : 8.0 + (9.5e-3 + 12e-3 * load) * k;
+  const double least = std::min(t64, std::min(t128x64, t128));
+  if (least >= t256) return FewTile::kNone;
+  return least == t64 ? FewTile::k64 : least == t128x64 ? FewTile::k128x64 : FewTile::k128;
+}
+
+template <int BM, int BN, int WM, int WN, int NS, int G, int KB>
+void launch_few(const int8_t* q, const float* sa, const int8_t* w, const float* sw, const _Float16* b, int64_t m, int n,
+                int k, _Float16* o, int32_t* acc_out, hipStream_t stream) {
+  const int ntiles = static_cast<int>(ceil_div(n, BN));
+  hipLaunchKernelGGL((w8a8_gemm_few_kernel<BM, BN, WM, WN, NS, G, KB>), dim3(static_cast<unsigned>(ceil_div(m, BM) * ntiles)),
+                     dim3(64 * WM * WN * G), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out, ntiles);
+}
+
+template <int NP, bool kFull, bool kBlock>
+void launch_quant_as(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, hipStream_t stream) {
+  const int64_t most = int64_t(compute_units()) * 8;
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(kBlock ? m : ceil_div(m, 4), most)));
+  const size_t lds = static_cast<size_t>(k) * sizeof(float);
+  if (signs) hipLaunchKernelGGL((quant_kernel<NP, true, kFull, kBlock>), grid, dim3(256), lds, stream, x, m, k, signs, q, s);
+  else hipLaunchKernelGGL((quant_kernel<NP, false, kFull, kBlock>), grid, dim3(256), 0, stream, x, m, k, signs, q, s);
+}
+
 template <int NP>
 void launch_quant(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(m, 4), int64_t(compute_units()) * 8)));
-  const size_t lds = static_cast<size_t>(k) * sizeof(float);
-  if (k % kQuantCols == 0) {
-    if (signs) hipLaunchKernelGGL((quant_kernel<NP, true, true>), grid, dim3(256), lds, stream, x, m, k, signs, q, s);
-    else hipLaunchKernelGGL((quant_kernel<NP, false, true>), grid, dim3(256), 0, stream, x, m, k, signs, q, s);
-  } else {
-    if (signs) hipLaunchKernelGGL((quant_kernel<NP, true, false>), grid, dim3(256), lds, stream, x, m, k, signs, q, s);
-    else hipLaunchKernelGGL((quant_kernel<NP, false, false>), grid, dim3(256), 0, stream, x, m, k, signs, q, s);
-  }
+  if (k % kQuantCols == 0) launch_quant_as<NP, true, false>(x, m, k, signs, q, s, stream);
+  else launch_quant_as<NP, false, false>(x, m, k, signs, q, s, stream);
 }
 
 }  // namespace
@@ -1458,11 +1657,15 @@ int hi3d_w8a8_quantize(const void* x, int64_t m, int32_t k, const float* signs, 
   const _Float16* xh = static_cast<const _Float16*>(x);
   if (signs) HI3D_REQUIRE((reinterpret_cast<uintptr_t>(signs) & 15) == 0, "multipliers must be 16-byte aligned");
   const int passes = (k + kQuantCols - 1) / kQuantCols;
+  // From three passes on a row per workgroup, NP passes a wave: kernel time 7.6 -> 6.5 us on
+  // 1030 x 2112, 53 -> 50 us on 20011 x 2112, 72 -> 69 us on 24000 x 4096; rows past 8192
+  // columns used to be read twice by one wave (1030 x 8448: 36 -> 14 us).
   if (passes <= 1) launch_quant<1>(xh, m, k, signs, q, scale, stream);
   else if (passes <= 2) launch_quant<2>(xh, m, k, signs, q, scale, stream);
-  else if (passes <= 4) launch_quant<4>(xh, m, k, signs, q, scale, stream);
-  else if (passes <= 8) launch_quant<8>(xh, m, k, signs, q, scale, stream);
-  else launch_quant<16>(xh, m, k, signs, q, scale, stream);
+  else if (passes <= 4) launch_quant_as<1, false, true>(xh, m, k, signs, q, scale, stream);
+  else if (passes <= 8) launch_quant_as<2, false, true>(xh, m, k, signs, q, scale, stream);
+  else if (passes <= 12) launch_quant_as<3, false, true>(xh, m, k, signs, q, scale, stream);
+  else launch_quant_as<4, false, true>(xh, m, k, signs, q, scale, stream);
   HI3D_LAUNCH_CHECK();
   return HI3D_OK;
 }
@@ -1482,6 +1685,16 @@ int hi3d_w8a8_gemm(const int8_t* q, const float* sa, const int8_t* w, const floa
   HI3D_REQUIRE(blocks < (int64_t(1) << 31), "problem too large");
   const _Float16* b = static_cast<const _Float16*>(bias);
   _Float16* o = static_cast<_Float16*>(out);
+  if (k % 64 == 0 && n % 8 == 0) {
+    const FewTile t = few_tile(m, n, k, blocks);
+    if (t != FewTile::kNone) {
+      if (t == FewTile::k64) launch_few<64, 64, 2, 2, 2, 4, 128>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
+      else if (t == FewTile::k128x64) launch_few<128, 64, 2, 2, 3, 4, 64>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
+      else launch_few<128, 128, 2, 2, 3, 3, 64>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
+      HI3D_LAUNCH_CHECK();
+      return HI3D_OK;
+    }
+  }
   // per-lane source offsets within a 256-row tile are 32-bit
   // The persistent kernel removes the per-tile load latency and overlaps tiles; its stage
   // loop is slower than the one-tile kernel's, so it pays off for short K loops only

@@ -381,3 +381,57 @@ def test_norm_linear_workload4_shape_a(cuda):
     fused = w8a8.norm_linear(x, 1e-6, wq, sw, bias, scale=scale, shift=shift)
     composed = w8a8.linear(kernels.layer_norm_modulate(x, 1e-6, scale=scale, shift=shift), wq, sw, bias)
     assert torch.equal(fused, composed)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 64), (63, 72, 128), (65, 64, 192), (64, 1024, 8448), (129, 520, 2112),   # 64 x 64 tiles, K = 64 mod 128
+    (1030, 1024, 1024), (897, 1032, 1088),                                         # 128 x 64
+    (1030, 2112, 512), (1025, 2120, 704), (500, 6336, 2112),                       # 128 x 128, three K groups
+])
+def test_few_tile_gemm(cuda, m, n, k):
+    """GEMMs of few 256 x 256 tiles: partial tiles in both dimensions, K stages that do not
+    divide among the K groups (fewer stages than groups too), and codes at the extremes:
+    the accumulators exactly, the outputs bit for bit."""
+    from hi3d_amd import w8a8
+
+    rng = np.random.default_rng(m + n + k)
+    q, w = rng.integers(-127, 128, (m, k), dtype=np.int8), rng.integers(-127, 128, (n, k), dtype=np.int8)
+    q[0], w[0] = 127, -127
+    sa, sw = rng.uniform(1e-3, 1e-2, m).astype(np.float32), rng.uniform(1e-5, 1e-4, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float16)
+    acc = (torch.from_numpy(q).double() @ torch.from_numpy(w).double().T).numpy().astype(np.int32)
+    args = [torch.from_numpy(t).to(cuda) for t in (q, sa, w, sw, bias)]
+    out, got = w8a8.gemm(*args, return_acc=True)
+    assert np.array_equal(got.cpu().numpy(), acc)
+    want = ((acc.astype(np.float32) * sa[:, None]) * sw + bias.astype(np.float32)).astype(np.float16)
+    assert np.array_equal(out.cpu().numpy(), want)
+    assert torch.equal(w8a8.gemm(*args), out)
+    plain = ((acc.astype(np.float32) * sa[:, None]) * sw).astype(np.float16)
+    assert np.array_equal(w8a8.gemm(*args[:4], None).cpu().numpy(), plain)
+
+
+@pytest.mark.parametrize("m,k", [(1, 2112), (5, 4096), (3, 8192), (2, 8256), (7, 12352), (9000, 2112), (2, 16384)])
+@pytest.mark.parametrize("rotation", ["h64", "none"])
+def test_wide_row_quantiser(cuda, m, k, rotation):
+    """Rows of a workgroup each (more than 2048 columns): waves with no columns in their
+    last pass, more rows than workgroups, zero rows and rows whose scale is not finite,
+    against the oracle's codes and scales."""
+    from hi3d_amd import w8a8
+
+    rng = np.random.default_rng(m + k)
+    x = (rng.standard_normal((m, k)) * 3).astype(np.float16)
+    x[0, k - 1] = 60000
+    if m > 2:
+        x[1] = 0
+    if m > 4:
+        x[2, 5], x[4, k - 3] = np.inf, -np.inf
+    q, s = w8a8.quantize_activation(torch.from_numpy(x).to(cuda), None, rotation)
+    with np.errstate(all="ignore"):
+        want_q, want_s = ow8a8.quantize_activation(x[:8], None, rotation)
+    fine = np.isfinite(want_s)
+    assert np.array_equal(s[:8].cpu().numpy()[fine], want_s[fine])
+    assert np.array_equal(q[:8].cpu().numpy()[fine], want_q[fine])
+    # rows one at a time give the same bits as together
+    for i in ([m - 1, m // 2] if m > 8 else []):
+        q1, s1 = w8a8.quantize_activation(torch.from_numpy(x[i:i + 1]).to(cuda), None, rotation)
+        assert torch.equal(q1[0], q[i]) and torch.equal(s1[0], s[i])
