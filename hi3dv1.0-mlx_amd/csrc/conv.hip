@@ -18,6 +18,7 @@
 #include <utility>
 
 #include "common.h"
+#include "conv_group.h"
 #include "conv_tile.h"
 #include "quant.h"
 #include "rownorm.h"
@@ -1501,20 +1502,14 @@ __global__ __launch_bounds__(NW * 64, 1) void conv_wide_kernel(ConvArgs a) {
   if constexpr (kLN) {
     // The res block's second norm on whole output rows (cout == BN == 128): each row's
     // 16 chunks sit in the staged blocks of waves (row / 64) (chunks 0..7) and
-    // (row / 64) + 4 (chunks 8..15). Eight lanes per row, lane g holding chunks g and
-    // g + 8: the lanes, chunks, summation order and reduction partners of ln_kernel<8, 2>
-    // (the LayerNorm of 128-channel rows), so the result is bitwise the convolution
-    // followed by that kernel.
-#pragma clang fp contract(off)
+    // (row / 64) + 4 (chunks 8..15).
     static_assert(BN == 128 && NB == 2 && Sh::WM == 4 && NW == 8, "the row norm takes whole 128-channel rows");
     __syncthreads();
     const _Float16* scale = static_cast<const _Float16*>(a.ln_scale);
     const _Float16* shift = static_cast<const _Float16*>(a.ln_shift);
     const int g = lane & 7;
-    const float c = static_cast<float>(BN);
     // the four passes are unrolled so that their independent chains (LDS reads, sums,
-    // lane moves, the square root and the SiLU) overlap; lane moves by DPP (the same
-    // partners as ln_kernel's shuffles)
+    // lane moves, the square root and the SiLU) overlap
 #pragma unroll
     for (int pass = 0; pass < BM / (NW * 8); ++pass) {
       const int tr = pass * (NW * 8) + wave * 8 + (lane >> 3);  // tile row
@@ -1522,48 +1517,17 @@ __global__ __launch_bounds__(NW * 64, 1) void conv_wide_kernel(ConvArgs a) {
       const int32_t lrow = pt < a.ntiles ? reinterpret_cast<const int32_t*>(rows_lds)[tr] : -1;
       const bool live = lrow >= 0 && lrow < a.n_out;
       const int wr = tr & 63;
-      float v[2][8];
-      float sum = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const f16x8 h = *reinterpret_cast<const f16x8*>(smem + ((tr >> 6) + 4 * i) * (64 * ROWB) + wr * ROWB +
-                                                        ((g ^ (wr & (CPR - 1))) << 4));
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          v[i][e] = static_cast<float>(h[e]);
-          sum += v[i][e];
-        }
-      }
-      sum += dpp_xor4(sum);
-      sum += dpp_xor2(sum);
-      sum += dpp_xor1(sum);
-      const float mean = sum / c;
-      float sq = 0.0f;
+      f16x8 h[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float d = v[i][e] - mean;
-          sq += d * d;
-        }
-      sq += dpp_xor4(sq);
-      sq += dpp_xor2(sq);
-      sq += dpp_xor1(sq);
-      const float inv = 1.0f / sqrtf(sq / c + a.ln_eps);
+        h[i] = *reinterpret_cast<const f16x8*>(smem + ((tr >> 6) + 4 * i) * (64 * ROWB) + wr * ROWB +
+                                               ((g ^ (wr & (CPR - 1))) << 4));
       int b = live ? a.ln_coords[static_cast<int64_t>(lrow) * 4] : 0;
       b = b < 0 ? 0 : (b >= a.ln_batches ? a.ln_batches - 1 : b);
+      ln_modulate_silu_row128(h, a.ln_eps, scale + b * BN, shift + b * BN, g);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int ch = g + 8 * i;
-        f16x8 o;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = static_cast<_Float16>(f32_rounded((v[i][e] - mean) * inv));
-        o = modulate8(o, *reinterpret_cast<const f16x8*>(scale + b * BN + ch * 8),
-                      *reinterpret_cast<const f16x8*>(shift + b * BN + ch * 8));
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = silu_h(o[e]);
-        if (live) *reinterpret_cast<f16x8*>(a.out + (static_cast<int64_t>(lrow) * BN + ch * 8) * 2) = o;
-      }
+      for (int i = 0; i < 2; ++i)
+        if (live) *reinterpret_cast<f16x8*>(a.out + (static_cast<int64_t>(lrow) * BN + (g + 8 * i) * 8) * 2) = h[i];
     }
     return;
   }
@@ -1950,10 +1914,35 @@ int launch_pipe(const ConvArgs& base, hipStream_t stream) {
   return HI3D_OK;
 }
 
+GroupConv group_args(const ConvArgs& a) {
+  GroupConv c{};
+  c.in = a.in;
+  c.n_in = a.n_in;
+  c.cin = a.cin;
+  c.weight = a.weight;
+  c.bias = static_cast<const char*>(a.bias);
+  c.cout = a.cout;
+  c.kvol = a.kvol;
+  c.rows = a.rows;
+  c.gidx = a.gidx;
+  c.n_out = a.n_out;
+  c.residual = a.residual;
+  c.act = a.act;
+  c.out = a.out;
+  c.ln_coords = a.ln_coords;
+  c.ln_scale = a.ln_scale;
+  c.ln_shift = a.ln_shift;
+  c.ln_batches = a.ln_batches;
+  c.ln_eps = a.ln_eps;
+  return c;
+}
+
 template <typename T>
 int launch_mfma(const ConvArgs& base, hipStream_t stream) {
   ConvArgs a = base;
   if constexpr (sizeof(T) == 2) {
+    if (group_conv16_takes(a.n_out, a.cin, a.cout, a.kvol))
+      return group_conv16(group_args(a), std::is_same_v<T, __bf16>, stream);
     const int rb = a.cin * static_cast<int>(sizeof(T));
     const bool ring_rows = rb % 64 == 0 && rb >= 4 * 64 && rb <= 1024;
     const bool few = a.kvol <= 8 && (rb == 128 || rb == 256) && (a.cout == 64 || a.cout == 128);
@@ -2199,6 +2188,8 @@ int hi3d_gather_conv_ln_silu(const void* in, int64_t n_in, int32_t cin, const vo
   a.ln_shift = shift;
   a.ln_batches = batches;
   a.ln_eps = eps;
+  // the kernel that hi3d_gather_conv takes, so that the sums are the same
+  if (group_conv16_takes(n_out, cin, cout, kvol)) return group_conv16(group_args(a), false, as_stream(stream));
   return launch_wide<_Float16, 128, 8, false, true>(a, as_stream(stream));
 }
 

@@ -1,9 +1,10 @@
-// fp32 gather convolution on the bf16 matrix cores (gfx950): each fp32 operand as the sum
-// of three bf16 values.
+// Gather convolution over 64-row tiles whose offsets can be split over groups of waves
+// (gfx950): fp32 sets of any size, each fp32 operand as the sum of three bf16 values, and
+// 16-bit sets of few tiles.
 //
 //   out[o] = act(bias + sum_k in[gidx[o, k]] . W[:, k, :]^T) (+ residual[o])
 //
-// x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2), each
+// fp32: x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2), each
 // rounded to nearest: 24 bits, so the three hold every fp32 bit. Of the nine products
 // the kernel keeps w1 x1, w1 x2, w2 x1, w2 x2, w1 x3 and w3 x1; the others are below
 // 2^-25 of the product, under half an fp32 ulp. Products of two bf16 values are exact in
@@ -23,13 +24,16 @@
 #include <type_traits>
 
 #include "common.h"
+#include "conv_group.h"
 #include "conv_tile.h"
+#include "rownorm.h"
 
 namespace hi3d {
 namespace {
 
-constexpr int kSplitMaxKvol = 27;
-constexpr int kSplitMaxCin = 512;
+constexpr int kGroupMaxKvol = 27;
+constexpr int kGroupMaxRowBytes = 2048;
+constexpr int kSplitMaxCin = kGroupMaxRowBytes / 4;
 constexpr int kGroupThreads = 256;
 // Tables of few offsets (the strided pair, the child projection) are bound by their rows'
 // traffic until the products per row are many: the fp32 MFMA kernels ran the 64 -> 64
@@ -40,27 +44,7 @@ constexpr int kFewOffsets = 8;
 constexpr int64_t kFewOffsetsWork = 128 * 256;
 
 // row that absent neighbours read
-__device__ __attribute__((aligned(16))) const uint32_t g_split_zero_row[kSplitMaxCin] = {};
-
-struct SplitArgs {
-  const float* in;
-  int64_t n_in;
-  int32_t cin;
-  const char* packed;  // [kvol][cin / 16][col_blocks][3 parts][64 lanes][16 bytes]
-  int32_t col_blocks;  // 32-channel blocks of the packed weights (the last may be padding)
-  const float* weight;
-  int64_t wn, wk, wc;  // weight strides: output channel, offset, input channel
-  const float* bias;
-  int32_t cout;
-  int32_t kvol;
-  const int32_t* rows;
-  const int32_t* gidx;
-  int64_t n_out;
-  int32_t ny;  // column tiles
-  const float* residual;
-  int32_t act;
-  float* out;
-};
+__device__ __attribute__((aligned(16))) const uint32_t g_group_zero_row[kGroupMaxRowBytes / 4] = {};
 
 // The three bf16 parts of 8 fp32 values.
 __device__ __forceinline__ void split8(const f32x4 lo, const f32x4 hi, bf16x8 (&p)[3]) {
@@ -119,34 +103,37 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* __restri
   for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(packed + block * 3072 + i * 1024 + lane * 16) = p[i];
 }
 
-// A workgroup owns BM plan rows and BN channels; its 4 G waves form G groups, each a 2 x 2
-// grid of waves over the whole tile that takes every G-th offset, so that a set of
+// A workgroup owns BM = 64 plan rows and BN channels; its 4 G waves form G groups, each a
+// 2 x 2 grid of waves over the whole tile that takes every G-th offset, so that a set of
 // few tiles spreads its chain of offsets over a CU's four SIMDs' worth of waves. The
 // groups' sums are added in order in the epilogue.
-//  * Stages (per group): (present offset, 16 KS inputs): BM gathered fp32 rows of 64 KS
-//    bytes and the packed weights' BN / 32 x KS x 3 KB, by direct-to-LDS 16-byte loads
-//    NS - 1 stages ahead into a ring of NS slots, one barrier a stage.
-//  * The weights' parts are laid out as the fragments are read (1 KB a wave-wide read);
-//    the rows stay fp32 in LDS and each wave splits its fragments in registers (11
-//    vector ops per pair of values).
+//  * Stages (per group): (present offset, 64 KS bytes of the input rows): BM gathered rows
+//    and the weights (fp32: BN / 32 x KS x 3 KB of parts, laid out as the fragments are
+//    read; 16-bit: BN rows), by direct-to-LDS 16-byte loads NS - 1 stages ahead into a
+//    ring of NS slots, one barrier a stage. A stage's fragments are all read before the
+//    next loads are issued and the first product runs.
+//  * fp32 rows stay fp32 in LDS and each wave splits its fragments in registers (11 vector
+//    ops per pair of values).
 //  * The gather indices of all offsets reach LDS once, and with them the offsets that each
-//    32-row block has; a wave skips its blocks' products of the others.
+//    32-row block has; a wave skips its block's products of the others.
 //  * The MFMAs take the weights as their first operand: a lane ends with four consecutive
 //    channels of one row. The output leaves through LDS as whole row pieces.
-template <int BM, int BN, int KS, int NS, int G>
-__global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitArgs a) {
-  constexpr int KV = kSplitMaxKvol, THREADS = kGroupThreads * G, NWG = kGroupThreads / 64, NW = NWG * G;  // waves of a group, of all
-  constexpr int WM = BM / 2, WN = BN / 2, MB = WM / 32, NB = WN / 32, RB = BM / 32;
-  constexpr int ROWB = 64 * KS;
-  constexpr int A_BYTES = BM * ROWB, B_BYTES = (BN / 32) * KS * 3072, STAGE = A_BYTES + B_BYTES;
+template <typename T, int BN, int KS, int NS, int G, bool kLN = false>
+__global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupConv a) {
+  constexpr bool kSplit = sizeof(T) == 4;
+  constexpr int BM = 64, KV = kGroupMaxKvol, THREADS = kGroupThreads * G, NWG = kGroupThreads / 64, NW = NWG * G;
+  constexpr int WN = BN / 2, NB = WN / 32;
+  constexpr int ES = static_cast<int>(sizeof(T));
+  constexpr int ROWB = 64 * KS, LPR = 4 * KS;  // staged row: bytes, 16-byte chunks
+  constexpr int A_BYTES = BM * ROWB, B_BYTES = kSplit ? (BN / 32) * KS * 3072 : BN * ROWB, STAGE = A_BYTES + B_BYTES;
   constexpr int LA = A_BYTES / (1024 * NWG), BKB = B_BYTES / 1024;
   constexpr int LB = (BKB + NWG - 1) / NWG, LBMIN = BKB / NWG;  // loads of the waves below BKB % NWG, of the others
   static_assert(LA * 1024 * NWG == A_BYTES && (KS == 1 || KS == 2) && NS >= 2 && NS <= 4, "stage shape");
-  static_assert(BM % 64 == 0 && kTileRows % BM == 0, "a workgroup's rows lie in one plan tile");
+  static_assert(kTileRows % BM == 0, "a workgroup's rows lie in one plan tile");
   constexpr int RING = G * NS * STAGE;
-  constexpr int OUTB = BN * 4, CPR = BN / 4;  // staged row: bytes, 16-byte chunks
-  static_assert(G * 64 * OUTB <= RING, "one row block of each wave, staged");
-  __shared__ __attribute__((aligned(16))) char smem[RING + (KV + 1) * BM * 4 + NW * RB * 4];
+  constexpr int SROW = BN * 4;  // staged sums: bytes of a row
+  static_assert(G * BM * SROW <= RING, "staged sums");
+  __shared__ __attribute__((aligned(16))) char smem[RING + (KV + 1) * BM * 4 + NW * 8];
   int32_t* const gl = reinterpret_cast<int32_t*>(smem + RING);
   int32_t* const srow = gl + KV * BM;
   uint32_t* const smask = reinterpret_cast<uint32_t*>(srow + BM);  // [wave][32-row block]
@@ -167,47 +154,38 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
   // gather indices of all offsets (-1: absent), this wave's offsets wave_all, + NW, ...
   {
     constexpr int PER = (KV + NW - 1) / NW;
-    int32_t g[PER][BM / 64];
+    int32_t g[PER];
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int k = wave_all + NW * j;
-#pragma unroll
-      for (int h = 0; h < BM / 64; ++h) g[j][h] = gsrc[(k < kvol ? k : 0) * kTileRows + 64 * h + lane];
+      g[j] = gsrc[(k < kvol ? k : 0) * kTileRows + lane];
     }
     if (tid < BM) srow[tid] = a.rows[p0 + tid];
-    uint32_t m[RB] = {};
+    uint32_t lo = 0, hi = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int k = wave_all + NW * j;
       if (k >= kvol) continue;
-#pragma unroll
-      for (int h = 0; h < BM / 64; ++h) {
-        const bool ok = static_cast<uint64_t>(static_cast<uint32_t>(g[j][h])) < n_in;
-        const uint64_t b = __builtin_amdgcn_ballot_w64(ok);
-        if (static_cast<uint32_t>(b) != 0) m[2 * h] |= 1u << k;
-        if (static_cast<uint32_t>(b >> 32) != 0) m[2 * h + 1] |= 1u << k;
-        gl[k * BM + 64 * h + lane] = ok ? g[j][h] : -1;
-      }
+      const bool ok = static_cast<uint64_t>(static_cast<uint32_t>(g[j])) < n_in;
+      const uint64_t b = __builtin_amdgcn_ballot_w64(ok);
+      if (static_cast<uint32_t>(b) != 0) lo |= 1u << k;
+      if (static_cast<uint32_t>(b >> 32) != 0) hi |= 1u << k;
+      gl[k * BM + lane] = ok ? g[j] : -1;
     }
     if (lane == 0) {
-#pragma unroll
-      for (int i = 0; i < RB; ++i) smask[wave_all * RB + i] = m[i];
+      smask[wave_all * 2] = lo;
+      smask[wave_all * 2 + 1] = hi;
     }
   }
   __syncthreads();
-  uint32_t mask = 0, bmask[MB];  // offsets of the tile, of this wave's row blocks
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) bmask[mb] = 0;
+  uint32_t mask = 0, bmask = 0;  // offsets of the tile, of this wave's row block
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-#pragma unroll
-    for (int i = 0; i < RB; ++i) mask |= smask[w * RB + i];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) bmask[mb] |= smask[w * RB + wm * MB + mb];
+    mask |= smask[w * 2] | smask[w * 2 + 1];
+    bmask |= smask[w * 2 + wm];
   }
   mask = __builtin_amdgcn_readfirstlane(mask);
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) bmask[mb] = __builtin_amdgcn_readfirstlane(bmask[mb]);
+  bmask = __builtin_amdgcn_readfirstlane(bmask);
 
   // this group's offsets k = group mod G, whatever the tile: a row's sum does not depend on
   // the rows it shares a tile with (absent neighbours add zeros)
@@ -217,34 +195,36 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
   int most = 0;
 #pragma unroll
   for (int g = 0; g < G; ++g) most = max(most, __popc(mask & (EVERY << g)));
-  const int ksteps = a.cin / (16 * KS);  // stages per offset
+  const int row_bytes = a.cin * ES;
+  const int ksteps = row_bytes / ROWB;  // stages per offset
   const int S = __popc(mine) * ksteps;
   const int SMAX = most * ksteps;  // barriers are the workgroup's
-  const int64_t row_bytes = static_cast<int64_t>(a.cin) * 4;
   char* const ring = smem + group * (NS * STAGE);
 
   // load u of this wave fills 1 KB of the stage's rows: 16 / KS rows, 4 KS lanes a row
-  constexpr int LPR = 4 * KS;
-  auto a_off = [](int row, int chunk) {
+  auto row_off = [](int row, int chunk) {
     return KS == 1 ? row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4) : lds_offset(row, chunk);
   };
-  int r_ld[LA], c_ld[LA];
-#pragma unroll
-  for (int u = 0; u < LA; ++u) {
-    r_ld[u] = (wave + NWG * u) * (64 / LPR) + lane / LPR;
-    const int c = lane % LPR;
-    c_ld[u] = (KS == 1 ? (c ^ ((r_ld[u] >> 2) & 3)) : (c ^ ((r_ld[u] >> 1) & 7))) * 16;
-  }
+  auto load_row = [&](int u) { return (wave + NWG * u) * (64 / LPR) + lane / LPR; };
+  auto load_byte = [&](int u) {  // of the row, at this lane's place
+    const int r = load_row(u), c = lane % LPR;
+    return (KS == 1 ? (c ^ ((r >> 2) & 3)) : (c ^ ((r >> 1) & 7))) * 16;
+  };
   uint32_t rest = mine;
   int lks = 0, lslot = 0;
   const char* src[LA];
   const char* wsrc = nullptr;
-  const int wstep = a.col_blocks * 3072;  // one 16-input step
-  int woff[LB];                           // KB wave + 4 u of a stage's weights
+  const int wstep = kSplit ? KS * a.col_blocks * 3072 : ROWB;  // to the weights of the next stage
+  int64_t woff[LB];  // KB wave + 4 u of a stage's weights
 #pragma unroll
   for (int u = 0; u < LB; ++u) {
-    const int i = wave + NWG * u, s = i / (3 * (BN / 32));
-    woff[u] = s * wstep + (i - s * (3 * (BN / 32))) * 1024 + lane * 16;
+    if constexpr (kSplit) {
+      const int i = wave + NWG * u, s = i / (3 * (BN / 32));
+      woff[u] = s * (a.col_blocks * 3072) + (i - s * (3 * (BN / 32))) * 1024 + lane * 16;
+    } else {
+      const int n = n0 + load_row(u);  // channels past cout re-read the last (never stored)
+      woff[u] = static_cast<int64_t>(n < a.cout ? n : a.cout - 1) * kvol * row_bytes + load_byte(u);
+    }
   }
   auto issue = [&]() __attribute__((always_inline)) {
     if (lks == 0) {
@@ -252,12 +232,13 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
       rest &= rest - 1u;
 #pragma unroll
       for (int u = 0; u < LA; ++u) {
-        const int32_t g = gl[k * BM + r_ld[u]];
-        uint64_t pin = reinterpret_cast<uint64_t>(a.in) + static_cast<uint64_t>(g * row_bytes);
+        const int32_t g = gl[k * BM + load_row(u)];
+        uint64_t pin = reinterpret_cast<uint64_t>(a.in) + static_cast<uint64_t>(static_cast<int64_t>(g) * row_bytes);
         asm volatile("" : "+v"(pin));  // a select of addresses, not a branch
-        src[u] = (g >= 0 ? reinterpret_cast<const char*>(pin) : reinterpret_cast<const char*>(g_split_zero_row)) + c_ld[u];
+        src[u] = (g >= 0 ? reinterpret_cast<const char*>(pin) : reinterpret_cast<const char*>(g_group_zero_row)) + load_byte(u);
       }
-      wsrc = a.packed + (static_cast<int64_t>(k) * ksteps * KS * a.col_blocks + ct * (BN / 32)) * 3072;
+      wsrc = kSplit ? a.packed + (static_cast<int64_t>(k) * ksteps * KS * a.col_blocks + ct * (BN / 32)) * 3072
+                    : a.weight + static_cast<int64_t>(k) * row_bytes;
     }
     char* st = ring + lslot * STAGE;
 #pragma unroll
@@ -265,72 +246,60 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
 #pragma unroll
     for (int u = 0; u < LB; ++u)
       if (u < LBMIN || wave < BKB % NWG) lds_dma16(wsrc + woff[u], st + A_BYTES + (wave + NWG * u) * 1024);
-    wsrc += KS * wstep;
+    wsrc += wstep;
     lslot = lslot == NS - 1 ? 0 : lslot + 1;
     if (++lks == ksteps) lks = 0;
   };
 
-  f32x16 acc[NB][MB];
+  f32x16 acc[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[nb][mb][v] = 0.0f;
+    for (int v = 0; v < 16; ++v) acc[nb][v] = 0.0f;
 
-  uint32_t crest = mine;
-  int cks = 0, ck = mine ? __builtin_ctz(mine) : 0;  // the offset being multiplied
-  auto compute = [&](int slot) __attribute__((always_inline)) {
+  // a stage's fragments: rows x, weights w (fp32: KS steps of 16 inputs, a step's row
+  // fragment as two 16-byte chunks and its weights as three parts; 16-bit: 2 KS groups)
+  constexpr int XF = 2 * KS, WF = kSplit ? 3 * KS : 2 * KS;
+  u32x4 x[XF], w[NB][WF];
+  auto frags = [&](int slot) __attribute__((always_inline)) {
     const char* st = ring + slot * STAGE;
-    uint32_t have = 0;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) have |= ((bmask[mb] >> ck) & 1u) << mb;
-    if (have != 0) {
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int f = 0; f < WF; ++f) {
+        if constexpr (kSplit)
+          w[nb][f] = *reinterpret_cast<const u32x4*>(
+              st + A_BYTES + (((f / 3) * (BN / 32) + wn * NB + nb) * 3 + f % 3) * 1024 + lane * 16);
+        else
+          w[nb][f] = *reinterpret_cast<const u32x4*>(
+              st + A_BYTES + row_off((wn * NB + nb) * 32 + (lane & 31), 2 * f + (lane >> 5)));
+      }
+#pragma unroll
+    for (int f = 0; f < XF; ++f) {
+      const int c = kSplit ? 4 * (f / 2) + 2 * (lane >> 5) + f % 2 : 2 * f + (lane >> 5);
+      x[f] = *reinterpret_cast<const u32x4*>(st + row_off(wm * 32 + (lane & 31), c));
+    }
+  };
+  auto products = [&]() __attribute__((always_inline)) {
+    if constexpr (kSplit) {
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        bf16x8 w[NB][3];
+        bf16x8 xp[3];
+        split8(__builtin_bit_cast(f32x4, x[2 * s]), __builtin_bit_cast(f32x4, x[2 * s + 1]), xp);
+        // small products first
+        constexpr int WP[6] = {2, 0, 1, 1, 0, 0}, XP[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+        for (int t = 0; t < 6; ++t)
 #pragma unroll
-          for (int t = 0; t < 3; ++t)
-            w[nb][t] = *reinterpret_cast<const bf16x8*>(
-                st + A_BYTES + ((s * (BN / 32) + wn * NB + nb) * 3 + t) * 1024 + lane * 16);
-        auto products = [&](auto first, auto count) __attribute__((always_inline)) {
-          constexpr int M0 = decltype(first)::value, MN = decltype(count)::value;
-          bf16x8 x[MN][3];
-#pragma unroll
-          for (int i = 0; i < MN; ++i) {
-            const int row = wm * WM + (M0 + i) * 32 + (lane & 31), c = 4 * s + 2 * (lane >> 5);
-            split8(*reinterpret_cast<const f32x4*>(st + a_off(row, c)),
-                   *reinterpret_cast<const f32x4*>(st + a_off(row, c + 1)), x[i]);
-          }
-          // small products first
-          constexpr int WP[6] = {2, 0, 1, 1, 0, 0}, XP[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-          for (int t = 0; t < 6; ++t)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-              for (int i = 0; i < MN; ++i)
-                acc[nb][M0 + i] =
-                    __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[nb][WP[t]], x[i][XP[t]], acc[nb][M0 + i], 0, 0, 0);
-        };
-        using I0 = std::integral_constant<int, 0>;
-        using I1 = std::integral_constant<int, 1>;
-        if constexpr (MB == 1) {
-          products(I0{}, I1{});
-        } else {
-          static_assert(MB == 2, "row blocks of a wave");
-          if (have == 3) products(I0{}, std::integral_constant<int, 2>{});
-          else if (have == 1) products(I0{}, I1{});
-          else products(I1{}, I1{});
-        }
+          for (int nb = 0; nb < NB; ++nb)
+            acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[nb][3 * s + WP[t]]), xp[XP[t]],
+                                                              acc[nb], 0, 0, 0);
       }
-    }
-    if (++cks == ksteps) {
-      cks = 0;
-      crest &= crest - 1u;
-      ck = crest ? __builtin_ctz(crest) : 0;
+    } else {
+#pragma unroll
+      for (int f = 0; f < XF; ++f)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) Mfma<T>::run(w[nb][f], x[f], acc[nb]);
     }
   };
 
@@ -339,7 +308,8 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
 #pragma unroll
   for (int s = 0; s < NS - 1; ++s)
     if (s < S) issue();
-  int slot = 0;
+  uint32_t crest = mine;
+  int cks = 0, slot = 0;
   for (int s = 0; s < SMAX; ++s) {
     constexpr int AHEAD = NS - 2;  // stages that may stay in flight
     if (s + AHEAD < S) {
@@ -350,30 +320,37 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
     }
     wait_lgkm0();
     raw_barrier();
+    // this block has the offset (none left: false)
+    const bool have = s < S && (bmask & (crest & (0u - crest))) != 0;
+    if (have) frags(slot);
+    __builtin_amdgcn_sched_barrier(0);
     if (s + NS - 1 < S) issue();
-    if (s < S) compute(slot);
+    __builtin_amdgcn_sched_barrier(0);
+    if (have) products();
     slot = slot == NS - 1 ? 0 : slot + 1;
+    if (++cks == ksteps) {
+      cks = 0;
+      crest &= crest - 1u;
+    }
   }
 
-  // plain fp32 sum of one output, for sums that are not finite
+  // plain fp32 sum of one output, for fp32 sums that are not finite
   auto plain = [&](int row, int n) {
     float s = 0.0f;
     for (int k = 0; k < kvol; ++k) {
       const int32_t g = gl[k * BM + row];
       if (g < 0) continue;
-      const float* x = a.in + static_cast<int64_t>(g) * a.cin;
-      const float* w = a.weight + n * a.wn + k * a.wk;
-      for (int c = 0; c < a.cin; ++c) s = fmaf(x[c], w[c * a.wc], s);
+      const float* xr = reinterpret_cast<const float*>(a.in) + static_cast<int64_t>(g) * a.cin;
+      const float* wr = reinterpret_cast<const float*>(a.weight) + n * a.wn + k * a.wk;
+      for (int c = 0; c < a.cin; ++c) s = fmaf(xr[c], wr[c * a.wc], s);
     }
     return s;
   };
-  // one 32-row block of each wave at a time: [group][2 x 32 rows][BN], 16-byte chunk c of
-  // row r at c ^ (r % 16)
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    wait_lgkm0();
-    raw_barrier();
-    char* const stg = smem + (group * 64 + wm * 32 + (lane & 31)) * OUTB;
+  // the sums: [group][64 rows][BN] fp32, 16-byte chunk c of row r at c ^ (r % 16)
+  wait_lgkm0();
+  raw_barrier();
+  {
+    char* const stg = smem + (group * BM + wm * 32 + (lane & 31)) * SROW;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -381,53 +358,86 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_split_kernel(SplitA
         const int chunk = (wn * WN + nb * 32 + 8 * q + 4 * (lane >> 5)) >> 2;
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[nb][mb][4 * q + e];
+        for (int e = 0; e < 4; ++e) v[e] = acc[nb][4 * q + e];
         *reinterpret_cast<f32x4*>(stg + ((chunk ^ (lane & 15)) << 4)) = v;
       }
     }
-    wait_lgkm0();
-    raw_barrier();
-    constexpr int PASS = 64 * CPR / THREADS;
+  }
+  wait_lgkm0();
+  raw_barrier();
+  constexpr int E = 16 / ES, CPR = BN / E;                 // 16-byte output pieces of a row
+  constexpr int TPR = kLN ? 8 : CPR;                       // threads of a row
+  constexpr int PASS = (BM * TPR + THREADS - 1) / THREADS;
+  static_assert(!kLN || (ES == 2 && BN == 128), "the row norm takes whole 128-channel rows");
 #pragma unroll
-    for (int i = 0; i < PASS; ++i) {
-      const int r = tid / CPR + (THREADS / CPR) * i, chunk = tid % CPR;
-      const int lrow = (r >> 5) * WM + mb * 32 + (r & 31);  // the tile's row
-      const int32_t orow = srow[lrow];
-      const int n = n0 + chunk * 4;
-      if (orow < 0 || orow >= a.n_out || n >= a.cout) continue;  // cout is a multiple of 4
-      f32x4 v = *reinterpret_cast<const f32x4*>(smem + r * OUTB + ((chunk ^ (r & 15)) << 4));
+  for (int i = 0; i < PASS; ++i) {
+    // (with the norm eight lanes share a row, lane g its pieces g and g + 8)
+    const int r = tid / TPR + (THREADS / TPR) * i;
+    if (r >= BM) break;
+    const int32_t orow = srow[r];
+    const bool live = orow >= 0 && orow < a.n_out;
+    T h[kLN ? 2 : 1][E];
 #pragma unroll
-      for (int g = 1; g < G; ++g)
-        v += *reinterpret_cast<const f32x4*>(smem + (g * 64 + r) * OUTB + ((chunk ^ (r & 15)) << 4));
-      if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY)) {
+    for (int j = 0; j < (kLN ? 2 : 1); ++j) {
+      const int piece = kLN ? tid % 8 + 8 * j : tid % CPR;
+      const int n = n0 + piece * E;
+      if (!kLN && (!live || n >= a.cout)) continue;  // cout is a multiple of E
+#pragma unroll
+      for (int p = 0; p < E / 4; ++p) {
+        const int chunk = piece * (E / 4) + p;
+        f32x4 v = *reinterpret_cast<const f32x4*>(smem + r * SROW + ((chunk ^ (r & 15)) << 4));
+#pragma unroll
+        for (int g = 1; g < G; ++g)
+          v += *reinterpret_cast<const f32x4*>(smem + (g * BM + r) * SROW + ((chunk ^ (r & 15)) << 4));
+        if constexpr (kSplit) {
+          if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY)) {
 #pragma unroll 1
+            for (int e = 0; e < 4; ++e) {
+              const float y = plain(r, n + e);
+              v = f32x4{e == 0 ? y : v[0], e == 1 ? y : v[1], e == 2 ? y : v[2], e == 3 ? y : v[3]};
+            }
+          }
+        }
+#pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float y = plain(lrow, n + e);
-          v = f32x4{e == 0 ? y : v[0], e == 1 ? y : v[1], e == 2 ? y : v[2], e == 3 ? y : v[3]};
+          float y = v[e];
+          if (a.bias != nullptr) y += static_cast<float>(reinterpret_cast<const T*>(a.bias)[n + 4 * p + e]);
+          if (a.act == HI3D_ACT_SILU) y = silu_f32(y);
+          h[j][4 * p + e] = static_cast<T>(y);
         }
       }
-      if (a.bias != nullptr) {
+    }
+    if constexpr (kLN) {
+      f16x8 o[2];
+      __builtin_memcpy(o, h, sizeof(o));
+      int b = live ? a.ln_coords[static_cast<int64_t>(orow) * 4] : 0;
+      b = b < 0 ? 0 : (b >= a.ln_batches ? a.ln_batches - 1 : b);
+      const int g = tid % 8;
+      ln_modulate_silu_row128(o, a.ln_eps, static_cast<const _Float16*>(a.ln_scale) + b * BN,
+                              static_cast<const _Float16*>(a.ln_shift) + b * BN, g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += a.bias[n + e];
-      }
-      if (a.act == HI3D_ACT_SILU) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = silu_f32(v[e]);
-      }
-      const int64_t off = static_cast<int64_t>(orow) * a.cout + n;
-      if (a.residual != nullptr) v += *reinterpret_cast<const f32x4*>(a.residual + off);
-      *reinterpret_cast<f32x4*>(a.out + off) = v;
+      for (int j = 0; j < 2; ++j)
+        if (live) *reinterpret_cast<f16x8*>(a.out + (static_cast<int64_t>(orow) * BN + (g + 8 * j) * 8) * 2) = o[j];
+    } else {
+      const int n = n0 + tid % CPR * E;
+      if (!live || n >= a.cout) continue;
+      const int64_t off = (static_cast<int64_t>(orow) * a.cout + n) * ES;
+      u32x4 v;
+      __builtin_memcpy(&v, h, sizeof(v));
+      if (a.residual != nullptr) v = add_chunk<T>(v, *reinterpret_cast<const u32x4*>(a.residual + off));
+      *reinterpret_cast<u32x4*>(a.out + off) = v;
     }
   }
 }
 
-template <int BM, int BN, int KS, int NS, int G>
-int launch_split(const SplitArgs& base, hipStream_t stream) {
-  SplitArgs a = base;
+template <typename T, int BN, int KS, int NS, int G, bool kLN = false>
+int launch_group(const GroupConv& base, hipStream_t stream) {
+  GroupConv a = base;
   a.ny = static_cast<int32_t>(ceil_div(a.cout, BN));
-  const int64_t blocks = ceil_div(a.n_out, BM) * a.ny;
+  const int64_t blocks = ceil_div(a.n_out, 64) * a.ny;
   HI3D_REQUIRE(blocks < (int64_t(1) << 31), "too many tiles");
-  hipLaunchKernelGGL((conv_split_kernel<BM, BN, KS, NS, G>), dim3(static_cast<unsigned>(blocks)), dim3(kGroupThreads * G), 0, stream, a);
+  hipLaunchKernelGGL((conv_group_kernel<T, BN, KS, NS, G, kLN>), dim3(static_cast<unsigned>(blocks)),
+                     dim3(kGroupThreads * G), 0, stream, a);
   HI3D_LAUNCH_CHECK();
   return HI3D_OK;
 }
@@ -436,6 +446,56 @@ int launch_split(const SplitArgs& base, hipStream_t stream) {
 int col_blocks(int cout) { return cout % 128 == 0 ? cout / 32 : static_cast<int>(ceil_div(cout, 64)) * 2; }
 
 }  // namespace
+
+namespace {
+
+// Which 16-bit convolutions run here, from 9 offsets on (one GPU, fp16, microseconds there
+// -> here):
+//  * Few 64 x 64 tiles: four offset groups a workgroup, one round of workgroups over the
+//    CUs, or two where a tile is worth 128 x 64 products an offset (1,531 voxels C128
+//    40 -> 16, 16,000 voxels 42 -> 32; C256 4,000 voxels 130 -> 32; three rounds lose:
+//    24,000 voxels C128 41.5 against 48; C64, two rounds, 19.9 against 20.2).
+//  * From 256 x 256 channels on, two rounds of 64 x 128 tiles (16,000 voxels C256
+//    129 -> 73; three rounds 131 against 131).
+//  * Channel counts that the ring and wide kernels do not take, at any size (96 -> 160 on
+//    1.1M voxels 1503 -> 1094, on 33k 139 -> 63; 32 -> 32 on 1.1M 375 -> 192).
+enum class Group16 { kNone, kFew, kWide, kAny };
+
+Group16 group16(int64_t n_out, int cin, int cout, int kvol) {
+  const int rb = cin * 2;
+  if (kvol <= kFewOffsets || kvol > kGroupMaxKvol || cin % 32 != 0 || rb > kGroupMaxRowBytes || cout % 8 != 0)
+    return Group16::kNone;
+  const int64_t cus = compute_units(), row_tiles = ceil_div(n_out, 64);
+  if (row_tiles * ceil_div(cout, 64) <= (static_cast<int64_t>(cin) * cout >= 128 * 64 ? 2 : 1) * cus)
+    return Group16::kFew;
+  if (cin % 64 == 0 && cin >= 256 && cout % 256 == 0 && row_tiles * (cout / 128) <= 2 * cus) return Group16::kWide;
+  const bool ring = (rb % 64 == 0 && rb >= 256 && rb <= 1024 && cout % 128 == 0) ||
+                    ((rb == 128 || rb == 256) && (cout == 64 || cout == 128));
+  return ring ? Group16::kNone : Group16::kAny;
+}
+
+template <typename T>
+int group16_run(const GroupConv& c, hipStream_t stream) {
+  switch (group16(c.n_out, c.cin, c.cout, c.kvol)) {
+    case Group16::kFew:
+      return c.cin % 64 == 0 ? launch_group<T, 64, 2, 2, 4>(c, stream) : launch_group<T, 64, 1, 2, 4>(c, stream);
+    case Group16::kWide: return launch_group<T, 128, 2, 2, 1>(c, stream);
+    default: return launch_group<T, 64, 1, 3, 1>(c, stream);
+  }
+}
+
+}  // namespace
+
+bool group_conv16_takes(int64_t n_out, int cin, int cout, int kvol) {
+  return group16(n_out, cin, cout, kvol) != Group16::kNone;
+}
+
+int group_conv16(const GroupConv& c, bool bf16, hipStream_t stream) {
+  // the row norm (fp16, 128 channels) takes few tiles: 128-channel ones, the same sums
+  if (c.ln_coords != nullptr) return launch_group<_Float16, 128, 1, 3, 4, true>(c, stream);
+  return bf16 ? group16_run<__bf16>(c, stream) : group16_run<_Float16>(c, stream);
+}
+
 }  // namespace hi3d
 
 using namespace hi3d;
@@ -445,7 +505,7 @@ extern "C" {
 int hi3d_gather_conv_f32_workspace(int32_t cin, int32_t cout, int32_t kvol, int64_t* bytes_host) {
   HI3D_REQUIRE(bytes_host != nullptr, "null pointer argument");
   HI3D_REQUIRE(cin > 0 && cout > 0 && kvol > 0, "channels and kvol must be positive");
-  const bool taken = kvol <= kSplitMaxKvol && cin <= kSplitMaxCin && cin % 32 == 0 && cout % 4 == 0 &&
+  const bool taken = kvol <= kGroupMaxKvol && cin <= kSplitMaxCin && cin % 32 == 0 && cout % 4 == 0 &&
                      (kvol > kFewOffsets || static_cast<int64_t>(cin) * cout >= kFewOffsetsWork);
   *bytes_host = taken ? static_cast<int64_t>(kvol) * (cin / 16) * col_blocks(cout) * 3072 : 0;
   return HI3D_OK;
@@ -458,7 +518,7 @@ int hi3d_gather_conv_f32(const float* in, int64_t n_in, int32_t cin, const float
   int64_t need = 0;
   if (const int e = hi3d_gather_conv_f32_workspace(cin, cout, kvol, &need)) return e;
   HI3D_REQUIRE(need > 0, "gather conv f32 takes Cin a multiple of 32 up to %d, Cout a multiple of 4 and at most %d offsets",
-               kSplitMaxCin, kSplitMaxKvol);
+               kSplitMaxCin, kGroupMaxKvol);
   HI3D_REQUIRE(n_in >= 0 && n_out >= 0, "sizes must be non-negative");
   HI3D_REQUIRE(act == HI3D_ACT_NONE || act == HI3D_ACT_SILU, "unknown activation %d", act);
   if (n_out == 0) return HI3D_OK;
@@ -474,25 +534,25 @@ int hi3d_gather_conv_f32(const float* in, int64_t n_in, int32_t cin, const float
                    (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
   HI3D_REQUIRE((reinterpret_cast<uintptr_t>(bias) & 3) == 0, "the bias must be 4-byte aligned");
   hipStream_t s = as_stream(stream);
-  SplitArgs a{};
-  a.in = in;
+  GroupConv a{};
+  a.in = reinterpret_cast<const char*>(in);
   a.n_in = n_in;
   a.cin = cin;
   a.packed = static_cast<const char*>(workspace);
   a.col_blocks = col_blocks(cout);
-  a.weight = weight;
+  a.weight = reinterpret_cast<const char*>(weight);
   a.wn = stride_out;
   a.wk = stride_offset;
   a.wc = stride_in;
-  a.bias = bias;
+  a.bias = reinterpret_cast<const char*>(bias);
   a.cout = cout;
   a.kvol = kvol;
   a.rows = rows;
   a.gidx = gidx;
   a.n_out = n_out;
-  a.residual = residual;
+  a.residual = reinterpret_cast<const char*>(residual);
   a.act = act;
-  a.out = out;
+  a.out = reinterpret_cast<char*>(out);
   const int64_t total = need / 3 / 16;
   hipLaunchKernelGGL(split_weight_kernel, dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0, s, weight, stride_out,
                      stride_offset, stride_in, vec, cout, cin, a.col_blocks, total, static_cast<char*>(workspace));
@@ -505,9 +565,9 @@ int hi3d_gather_conv_f32(const float* in, int64_t n_in, int32_t cin, const float
   // 805 us, 64-channel tiles 870, 128-row tiles with half the weight reads 808); the
   // others two stages in 48 KB, so that three workgroups share a CU (45,128 voxels C64:
   // 78 -> 61 us, three slots and two workgroups 84).
-  if (ceil_div(n_out, 64) * ceil_div(cout, 64) <= compute_units()) return launch_split<64, 64, 1, 2, 4>(a, s);
-  if (cout % 128 == 0) return launch_split<64, 128, 2, 2, 1>(a, s);
-  return launch_split<64, 64, 2, 2, 1>(a, s);
+  if (ceil_div(n_out, 64) * ceil_div(cout, 64) <= compute_units()) return launch_group<float, 64, 1, 2, 4>(a, s);
+  if (cout % 128 == 0) return launch_group<float, 128, 2, 2, 1>(a, s);
+  return launch_group<float, 64, 2, 2, 1>(a, s);
 }
 
 }  // extern "C"

@@ -318,6 +318,39 @@ def test_fp32_split_kernel(cuda, cin, cout, density, side, act, res):
     assert torch.equal(y, y2)
 
 
+@pytest.mark.parametrize("dtype,cin,cout,density,side,act,res", [
+    (torch.float16, 128, 128, 0.2, 16, "silu", True),   # four offset groups, 128-byte stages
+    (torch.bfloat16, 64, 64, 0.3, 24, None, True),
+    (torch.float16, 32, 8, 0.1, 16, None, False),       # 8 of a tile's 64 outputs, 64-byte stages
+    (torch.float16, 96, 160, 0.01, 40, "silu", False),  # groups and blocks without offsets
+    (torch.bfloat16, 1024, 72, 0.2, 12, None, True),    # the longest rows
+    (torch.float16, 256, 256, 0.35, 32, None, True),    # one group, 128-channel tiles
+    (torch.bfloat16, 96, 160, 0.3, 48, "silu", True),   # one group, 64-byte stages
+    (torch.float16, 32, 40, 0.4, 48, None, False),
+])
+def test_16bit_group_kernel(cuda, dtype, cin, cout, density, side, act, res):
+    """16-bit convolutions of few tiles and of channel counts outside the ring kernels',
+    every tile shape of the dispatch: against float64 into memory that held NaN (every
+    row written), and each row's sum independent of the tile order."""
+    from hi3d_amd import conv, kmap
+
+    rng = np.random.default_rng(cin + 3 * cout)
+    idx = _rand_indices(rng, side, density)
+    n = len(idx)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    x, w, b = _case(rng, n, cin, cout, dtype)
+    r = torch.as_tensor(rng.standard_normal((n, cout), dtype=np.float32)).to(dtype) if res else None
+    xd, wd, bd = x.to(cuda), w.to(cuda), b.to(cuda)
+    rd = None if r is None else r.to(cuda)
+    out = torch.full((n, cout), float("nan"), dtype=dtype, device=cuda)
+    y = conv.gather_conv(xd, km.plan(), wd, bd, act=act, residual=rd, out=out)
+    ref = oconv.gather_conv_f64(x.float().numpy(), km.table.cpu().numpy(), w.float().numpy(), b.float().numpy(),
+                                act=act, residual=None if r is None else r.float().numpy())
+    assert oconv.rel_err(y.float().cpu().numpy(), ref) <= GATE[dtype]
+    y2 = conv.gather_conv(xd, kmap.build_plan(km.table, n, window_rows=64), wd, bd, act=act, residual=rd)
+    assert torch.equal(y, y2)
+
+
 def test_fp32_split_kernel_not_finite(cuda):
     """Infinities, NaN and values past bf16's largest, in the features and in the weights:
     where the sum over a row's present neighbours is infinite or NaN so is the output,
