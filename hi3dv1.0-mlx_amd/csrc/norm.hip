@@ -437,6 +437,9 @@ void launch_ln_quant_width(const _Float16* x, int64_t rows, int c, float eps, co
   else if (chunks <= 64) launch_ln_quant<16, 4, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
   else if (chunks <= 128) launch_ln_quant<32, 4, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
   else if (chunks <= 256) launch_ln_quant<64, 4, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
+  // (eight chunks a lane for 264 of them computed 512: 20011 x 2112 95 -> 63 us)
+  else if (chunks <= 320) launch_ln_quant<64, 5, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
+  else if (chunks <= 384) launch_ln_quant<64, 6, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
   else launch_ln_quant<64, 8, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
 }
 

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(64 * WM * WN * G, 1) void w8a8_gemm_few_kernel(
   }
 }
 
-// Persistent variant for full tiles (m, n >= 256, n % 8 == 0, k % 64 == 0, k >= 256): one
+// Persistent variant for full tiles (m, n >= 256, n % 8 == 0, k % 64 == 0, 256 <= k < 512): one
 // workgroup per CU walks a list of tiles while the stage pipeline above runs on without a
 // break: the next tile's first stages load during the current tile's last ones, and the
 // per-tile work around the K loop shrinks to the epilogue.
@@ -1232,7 +1232,7 @@ struct PQSrc {
   __amdgpu_buffer_rsrc_t a, b;
 };
 
-template <bool kDump>
+template <bool kDump, bool kPad>
 __global__ __launch_bounds__(512, 1) void w8a8_gemm_pq_kernel(const int8_t* __restrict__ qa, const float* __restrict__ sa,
                                                               const int8_t* __restrict__ w, const float* __restrict__ sw,
                                                               const _Float16* __restrict__ bias, int64_t m, int n, int k,
@@ -1331,6 +1331,10 @@ __global__ __launch_bounds__(512, 1) void w8a8_gemm_pq_kernel(const int8_t* __re
                                              (d < n / 2 ? d : n / 2 - 1) * 4, 0, 0, 0);
   };
 
+  // kPad, K a multiple of 64 that is not one of 256: up to three stages run past it, whose
+  // channel rows come through an empty descriptor, as zeros, whatever the token rows read
+  const int stages = k >> 6;
+  const __amdgpu_buffer_rsrc_t none = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(w), 0, 0, kRawBufferFlags);
   const int c16 = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
   int vo[2];
 #pragma unroll
@@ -1341,9 +1345,10 @@ __global__ __launch_bounds__(512, 1) void w8a8_gemm_pq_kernel(const int8_t* __re
     for (int j = 0; j < 2; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r.a, lds_ptr(smem + SL * kPPStage + (8 * g + 2 * q + j) * 1024), 16,
                                                vo[j], s * 64, 0, 0);
+    const __amdgpu_buffer_rsrc_t rb = kPad && s >= stages ? none : r.b;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(r.b, lds_ptr(smem + SL * kPPStage + kPPHalf + (8 * g + 2 * q + j) * 1024),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, lds_ptr(smem + SL * kPPStage + kPPHalf + (8 * g + 2 * q + j) * 1024),
                                                16, vo[j], s * 64, 0, 0);
   };
 
@@ -1465,7 +1470,7 @@ __global__ __launch_bounds__(512, 1) void w8a8_gemm_pq_kernel(const int8_t* __re
   using WE1 = std::integral_constant<int, 8 + kPQEpiOps>;      // group 1, stages 0-1
 
   // Prologue: scales of tile 0, stages 0-2 of tile 0 from every wave, all complete.
-  const int S = k >> 6;  // a multiple of 4, at least 8
+  const int S = kPad ? (stages + 3) & ~3 : stages;  // a multiple of 4, at least 8
   PQTile t0 = {0, static_cast<int>(local / ntg), static_cast<int>(local % ntg)};
   PQTile t1 = advance(t0);
   PQSrc cur = src_of(t0), nxt = src_of(t1);
@@ -1591,10 +1596,9 @@ int pp_groups(int64_t mt, int nt, int k) {
 // Which tile a GEMM of few 256 x 256 tiles takes, by its estimated time in microseconds:
 // rounds of workgroups over the CUs times a + b K per round. The constants were fitted to
 // K 1024..8448, N 1024..8448 and 16..4000 tokens on one GPU (per round at K 2112 / 8448:
-// 64 x 64 8.5 / 22.6, 128 x 64 11.2 / 29.5, 128 x 128 17 / 42 us; the 256 x 256 kernels of
-// one round 71 us at K 8448 (K a multiple of 256) and 28 us, up to 54 as the CUs fill, at
-// K 2112). With them 1030 x 8448 x 2112 went 71 -> 42 us, 16 x 8448 x 2112 66 -> 16,
-// 500 x 2112 x 6336 36 -> 18, 2500 x 2112 x 2112 38 -> 31.
+// 64 x 64 8.5 / 22.6, 128 x 64 11.2 / 29.5, 128 x 128 17 / 42 us; one round of 256 x 256
+// tiles 71 us at K 8448, 16 us at K 1024, 9 us more as the CUs fill). With them
+// 1030 x 8448 x 2112 went 71 -> 42 us, 16 x 8448 x 2112 66 -> 16, 500 x 2112 x 6336 36 -> 18.
 // What bounds the 128 x 128 tile: LDS traffic, 80 KB per 128 bytes of K against 512
 // cycles of MFMA.
 enum class FewTile { kNone, k64, k128x64, k128 };
@@ -1607,7 +1611,7 @@ FewTile few_tile(int64_t m, int n, int k, int64_t tiles256) {
   };
   const double t64 = time(64, 64, 3.8, 2.2e-3), t128x64 = time(128, 64, 5.0, 2.9e-3), t128 = time(128, 128, 8.6, 3.95e-3);
   const double load = static_cast<double>(tiles256) / static_cast<double>(cus);
-  const double t256 = k % 256 == 0 ? 9.0 + 7.4e-3 * k : 8.0 + (9.5e-3 + 12e-3 * load) * k;
+  const double t256 = 9.0 + 7.4e-3 * static_cast<double>(align_up(k, 256)) + 9.0 * load;
   const double least = std::min(t64, std::min(t128x64, t128));
   if (least >= t256) return FewTile::kNone;
   return least == t64 ? FewTile::k64 : least == t128x64 ? FewTile::k128x64 : FewTile::k128;
@@ -1696,16 +1700,16 @@ int hi3d_w8a8_gemm(const int8_t* q, const float* sa, const int8_t* w, const floa
     }
   }
   // per-lane source offsets within a 256-row tile are 32-bit
-  // The persistent kernel removes the per-tile load latency and overlaps tiles; its stage
-  // loop is slower than the one-tile kernel's, so it pays off for short K loops only
-  // (measured: K = 1024 faster, K = 4096 slower).
-  // The persistent ping-pong kernel takes K a multiple of 256 from 512 on with n % 8 == 0
+  // The persistent ping-pong kernel takes K a multiple of 64 from 512 on with n % 8 == 0
+  // (up to three stages of zeros where K is not a multiple of 256, still faster than the
+  // 4-wave kernels: 20011 x 2112 x 6336 342 -> 311 us, 20011 x 704 x 4096 104 -> 84, and
+  // 95 -> 83 us at K 576, where a quarter of the stages are zeros)
   // and 32-bit byte offsets within a tile of the output (and of acc_out, 16-byte aligned,
   // whose int32 accumulators it also stores).
   const bool aligned4 = ((reinterpret_cast<uintptr_t>(sa) | reinterpret_cast<uintptr_t>(sw) |
                           reinterpret_cast<uintptr_t>(bias)) & 3) == 0 &&
                         (reinterpret_cast<uintptr_t>(acc_out) & 15) == 0;
-  if (k % 256 == 0 && k >= 512 && n % 8 == 0 && static_cast<int64_t>(k) * 256 < (int64_t(1) << 31) &&
+  if (k % 64 == 0 && k >= 512 && n % 8 == 0 && static_cast<int64_t>(k) * 256 < (int64_t(1) << 31) &&
       m < (int64_t(1) << 29) &&
       static_cast<int64_t>(n) * (acc_out ? 1024 : 512) < (int64_t(1) << 31) - 4096 && aligned4) {
     const int gr = pp_groups(mtiles, ntiles, k);
@@ -1715,12 +1719,11 @@ int hi3d_w8a8_gemm(const int8_t* q, const float* sa, const int8_t* w, const floa
     HI3D_REQUIRE(cus > 0, "cannot query the compute unit count");
     const int64_t wpx = std::min<int64_t>(per_xcd, std::max(1, cus / 8));
     const dim3 grid(static_cast<unsigned>(wpx * 8));
-    if (acc_out)
-      hipLaunchKernelGGL(w8a8_gemm_pq_kernel<true>, grid, dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out,
-                         mtiles, ntiles, gr);
-    else
-      hipLaunchKernelGGL(w8a8_gemm_pq_kernel<false>, grid, dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out,
-                         mtiles, ntiles, gr);
+    auto launch = [&](auto* kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out, mtiles, ntiles, gr);
+    };
+    if (k % 256 == 0) launch(acc_out ? w8a8_gemm_pq_kernel<true, false> : w8a8_gemm_pq_kernel<false, false>);
+    else launch(acc_out ? w8a8_gemm_pq_kernel<true, true> : w8a8_gemm_pq_kernel<false, true>);
     HI3D_LAUNCH_CHECK();
     return HI3D_OK;
   }
@@ -1744,7 +1747,7 @@ int hi3d_w8a8_gemm(const int8_t* q, const float* sa, const int8_t* w, const floa
     return HI3D_OK;
   }
   // With acc_out the same kernel also stores the int32 accumulators (16-byte aligned).
-  if (k % 64 == 0 && k >= 4 * 64 && k < 32 * 64 && m >= kGemmBM && n >= kGemmBN && n % 8 == 0 &&
+  if (k % 64 == 0 && k >= 4 * 64 && k < 8 * 64 && m >= kGemmBM && n >= kGemmBN && n % 8 == 0 &&
       static_cast<int64_t>(kGemmBM) * k < (int64_t(1) << 32) && (reinterpret_cast<uintptr_t>(sa) & 3) == 0 &&
       (reinterpret_cast<uintptr_t>(sw) & 3) == 0 && (reinterpret_cast<uintptr_t>(bias) & 3) == 0 &&
       (reinterpret_cast<uintptr_t>(acc_out) & 15) == 0) {

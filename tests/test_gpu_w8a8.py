@@ -387,11 +387,13 @@ def test_norm_linear_workload4_shape_a(cuda):
     (1, 8, 64), (63, 72, 128), (65, 64, 192), (64, 1024, 8448), (129, 520, 2112),   # 64 x 64 tiles, K = 64 mod 128
     (1030, 1024, 1024), (897, 1032, 1088),                                         # 128 x 64
     (1030, 2112, 512), (1025, 2120, 704), (500, 6336, 2112),                       # 128 x 128, three K groups
+    (4200, 4104, 576), (4200, 4104, 704), (2900, 6000, 1152),                      # 256 x 256, K = 64, 192, 128 mod 256
 ])
 def test_few_tile_gemm(cuda, m, n, k):
     """GEMMs of few 256 x 256 tiles: partial tiles in both dimensions, K stages that do not
-    divide among the K groups (fewer stages than groups too), and codes at the extremes:
-    the accumulators exactly, the outputs bit for bit."""
+    divide among the K groups (fewer stages than groups too), codes at the extremes, and
+    more tiles than CUs where the stage loop runs past K: the accumulators exactly, the
+    outputs bit for bit."""
     from hi3d_amd import w8a8
 
     rng = np.random.default_rng(m + n + k)
