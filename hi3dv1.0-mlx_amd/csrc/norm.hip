@@ -6,6 +6,8 @@
 // 95-102; src/hi3d_mac/mlx_backend/transformer.py:548-549, 570-571, 575-577), the res-block modulation
 // (src/sparc3d/models/transformers/sparc3d_transformer.py:132-144,
 // src/hi3d_mac/mlx_backend/transformer.py:413-424).
+#include <type_traits>
+
 #include "common.h"
 #include "conv_tile.h"
 #include "quant.h"
@@ -14,15 +16,26 @@
 namespace hi3d {
 namespace {
 
+// 8 affine values as fp32 (fp16 parameters convert exactly).
+__device__ __forceinline__ void load8(const float* p, f32x4 (&v)[2]) {
+  v[0] = *reinterpret_cast<const f32x4*>(p);
+  v[1] = *reinterpret_cast<const f32x4*>(p + 4);
+}
+__device__ __forceinline__ void load8(const _Float16* p, f32x4 (&v)[2]) {
+  const f16x8 h = *reinterpret_cast<const f16x8*>(p);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e >> 2][e & 3] = static_cast<float>(h[e]);
+}
+
 // G lanes per row, CPL 8-element chunks per lane (chunk g + i G), held in registers;
 // fp32 two-pass statistics; y = (x - mean) * inv [* w + b]; h = fp16(y); modulate
 // h = fp16(fp16(h * scale) + shift) (two roundings, no FMA, modulate8); kSilu: h =
 // silu(h) in fp16.
 // The per-channel vectors of a lane's chunks are loaded once; blocks stride over groups
 // of 256 / G rows.
-template <int G, int CPL, bool kAffine, bool kModulate, bool kSilu = false>
+template <int G, int CPL, bool kAffine, bool kModulate, bool kSilu, typename W>
 __global__ __launch_bounds__(256) void ln_kernel(const _Float16* __restrict__ x, int64_t rows, int c, float eps,
-                                                 const float* __restrict__ weight, const float* __restrict__ bias,
+                                                 const W* __restrict__ weight, const W* __restrict__ bias,
                                                  const _Float16* __restrict__ scale,
                                                  const _Float16* __restrict__ shift, _Float16* __restrict__ out) {
 #pragma clang fp contract(off)
@@ -39,10 +52,8 @@ __global__ __launch_bounds__(256) void ln_kernel(const _Float16* __restrict__ x,
     const bool ok = ch < chunks;
     if constexpr (affine) {
       if (!ok) continue;
-      wv[i][0] = *reinterpret_cast<const f32x4*>(weight + ch * 8);
-      wv[i][1] = *reinterpret_cast<const f32x4*>(weight + ch * 8 + 4);
-      bv[i][0] = *reinterpret_cast<const f32x4*>(bias + ch * 8);
-      bv[i][1] = *reinterpret_cast<const f32x4*>(bias + ch * 8 + 4);
+      load8(weight + ch * 8, wv[i]);
+      load8(bias + ch * 8, bv[i]);
     }
     if constexpr (modulate) {
       if (!ok) continue;
@@ -111,9 +122,9 @@ __global__ __launch_bounds__(256) void ln_kernel(const _Float16* __restrict__ x,
 }
 
 // Any width: one wave per row, three passes over the row in global memory.
+template <typename W>
 __global__ __launch_bounds__(256) void ln_generic_kernel(const _Float16* __restrict__ x, int64_t rows, int c, float eps,
-                                                         const float* __restrict__ weight,
-                                                         const float* __restrict__ bias,
+                                                         const W* __restrict__ weight, const W* __restrict__ bias,
                                                          const _Float16* __restrict__ scale,
                                                          const _Float16* __restrict__ shift, int act,
                                                          _Float16* __restrict__ out) {
@@ -136,7 +147,7 @@ __global__ __launch_bounds__(256) void ln_generic_kernel(const _Float16* __restr
   _Float16* orow = out + row * c;
   for (int i = lane; i < c; i += 64) {
     float y = (static_cast<float>(xr[i]) - mean) * inv;
-    if (weight != nullptr) y = y * weight[i] + bias[i];
+    if (weight != nullptr) y = y * static_cast<float>(weight[i]) + static_cast<float>(bias[i]);
     _Float16 h = static_cast<_Float16>(f32_rounded(y));
     if (scale != nullptr) {
       const _Float16 p = static_cast<_Float16>(static_cast<float>(h) * static_cast<float>(scale[i]));
@@ -336,33 +347,62 @@ __global__ __launch_bounds__(256) void ln_quant_kernel(const _Float16* __restric
   }
 }
 
-// One wave per output feature: y = W . cond' + b (fp32), then the fp16 (1 + scale) and
-// shift halves.
-__global__ __launch_bounds__(256) void adaln_kernel(const float* __restrict__ w, const float* __restrict__ b,
-                                                    const float* __restrict__ cond, int n_out, int n_in, int apply_silu,
+// One wave per output feature and batch element (blockIdx.y): y = W . cond' + b in fp32,
+// then the fp16 (1 + scale) and shift halves. Parameters and cond in their own types
+// (16-bit values convert exactly); a lane's loads go out eight at a time, its sum stays in
+// column order.
+template <typename W, typename C>
+__global__ __launch_bounds__(256) void adaln_kernel(const W* __restrict__ w, const W* __restrict__ b,
+                                                    const C* __restrict__ cond, int n_out, int n_in, int apply_silu,
                                                     _Float16* __restrict__ scale1p, _Float16* __restrict__ shift) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (j >= n_out) return;
-  const float* wr = w + static_cast<int64_t>(j) * n_in;
+  const W* wr = w + static_cast<int64_t>(j) * n_in;
+  const C* cr = cond + static_cast<int64_t>(blockIdx.y) * n_in;
   float acc = 0.0f;
-  for (int i = lane; i < n_in; i += 64) {
-    float ci = cond[i];
-    if (apply_silu) ci = ci / (1.0f + expf(-ci));
-    acc += wr[i] * ci;
+  for (int i0 = lane; i0 < n_in; i0 += 64 * 8) {
+    float wv[8], cv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = i0 + 64 * u < n_in ? i0 + 64 * u : i0;
+      wv[u] = static_cast<float>(wr[i]);
+      cv[u] = static_cast<float>(cr[i]);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      float ci = cv[u];
+      if (apply_silu) ci = ci / (1.0f + expf(-ci));
+      if (i0 + 64 * u < n_in) acc += wv[u] * ci;
+    }
   }
   for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
   if (lane != 0) return;
-  const float y = acc + (b != nullptr ? b[j] : 0.0f);
+  const float y = acc + (b != nullptr ? static_cast<float>(b[j]) : 0.0f);
   const int half = n_out / 2;
   const _Float16 yh = static_cast<_Float16>(y);
-  if (j < half) scale1p[j] = static_cast<_Float16>(1.0f + static_cast<float>(yh));
-  else shift[j - half] = yh;
+  const int64_t row = static_cast<int64_t>(blockIdx.y) * half;
+  if (j < half) scale1p[row + j] = static_cast<_Float16>(1.0f + static_cast<float>(yh));
+  else shift[row + j - half] = yh;
 }
 
-template <int G, int CPL, bool kSilu>
-void launch_ln(const _Float16* x, int64_t rows, int c, float eps, const float* w, const float* b, const _Float16* sc,
+template <typename W>
+void launch_adaln(const void* w, const void* b, const void* cond, int cond_dtype, int batches, int n_out, int n_in,
+                  int apply_silu, _Float16* scale1p, _Float16* shift, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4)), static_cast<unsigned>(batches));
+  auto launch = [&](auto* c) {
+    using C = std::remove_const_t<std::remove_pointer_t<decltype(c)>>;
+    hipLaunchKernelGGL((adaln_kernel<W, C>), grid, dim3(256), 0, stream, static_cast<const W*>(w), static_cast<const W*>(b),
+                       c, n_out, n_in, apply_silu, scale1p, shift);
+  };
+  if (cond_dtype == HI3D_F16) launch(static_cast<const _Float16*>(cond));
+  else if (cond_dtype == HI3D_BF16) launch(static_cast<const __bf16*>(cond));
+  else launch(static_cast<const float*>(cond));
+}
+
+template <int G, int CPL, bool kSilu, typename W>
+void launch_ln(const _Float16* x, int64_t rows, int c, float eps, const W* w, const W* b, const _Float16* sc,
                const _Float16* sh, _Float16* out, hipStream_t stream) {
   constexpr int RPB = 256 / G;
   const int64_t groups = ceil_div(rows, RPB);
@@ -370,21 +410,21 @@ void launch_ln(const _Float16* x, int64_t rows, int c, float eps, const float* w
   const int64_t cap = static_cast<int64_t>(cus > 0 ? cus : 256) * 16;  // a few strides per block
   const dim3 grid(static_cast<unsigned>(groups < cap ? groups : cap));
   if (w != nullptr && sc != nullptr)
-    hipLaunchKernelGGL((ln_kernel<G, CPL, true, true, kSilu>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc, sh,
+    hipLaunchKernelGGL((ln_kernel<G, CPL, true, true, kSilu, W>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc, sh,
                        out);
   else if (w != nullptr)
-    hipLaunchKernelGGL((ln_kernel<G, CPL, true, false, kSilu>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc,
+    hipLaunchKernelGGL((ln_kernel<G, CPL, true, false, kSilu, W>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc,
                        sh, out);
   else if (sc != nullptr)
-    hipLaunchKernelGGL((ln_kernel<G, CPL, false, true, kSilu>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc,
+    hipLaunchKernelGGL((ln_kernel<G, CPL, false, true, kSilu, W>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc,
                        sh, out);
   else
-    hipLaunchKernelGGL((ln_kernel<G, CPL, false, false, kSilu>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc,
+    hipLaunchKernelGGL((ln_kernel<G, CPL, false, false, kSilu, W>), grid, dim3(256), 0, stream, x, rows, c, eps, w, b, sc,
                        sh, out);
 }
 
-template <bool kSilu>
-void launch_ln_width(const _Float16* xh, int64_t rows, int c, float eps, const float* weight, const float* bias,
+template <bool kSilu, typename W>
+void launch_ln_width(const _Float16* xh, int64_t rows, int c, float eps, const W* weight, const W* bias,
                      const _Float16* sc, const _Float16* sh, _Float16* o, hipStream_t stream) {
   const int chunks = c / 8;
   if (chunks <= 4) launch_ln<4, 1, kSilu>(xh, rows, c, eps, weight, bias, sc, sh, o, stream);
@@ -443,7 +483,8 @@ void launch_ln_quant_width(const _Float16* x, int64_t rows, int c, float eps, co
   else launch_ln_quant<64, 8, kRotate>(x, rows, c, eps, w, b, sc, sh, signs, q, qs, stream);
 }
 
-int layer_norm(const void* x, int64_t rows, int32_t c, float eps, const float* weight, const float* bias,
+template <typename W>
+int layer_norm(const void* x, int64_t rows, int32_t c, float eps, const W* weight, const W* bias,
                const void* scale, const void* shift, int32_t act, void* out, hipStream_t stream) {
   HI3D_REQUIRE(rows >= 0 && c > 0, "bad sizes");
   HI3D_REQUIRE((weight == nullptr) == (bias == nullptr), "weight and bias must be given together");
@@ -462,7 +503,7 @@ int layer_norm(const void* x, int64_t rows, int32_t c, float eps, const float* w
     if (act == HI3D_ACT_SILU) launch_ln_width<true>(xh, rows, c, eps, weight, bias, sc, sh, o, stream);
     else launch_ln_width<false>(xh, rows, c, eps, weight, bias, sc, sh, o, stream);
   } else {
-    hipLaunchKernelGGL(ln_generic_kernel, dim3(static_cast<unsigned>(ceil_div(rows, 4))), dim3(256), 0, stream, xh, rows,
+    hipLaunchKernelGGL(ln_generic_kernel<W>, dim3(static_cast<unsigned>(ceil_div(rows, 4))), dim3(256), 0, stream, xh, rows,
                        c, eps, weight, bias, sc, sh, act, o);
   }
   HI3D_LAUNCH_CHECK();
@@ -484,6 +525,12 @@ int hi3d_layer_norm_modulate(const void* x, int64_t rows, int32_t c, float eps, 
 int hi3d_layer_norm_act(const void* x, int64_t rows, int32_t c, float eps, const float* weight, const float* bias,
                         const void* scale, const void* shift, int32_t act, void* out, void* stream) {
   return layer_norm(x, rows, c, eps, weight, bias, scale, shift, act, out, as_stream(stream));
+}
+
+int hi3d_layer_norm_act_h(const void* x, int64_t rows, int32_t c, float eps, const void* weight, const void* bias,
+                          const void* scale, const void* shift, int32_t act, void* out, void* stream) {
+  return layer_norm(x, rows, c, eps, static_cast<const _Float16*>(weight), static_cast<const _Float16*>(bias), scale,
+                    shift, act, out, as_stream(stream));
 }
 
 int hi3d_layer_norm_quantize(const void* x, int64_t rows, int32_t c, float eps, const float* weight, const float* bias,
@@ -511,15 +558,28 @@ int hi3d_layer_norm_quantize(const void* x, int64_t rows, int32_t c, float eps, 
   return HI3D_OK;
 }
 
-int hi3d_adaln_projection(const float* w, const float* b, const float* cond, int32_t n_out, int32_t n_in,
-                          int32_t apply_silu, void* scale1p, void* shift, void* stream_) {
+int hi3d_adaln_modulation(const void* w, const void* b, int32_t param_dtype, const void* cond, int32_t cond_dtype,
+                          int32_t batches, int32_t n_out, int32_t n_in, int32_t apply_silu, void* scale1p, void* shift,
+                          void* stream_) {
   hipStream_t stream = as_stream(stream_);
   HI3D_REQUIRE(n_out > 0 && n_out % 2 == 0 && n_in > 0, "n_out must be even and positive, n_in positive");
+  HI3D_REQUIRE(batches >= 0 && batches <= 65535, "batches must be 0..65535 (got %d)", batches);
+  for (const int32_t d : {param_dtype, cond_dtype})
+    HI3D_REQUIRE(d == HI3D_F32 || d == HI3D_F16 || d == HI3D_BF16, "unsupported dtype %d", d);
+  if (batches == 0) return HI3D_OK;
   HI3D_REQUIRE(w && cond && scale1p && shift, "null pointer argument");
-  hipLaunchKernelGGL(adaln_kernel, dim3(static_cast<unsigned>(ceil_div(n_out, 4))), dim3(256), 0, stream, w, b, cond,
-                     n_out, n_in, apply_silu, static_cast<_Float16*>(scale1p), static_cast<_Float16*>(shift));
+  auto* s1 = static_cast<_Float16*>(scale1p);
+  auto* sh = static_cast<_Float16*>(shift);
+  if (param_dtype == HI3D_F16) launch_adaln<_Float16>(w, b, cond, cond_dtype, batches, n_out, n_in, apply_silu, s1, sh, stream);
+  else if (param_dtype == HI3D_BF16) launch_adaln<__bf16>(w, b, cond, cond_dtype, batches, n_out, n_in, apply_silu, s1, sh, stream);
+  else launch_adaln<float>(w, b, cond, cond_dtype, batches, n_out, n_in, apply_silu, s1, sh, stream);
   HI3D_LAUNCH_CHECK();
   return HI3D_OK;
+}
+
+int hi3d_adaln_projection(const float* w, const float* b, const float* cond, int32_t n_out, int32_t n_in,
+                          int32_t apply_silu, void* scale1p, void* shift, void* stream) {
+  return hi3d_adaln_modulation(w, b, HI3D_F32, cond, HI3D_F32, 1, n_out, n_in, apply_silu, scale1p, shift, stream);
 }
 
 }  // extern "C"

@@ -12,6 +12,8 @@ import torch
 
 from . import _lib
 
+_PARAMS = (torch.float32, torch.float16, torch.bfloat16)
+
 
 def layer_norm_modulate(
     x: torch.Tensor,
@@ -33,8 +35,13 @@ def layer_norm_modulate(
     c = int(x.shape[-1])
     rows = x.numel() // c if c else 0
     xc = x.contiguous()
-    w = None if weight is None else weight.to(torch.float32).reshape(-1).contiguous()
-    b = None if bias is None else bias.to(torch.float32).reshape(-1).contiguous()
+    w = None if weight is None else weight.reshape(-1).contiguous()
+    b = None if bias is None else bias.reshape(-1).contiguous()
+    # fp16 parameters are read as they are (where a copy would not have been better aligned)
+    half = all(t is not None and t.dtype == torch.float16 and t.data_ptr() % 16 == 0 for t in (w, b))
+    if not half:
+        w = None if w is None else w.to(torch.float32)
+        b = None if b is None else b.to(torch.float32)
     if (w is None) != (b is None):
         raise ValueError("weight and bias must be given together")
     sc = None if scale is None else scale.to(torch.float16).reshape(-1).contiguous()
@@ -46,7 +53,7 @@ def layer_norm_modulate(
             raise ValueError(f"per-channel parameters must have {c} entries")
     out = torch.empty_like(xc)
     _lib.call(
-        "hi3d_layer_norm_act",
+        "hi3d_layer_norm_act_h" if half else "hi3d_layer_norm_act",
         _lib.ptr(xc), rows, c, float(eps), _lib.ptr(w), _lib.ptr(b), _lib.ptr(sc), _lib.ptr(sh),
         _lib.ACT_SILU if act == "silu" else _lib.ACT_NONE, _lib.ptr(out), _lib.stream(device),
     )
@@ -74,6 +81,34 @@ def adaln_projection(
         "hi3d_adaln_projection",
         _lib.ptr(w), _lib.ptr(b), _lib.ptr(c), n_out, n_in, int(bool(apply_silu)), _lib.ptr(scale1p), _lib.ptr(shift),
         _lib.stream(device),
+    )
+    return scale1p, shift
+
+
+def adaln_modulation(
+    weight: torch.Tensor, bias: torch.Tensor | None, cond: torch.Tensor, apply_silu: bool = False
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """:func:`adaln_projection` of every row of ``cond [B, n_in]`` in one launch:
+    ``(fp16(1 + scale), shift)``, both ``[B, n_out / 2]``, with the same bits. Parameters and
+    ``cond`` are read in their own floating-point types."""
+    device = _lib.require_gpu(weight, bias, cond)
+    if bias is not None and bias.dtype != weight.dtype:
+        weight, bias = weight.float(), bias.float()
+    w = (weight if weight.dtype in _PARAMS else weight.float()).contiguous()
+    b = None if bias is None else (bias if bias.dtype in _PARAMS else bias.float()).reshape(-1).contiguous()
+    c = (cond if cond.dtype in _PARAMS else cond.float()).contiguous()
+    n_out, n_in = int(w.shape[0]), int(w.shape[1])
+    if n_out % 2:
+        raise ValueError("the projection must produce an even number of features")
+    if c.dim() != 2 or int(c.shape[1]) != n_in:
+        raise ValueError(f"cond must have {n_in} entries")
+    batches = int(c.shape[0])
+    scale1p = torch.empty((batches, n_out // 2), dtype=torch.float16, device=device)
+    shift = torch.empty((batches, n_out // 2), dtype=torch.float16, device=device)
+    _lib.call(
+        "hi3d_adaln_modulation",
+        _lib.ptr(w), _lib.ptr(b), _lib.DTYPES[w.dtype], _lib.ptr(c), _lib.DTYPES[c.dtype], batches, n_out, n_in,
+        int(bool(apply_silu)), _lib.ptr(scale1p), _lib.ptr(shift), _lib.stream(device),
     )
     return scale1p, shift
 

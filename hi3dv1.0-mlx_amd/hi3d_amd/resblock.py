@@ -38,7 +38,7 @@ from torch import nn
 from . import conv as _conv
 from . import kmap as _kmap
 from . import spconv as _spconv
-from .kernels import adaln_projection, layer_norm_modulate
+from .kernels import adaln_modulation, layer_norm_modulate
 from .nn import SparseConv3d, SparseDownsample, SparseTensor, SparseUpsample
 
 
@@ -96,19 +96,19 @@ class SparseResBlock3d(nn.Module):
         elif upsample:
             self.updown = SparseUpsample(2)
 
-    def _modulation(self, embedding: torch.Tensor, batches: int) -> list[tuple[torch.Tensor, torch.Tensor]]:
-        """``(fp16(1 + scale), shift)`` of each batch element from ``SiLU -> Linear``."""
+    def _modulation(self, embedding: torch.Tensor, batches: int) -> tuple[torch.Tensor, torch.Tensor]:
+        """``(fp16(1 + scale), shift)`` ``[B, hidden]`` from ``SiLU -> Linear``."""
         emb = embedding.reshape(embedding.shape[0], -1) if embedding.dim() > 1 else embedding.reshape(1, -1)
         if emb.shape[0] != batches:
             raise ValueError(f"embedding holds {emb.shape[0]} rows for {batches} batch elements")
         proj = self.emb_layers[1]
-        return [adaln_projection(proj.weight.detach(), None if proj.bias is None else proj.bias.detach(), emb[b],
-                                 apply_silu=True) for b in range(batches)]
+        return adaln_modulation(proj.weight.detach(), None if proj.bias is None else proj.bias.detach(), emb,
+                                apply_silu=True)
 
     def forward(self, x: SparseTensor, embedding: torch.Tensor) -> SparseTensor:
         if x.feats.dtype != torch.float16 or x.feats.dim() != 2:
             raise NotImplementedError("the fused residual block takes fp16 feature rows [N, C] (the fp16 torso)")
-        modulation = self._modulation(embedding, int(x.shape[0]))
+        scale1p, shift = self._modulation(embedding, int(x.shape[0]))
         if self.updown is not None:
             x = self.updown(x)
         plan, rows = _plan_pair(self.conv1.conv, x)
@@ -119,16 +119,14 @@ class SparseResBlock3d(nn.Module):
         w1 = _half(c1.weight).reshape(self.hidden_channels, 27, -1)
         if _conv.conv_ln_silu_supported(h.dtype, self.channels, self.hidden_channels, plan.kvol) and not _conv.HALO:
             # conv1 with norm2, the modulation of each row's batch and SiLU in its epilogue
-            h = _conv.conv_ln_silu(h, plan, w1, _half(c1.bias), x.coords, torch.stack([m[0] for m in modulation]),
-                                   torch.stack([m[1] for m in modulation]), self.norm2.eps)
+            h = _conv.conv_ln_silu(h, plan, w1, _half(c1.bias), x.coords, scale1p, shift, self.norm2.eps)
         else:
             h = _conv.conv(h, plan, w1, _half(c1.bias))
-            if len(modulation) == 1:
-                scale1p, shift = modulation[0]
-                h = layer_norm_modulate(h, self.norm2.eps, scale=scale1p, shift=shift, act="silu")
+            if len(scale1p) == 1:
+                h = layer_norm_modulate(h, self.norm2.eps, scale=scale1p[0], shift=shift[0], act="silu")
             else:
                 h = torch.cat([layer_norm_modulate(h[span], self.norm2.eps, scale=s, shift=t, act="silu")
-                               for span, (s, t) in zip(x.layout, modulation)])
+                               for span, s, t in zip(x.layout, scale1p, shift)])
         h = _conv.conv(h, plan, _half(c2.weight).reshape(self.hidden_channels, 27, -1), _half(c2.bias), act="silu")
         if isinstance(self.skip_connection, nn.Linear):
             sw, sb = _half(self.skip_connection.weight), _half(self.skip_connection.bias)

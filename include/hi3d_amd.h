@@ -533,6 +533,11 @@ int hi3d_layer_norm_act(const void* x_dev, int64_t rows, int32_t c, float eps,
                         const void* scale_dev, const void* shift_dev, int32_t act,
                         void* out_dev, void* stream);
 
+/* hi3d_layer_norm_act with fp16 weight_dev and bias_dev [c]: the bits of their fp32 copies. */
+int hi3d_layer_norm_act_h(const void* x_dev, int64_t rows, int32_t c, float eps, const void* weight_dev,
+                          const void* bias_dev, const void* scale_dev, const void* shift_dev, int32_t act,
+                          void* out_dev, void* stream);
+
 /* The same LayerNorm (+ affine, + modulate) followed by the W8A8 activation quantiser
  * of its fp16 result, in one pass (the fp16 rows are not stored): q_dev [rows, c] int8
  * and q_scale_dev [rows] fp32, bitwise those of hi3d_layer_norm_modulate then
@@ -570,6 +575,13 @@ int hi3d_dense_linear(const void* x_dev, int64_t n, int32_t cin, const void* w_d
 int hi3d_adaln_projection(const float* w_dev, const float* b_dev, const float* cond_dev,
                           int32_t n_out, int32_t n_in, int32_t apply_silu, void* scale1p_dev,
                           void* shift_dev, void* stream);
+
+/* hi3d_adaln_projection of `batches` rows cond_dev [batches, n_in] in one launch, parameters
+ * (w_dev, b_dev) and cond_dev in F32, F16 or BF16: scale1p_dev and shift_dev
+ * [batches, n_out / 2] fp16, the bits of the projection of their fp32 copies. */
+int hi3d_adaln_modulation(const void* w_dev, const void* b_dev, int32_t param_dtype, const void* cond_dev,
+                          int32_t cond_dtype, int32_t batches, int32_t n_out, int32_t n_in, int32_t apply_silu,
+                          void* scale1p_dev, void* shift_dev, void* stream);
 
 #ifdef __cplusplus
 }

@@ -85,6 +85,41 @@ def test_adaln_projection(cuda):
     assert np.array_equal(sh.cpu().numpy(), cond[:256].astype(np.float16))
 
 
+@pytest.mark.parametrize("wdt,cdt", [(torch.float16, torch.float16), (torch.bfloat16, torch.float32),
+                                     (torch.float32, torch.bfloat16), (torch.float64, torch.float64)])
+@pytest.mark.parametrize("batches,n_out,n_in", [(1, 2, 1), (3, 256, 2112), (2, 10, 577), (5, 512, 512)])
+def test_adaln_modulation_equals_projection_of_each_row(cuda, wdt, cdt, batches, n_out, n_in):
+    """All batch elements in one launch, parameters in their own types: bitwise the
+    projection of each row's fp32 copy (rows around the eight loads a lane has in flight)."""
+    from hi3d_amd import kernels
+
+    rng = np.random.default_rng(n_in + batches)
+    w = torch.as_tensor(rng.standard_normal((n_out, n_in)) / np.sqrt(n_in)).to(cuda, wdt)
+    cond = torch.as_tensor(rng.standard_normal((batches, n_in))).to(cuda, cdt)
+    for b in (None, torch.as_tensor(rng.standard_normal(n_out)).to(cuda, wdt)):
+        for silu in (False, True):
+            s1p, sh = kernels.adaln_modulation(w, b, cond, silu)
+            assert s1p.shape == sh.shape == (batches, n_out // 2)
+            for i in range(batches):
+                ws, wh = kernels.adaln_projection(w, b, cond[i], silu)
+                assert torch.equal(s1p[i], ws) and torch.equal(sh[i], wh)
+
+
+@pytest.mark.parametrize("c", [32, 128, 256, 2112, 20])
+def test_layer_norm_fp16_parameters(cuda, c):
+    """fp16 weight and bias as they are (aligned, or in a view that is not): the bits of
+    their fp32 copies."""
+    from hi3d_amd import kernels
+
+    rng = np.random.default_rng(c)
+    x = torch.as_tensor(rng.standard_normal((77, c)).astype(np.float16)).to(cuda)
+    pad = torch.as_tensor(rng.standard_normal((2, c + 1)).astype(np.float16)).to(cuda)
+    for w, b in ((pad[0, :c].clone(), pad[1, :c].clone()), (pad[0, 1:], pad[1, 1:])):
+        for act in (None, "silu"):
+            got = kernels.layer_norm_modulate(x, 1e-6, weight=w, bias=b, act=act)
+            assert torch.equal(got, kernels.layer_norm_modulate(x, 1e-6, weight=w.float(), bias=b.float(), act=act))
+
+
 def _block_weights(rng, c, d, cuda):
     from hi3d_amd.block import ResBlockWeights
 
