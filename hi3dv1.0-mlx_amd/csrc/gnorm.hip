@@ -117,9 +117,22 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const float* __restr
   const int ch = blockIdx.x * 16 + j;
   double a = 0.0, b = 0.0;
   if (ch < c) {
-    for (int k = sl; k < blocks; k += 16) {
-      a += partial[(static_cast<int64_t>(k) * 2) * c + ch];
-      b += partial[(static_cast<int64_t>(k) * 2 + 1) * c + ch];
+    // eight partials' loads in flight, added in order (one after another each addition
+    // waited for its load: 22 us for 1024 partials)
+    for (int k = sl; k < blocks; k += 16 * 8) {
+      float pa[8], pb[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int64_t r = k + 16 * u < blocks ? k + 16 * u : k;
+        pa[u] = partial[(r * 2) * c + ch];
+        pb[u] = partial[(r * 2 + 1) * c + ch];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const bool in = k + 16 * u < blocks;  // a sum is never -0, so adding 0 keeps it
+        a += in ? pa[u] : 0.0f;
+        b += in ? pb[u] : 0.0f;
+      }
     }
   }
   red[0][sl][j] = a;

@@ -1218,71 +1218,118 @@ __global__ void stride2_tables_kernel(const int32_t* __restrict__ inverse,
 }
 
 // ---------------------------------------------------------------- child table --
-// For child slot s and offset k: parent-neighbourhood offset holding the neighbour
-// (pk) and the neighbour's own slot (ss); same construction as the reference's
-// _child_offset_tables (sparse.py:46-61).
-struct ChildTables {
-  int8_t pk[8][27];
-  int8_t ss[8][27];
-};
+// Child cells of a parent's neighbourhood: cell (x, y, z), each 0..3, lies at child
+// coordinates 2 p + (x, y, z) - 1, i.e. in the parent neighbour of offset
+// ((x + 1) / 2, (y + 1) / 2, (z + 1) / 2) and its slot ((x + 1) & 1, ..): the
+// _child_offset_tables of sparse.py:46-61. The 27 neighbours of the child in slot s are the
+// cells s + (0..2, 0..2, 0..2) (with s = (s / 4, s / 2 % 2, s % 2)).
 
-ChildTables make_child_tables() {
-  ChildTables t;
-  for (int s = 0; s < 8; ++s) {
-    int bits[3] = {(s >> 2) & 1, (s >> 1) & 1, s & 1};
-    for (int k = 0; k < 27; ++k) {
-      int d[3] = {k / 9 - 1, (k / 3) % 3 - 1, k % 3 - 1};
-      int pd[3], cb[3];
-      for (int a = 0; a < 3; ++a) {
-        int v = bits[a] + d[a];  // in -1..2
-        pd[a] = v >> 1;          // floor division
-        cb[a] = v & 1;
-      }
-      t.pk[s][k] = static_cast<int8_t>((pd[0] + 1) * 9 + (pd[1] + 1) * 3 + (pd[2] + 1));
-      t.ss[s][k] = static_cast<int8_t>(cb[0] * 4 + cb[1] * 2 + cb[2]);
-    }
-  }
-  return t;
+// Bit s: byte s of a parent's occupancy is not zero.
+__device__ __forceinline__ uint32_t slot_bits(const uint8_t* mask) {
+  uint64_t x;
+  __builtin_memcpy(&x, mask, 8);
+  uint32_t bits = 0;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) bits |= ((x >> (8 * s)) & 0xff) != 0 ? 1u << s : 0u;
+  return bits;
 }
 
-__global__ void mask_to_int_kernel(const uint8_t* __restrict__ mask, int64_t m, int32_t* __restrict__ out) {
-  int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  out[i] = mask[i] ? 1 : 0;
+__global__ void child_count_kernel(const uint8_t* __restrict__ mask, int64_t parents, int32_t* __restrict__ out) {
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (p < parents) out[p] = __popc(slot_bits(mask + p * 8));
 }
 
-// ids = exclusive scan of the mask: lookup[p*8+s] = child index (or C), plus parent/slot.
-__global__ void child_index_kernel(const uint8_t* __restrict__ mask, const int32_t* __restrict__ excl,
-                                   int64_t m, int32_t* __restrict__ lookup,
+// excl = exclusive scan of the parents' counts. info[p] = (first child, slot bits), info[P]
+// = (C, none), and each child's parent and slot.
+__global__ void child_index_kernel(const uint8_t* __restrict__ mask, const int32_t* __restrict__ counts,
+                                   const int32_t* __restrict__ excl, int64_t parents, uint2* __restrict__ info,
                                    int32_t* __restrict__ parent, int32_t* __restrict__ slot,
                                    int64_t* __restrict__ n_children) {
-  int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const int32_t total = excl[m - 1] + (mask[m - 1] ? 1 : 0);
-  if (i == 0) *n_children = total;
-  if (mask[i]) {
-    const int32_t c = excl[i];
-    lookup[i] = c;
-    parent[c] = static_cast<int32_t>(i >> 3);
-    slot[c] = static_cast<int32_t>(i & 7);
-  } else {
-    lookup[i] = total;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= parents * 8) return;
+  const int64_t p = i >> 3;
+  const int s = static_cast<int>(i & 7);
+  const uint32_t bits = slot_bits(mask + p * 8);
+  if (s == 0) info[p] = make_uint2(static_cast<uint32_t>(excl[p]), bits);
+  if ((bits >> s) & 1u) {
+    const int32_t c = excl[p] + __popc(bits & ((1u << s) - 1u));
+    parent[c] = static_cast<int32_t>(p);
+    slot[c] = s;
   }
-  if (i < 8) lookup[m + i] = total;  // target of absent parents (row P)
+  if (i == 0) {
+    const int32_t total = excl[parents - 1] + counts[parents - 1];
+    *n_children = total;
+    info[parents] = make_uint2(static_cast<uint32_t>(total), 0u);
+  }
 }
 
-__global__ void child_table_kernel(const int32_t* __restrict__ parent_table, const int32_t* __restrict__ lookup,
-                                   const int32_t* __restrict__ parent, const int32_t* __restrict__ slot,
-                                   const int64_t* __restrict__ n_children, int64_t cap, ChildTables t,
-                                   int32_t* __restrict__ table) {
-  int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t c = j / 27;
-  if (c >= cap || c >= *n_children) return;
-  const int k = static_cast<int>(j - c * 27);
-  const int s = slot[c];
-  const int32_t p = parent[c];
-  const int32_t np = parent_table[static_cast<int64_t>(p) * 27 + t.pk[s][k]];
-  table[j] = lookup[static_cast<int64_t>(np) * 8 + t.ss[s][k]];
+// A wave takes kChildParents parents: lane l looks up cell l of each (their loads in
+// flight together), and the rows of a parent's children, which are consecutive, are read
+// from the lanes that hold their cells (places worked out once a wave: per entry they took
+// most of 85 us on 327,581 parents). One 8-byte gather a neighbour. One thread per table entry, for eight children a parent
+// whether present or not, took 165 us (three dependent loads an entry).
+constexpr int kChildParents = 4;
+
+__global__ __launch_bounds__(256) void child_table_kernel(const int32_t* __restrict__ parent_table,
+                                                          const uint2* __restrict__ info, int64_t parents,
+                                                          int32_t* __restrict__ table) {
+  const int lane = threadIdx.x & 63;
+  const int64_t p0 = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * kChildParents;
+  const int x = (lane >> 4) + 1, y = ((lane >> 2) & 3) + 1, z = (lane & 3) + 1;
+  const int pk = (x >> 1) * 9 + (y >> 1) * 3 + (z >> 1), ss = (x & 1) * 4 + (y & 1) * 2 + (z & 1);
+  const int32_t total = static_cast<int32_t>(info[parents].x);
+  // table entry 64 j + lane of a parent's rows: which child, and its neighbour's cell from
+  // the child's slot (entries past eight children take the last)
+  int child[4], near[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int t = min(j * 64 + lane, 8 * 27 - 1), k = t % 27;
+    child[j] = t / 27;
+    near[j] = k / 9 * 16 + k / 3 % 3 * 4 + k % 3;
+  }
+  int32_t np[kChildParents], cell[kChildParents];
+  uint32_t bits[kChildParents];
+#pragma unroll
+  for (int i = 0; i < kChildParents; ++i) {
+    const int64_t p = p0 + i < parents ? p0 + i : parents - 1;
+    np[i] = parent_table[p * 27 + pk];
+    bits[i] = p0 + i < parents ? info[p].y : 0;
+  }
+  uint2 q[kChildParents];
+#pragma unroll
+  for (int i = 0; i < kChildParents; ++i) q[i] = info[np[i]];
+#pragma unroll
+  for (int i = 0; i < kChildParents; ++i)
+    cell[i] = (q[i].y >> ss) & 1u ? static_cast<int32_t>(q[i].x) + __popc(q[i].y & ((1u << ss) - 1u)) : total;
+#pragma unroll
+  for (int i = 0; i < kChildParents; ++i) {
+    const uint32_t b = __builtin_amdgcn_readfirstlane(bits[i]);
+    if (b == 0) continue;
+    uint64_t slots = 0;  // the set slots' cells relative to slot 0's, in order, a byte each
+    int n = 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if ((b >> s) & 1u) slots |= static_cast<uint64_t>((s >> 2) * 16 + ((s >> 1) & 1) * 4 + (s & 1)) << (8 * n++);
+    // a child's own cell: offset 13 of its 27
+    const int64_t first = __builtin_amdgcn_readlane(cell[i], static_cast<int>(slots & 0xff) + 16 + 4 + 1);
+    int32_t* const out = table + first * 27;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j * 64 >= n * 27) break;
+      const int32_t v = __shfl(cell[i], (static_cast<int>(slots >> (8 * child[j])) & 0xff) + near[j], 64);
+      if (j * 64 + lane < n * 27) out[j * 64 + lane] = v;
+    }
+  }
+}
+
+// out[i] = 2 coords[parent[i]] + (slot bits 2, 1, 0)
+__global__ void child_coords_kernel(const int32_t* __restrict__ coords, const int32_t* __restrict__ parent,
+                                    const int32_t* __restrict__ slot, int64_t n, int32_t* __restrict__ out) {
+  const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (j >= n * 3) return;
+  const int64_t i = j / 3;
+  const int axis = static_cast<int>(j - i * 3);
+  out[j] = coords[static_cast<int64_t>(parent[i]) * 3 + axis] * 2 + ((slot[i] >> (2 - axis)) & 1);
 }
 
 // Hash table of hi3d_kmap_subm_noalloc: a device array of this library, one copy per GPU,
@@ -1807,11 +1854,22 @@ int hi3d_gather_rows(const void* in, int64_t n_in, int32_t row_bytes, const int3
   return HI3D_OK;
 }
 
+int hi3d_child_coords(const int32_t* coords, const int32_t* parent, const int32_t* slot, int64_t n, int32_t* out,
+                      void* stream) {
+  HI3D_REQUIRE(n >= 0 && n < (int64_t(1) << 31), "bad n");
+  if (n == 0) return HI3D_OK;
+  HI3D_REQUIRE(coords && parent && slot && out, "null pointer argument");
+  hipLaunchKernelGGL(child_coords_kernel, dim3(static_cast<unsigned>(ceil_div(n * 3, 256))), dim3(256), 0,
+                     as_stream(stream), coords, parent, slot, n, out);
+  HI3D_LAUNCH_CHECK();
+  return HI3D_OK;
+}
+
 int hi3d_child_table_workspace(int64_t n_parents, int64_t* bytes) {
   HI3D_REQUIRE(bytes != nullptr, "bytes_host is NULL");
   HI3D_REQUIRE(n_parents >= 0 && n_parents * 8 < (int64_t(1) << 31) - 16, "bad n_parents");
-  const int64_t m = std::max<int64_t>(n_parents * 8, 1);
-  *bytes = 2 * align_up(m * 4, 256) + align_up((m + 8) * 4, 256) + radix::temp_bytes(m);
+  const int64_t p = std::max<int64_t>(n_parents, 1);
+  *bytes = 2 * align_up(p * 4, 256) + align_up((p + 1) * 8, 256) + radix::temp_bytes(p);
   return HI3D_OK;
 }
 
@@ -1830,21 +1888,19 @@ int hi3d_child_neighbour_table(const int32_t* parent_table, const uint8_t* mask,
   }
   HI3D_REQUIRE(parent_table && mask && table && parent && slot && workspace, "null pointer argument");
   HI3D_REQUIRE(workspace_bytes >= need, "workspace too small");
-  const int64_t m = n_parents * 8;
   Workspace ws(workspace, workspace_bytes);
-  int32_t* flags = ws.take<int32_t>(m);
-  int32_t* excl = ws.take<int32_t>(m);
-  int32_t* lookup = ws.take<int32_t>(m + 8);
-  const int64_t scan_bytes = radix::temp_bytes(m);
+  int32_t* counts = ws.take<int32_t>(n_parents);
+  int32_t* excl = ws.take<int32_t>(n_parents);
+  uint2* info = ws.take<uint2>(n_parents + 1);
+  const int64_t scan_bytes = radix::temp_bytes(n_parents);
   void* temp = ws.take<char>(scan_bytes);
-  const unsigned blocks = static_cast<unsigned>(ceil_div(m, 256));
-  hipLaunchKernelGGL(mask_to_int_kernel, dim3(blocks), dim3(256), 0, stream, mask, m, flags);
-  HI3D_HIP_CHECK(radix::scan(temp, scan_bytes, flags, excl, m, false, stream));
-  hipLaunchKernelGGL(child_index_kernel, dim3(blocks), dim3(256), 0, stream, mask, excl, m, lookup, parent, slot,
-                     n_children);
-  static const ChildTables tables = make_child_tables();
-  hipLaunchKernelGGL(child_table_kernel, dim3(static_cast<unsigned>(ceil_div(m * 27, 256))), dim3(256), 0, stream,
-                     parent_table, lookup, parent, slot, n_children, m, tables, table);
+  auto blocks = [](int64_t n) { return dim3(static_cast<unsigned>(ceil_div(n, 256))); };
+  hipLaunchKernelGGL(child_count_kernel, blocks(n_parents), dim3(256), 0, stream, mask, n_parents, counts);
+  HI3D_HIP_CHECK(radix::scan(temp, scan_bytes, counts, excl, n_parents, false, stream));
+  hipLaunchKernelGGL(child_index_kernel, blocks(n_parents * 8), dim3(256), 0, stream, mask, counts, excl, n_parents, info,
+                     parent, slot, n_children);
+  hipLaunchKernelGGL(child_table_kernel, blocks(ceil_div(n_parents, kChildParents) * 64), dim3(256), 0, stream, parent_table,
+                     info, n_parents, table);
   HI3D_LAUNCH_CHECK();
   return HI3D_OK;
 }

@@ -45,6 +45,7 @@ _SIGNATURES = {
     "hi3d_resample_down_table": [_p, _p, _i64, _i64, _i32, _p, _p],
     "hi3d_child_table_workspace": [_i64, _p],
     "hi3d_child_neighbour_table": [_p, _p, _i64, _p, _i64, _p, _p, _p, _p, _p],
+    "hi3d_child_coords": [_p, _p, _p, _i64, _p, _p],
     "hi3d_conv_tile_rows": [],
     "hi3d_conv_plan_workspace": [_i64, _p],
     "hi3d_conv_plan": [_p, _i64, _i32, _i64, _p, _i32, _i32, _i64, _p, _i64, _p, _p, _p, _p],

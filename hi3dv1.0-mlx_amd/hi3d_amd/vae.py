@@ -209,8 +209,10 @@ def upsample(x: torch.Tensor, level: Level, params: dict, name: str, out: torch.
     table, parent, slot = child_neighbour_table(level.table, mask)
     w = params[f"{name}.proj.weight"]
     y = children(x, parent, slot, w, out=out if out is not None else x.dtype)
-    coords = level.coords.to(table.device, torch.int32)
-    sl = slot.to(torch.int32)
-    bits = torch.stack([(sl >> 2) & 1, (sl >> 1) & 1, sl & 1], 1)
-    child_coords = coords[parent.long()] * 2 + bits
+    coords = level.coords.to(table.device, torch.int32).contiguous()
+    if tuple(coords.shape) != (int(level.table.shape[0]), 3):
+        raise ValueError(f"level coordinates must be [{int(level.table.shape[0])}, 3], got {tuple(coords.shape)}")
+    child_coords = torch.empty((int(parent.shape[0]), 3), dtype=torch.int32, device=table.device)
+    _lib.call("hi3d_child_coords", _lib.ptr(coords), _lib.ptr(parent), _lib.ptr(slot), int(parent.shape[0]),
+              _lib.ptr(child_coords), _lib.stream(table.device))
     return y, Level(child_coords, table), mask

@@ -245,6 +245,12 @@ int hi3d_child_neighbour_table(const int32_t* parent_table_dev, const uint8_t* m
                                int32_t* table_dev, int32_t* parent_dev, int32_t* slot_dev,
                                int64_t* n_children_dev, void* stream);
 
+/* Children's coordinates: out_dev[i] = 2 coords_dev[parent_dev[i]] + (slot bits 2, 1, 0),
+ * coords_dev [P, 3], out_dev [n, 3]. Replaces the coordinate arithmetic of the octree
+ * upsampling (src/hi3d_mac/mlx_backend/vae.py:316-327). */
+int hi3d_child_coords(const int32_t* coords_dev, const int32_t* parent_dev, const int32_t* slot_dev, int64_t n,
+                      int32_t* out_dev, void* stream);
+
 /* ------------------------------------------------------------ convolution plans -- */
 
 /* Rows per tile of the gather-MFMA convolution. */

@@ -226,6 +226,31 @@ def test_mlx_shaped_helpers(cuda):
     assert np.array_equal(cnt.cpu().numpy(), rc)
 
 
+@pytest.mark.parametrize("parents,fill", [(1, 1.0), (2, 0.0), (3, 0.5), (4, 1.0), (5, 0.2), (17, 0.4), (1000, 0.42), (1003, 1.0)])
+def test_child_table_and_coords(cuda, parents, fill):
+    """Parent counts around the four parents of a wave, no / some / all slots kept (eight
+    children's rows are 216 entries, four passes of a wave), and occupancy bytes other than
+    1: table, parents, slots and coordinates against the oracle."""
+    from hi3d_amd import _lib, sparse
+
+    rng = np.random.default_rng(parents)
+    side = max(2, round((2.5 * parents) ** (1 / 3)) + 1)
+    cells = rng.permutation(side ** 3)[:parents]
+    coords = np.stack([cells // side ** 2, cells // side % side, cells % side], 1).astype(np.int32)
+    table = okmap.neighbour_table_dense(coords)
+    mask = (rng.random((parents, 8)) < fill).astype(np.uint8)
+    ct, par, slot = okmap.child_neighbour_table(table, mask > 0)
+    got = sparse.child_neighbour_table(torch.as_tensor(table).to(cuda), torch.as_tensor(mask * 130).to(cuda))
+    for g, w in zip(got, (ct, par, slot)):
+        assert np.array_equal(g.cpu().numpy(), w)
+    out = torch.empty((len(par), 3), dtype=torch.int32, device=cuda)
+    c = torch.as_tensor(coords).to(cuda)
+    _lib.call("hi3d_child_coords", _lib.ptr(c), _lib.ptr(got[1]), _lib.ptr(got[2]), len(par), _lib.ptr(out),
+              _lib.stream(c.device))
+    bits = np.stack([slot >> 2 & 1, slot >> 1 & 1, slot & 1], 1)
+    assert np.array_equal(out.cpu().numpy(), coords[par] * 2 + bits)
+
+
 def test_plan_covers_every_row_once(cuda):
     from hi3d_amd import kmap, workloads
 
