@@ -1868,8 +1868,10 @@ int hi3d_child_coords(const int32_t* coords, const int32_t* parent, const int32_
 int hi3d_child_table_workspace(int64_t n_parents, int64_t* bytes) {
   HI3D_REQUIRE(bytes != nullptr, "bytes_host is NULL");
   HI3D_REQUIRE(n_parents >= 0 && n_parents * 8 < (int64_t(1) << 31) - 16, "bad n_parents");
-  const int64_t p = std::max<int64_t>(n_parents, 1);
-  *bytes = 2 * align_up(p * 4, 256) + align_up((p + 1) * 8, 256) + radix::temp_bytes(p);
+  // more than the parents' counts, scan and (first child, slots) pairs take: the size stays
+  // the 12 bytes per slot that callers have been given
+  const int64_t m = std::max<int64_t>(n_parents * 8, 1);
+  *bytes = 2 * align_up(m * 4, 256) + align_up((m + 8) * 4, 256) + radix::temp_bytes(m);
   return HI3D_OK;
 }
 

@@ -43,8 +43,12 @@ constexpr int64_t kFewKeys = int64_t(1) << 20;
 inline int sort_items(int64_t n) { return n <= kFewKeys ? kFewItems : kItems; }
 inline int64_t sort_tiles(int64_t n) { return std::max<int64_t>(ceil_div(n, kThreads * sort_items(n)), 1); }
 
-// Workspace bytes of sort_pairs and scan for n elements: per-tile counts and totals.
-inline int64_t temp_bytes(int64_t n) { return align_up(sort_tiles(n) * kBins * 4, 256) + align_up(kBins * 4, 256); }
+// Workspace bytes of sort_pairs and scan for up to n elements (a smaller set may have more
+// tiles): per-tile counts and totals.
+inline int64_t temp_bytes(int64_t n) {
+  const int64_t most = std::max(sort_tiles(n), sort_tiles(std::min(n, kFewKeys)));
+  return align_up(most * kBins * 4, 256) + align_up(kBins * 4, 256);
+}
 
 // Exclusive prefix of v over the block's 256 threads; *total gets the sum. part holds
 // kWaves ints of LDS; the function ends with a barrier, so part can be reused.
