@@ -1266,8 +1266,9 @@ __global__ void child_index_kernel(const uint8_t* __restrict__ mask, const int32
 // A wave takes kChildParents parents: lane l looks up cell l of each (their loads in
 // flight together), and the rows of a parent's children, which are consecutive, are read
 // from the lanes that hold their cells (places worked out once a wave: per entry they took
-// most of 85 us on 327,581 parents). One 8-byte gather a neighbour. One thread per table entry, for eight children a parent
-// whether present or not, took 165 us (three dependent loads an entry).
+// most of 85 us on 327,581 parents). One 8-byte gather a neighbour. Where the rows go comes
+// from the scan alone, whatever the table holds. One thread per table entry, for eight
+// children a parent whether present or not, took 165 us (three dependent loads an entry).
 constexpr int kChildParents = 4;
 
 __global__ __launch_bounds__(256) void child_table_kernel(const int32_t* __restrict__ parent_table,
@@ -1288,12 +1289,12 @@ __global__ __launch_bounds__(256) void child_table_kernel(const int32_t* __restr
     near[j] = k / 9 * 16 + k / 3 % 3 * 4 + k % 3;
   }
   int32_t np[kChildParents], cell[kChildParents];
-  uint32_t bits[kChildParents];
+  uint2 own[kChildParents];  // the parent's first child and slots (past the last parent: no slots)
 #pragma unroll
   for (int i = 0; i < kChildParents; ++i) {
     const int64_t p = p0 + i < parents ? p0 + i : parents - 1;
     np[i] = parent_table[p * 27 + pk];
-    bits[i] = p0 + i < parents ? info[p].y : 0;
+    own[i] = info[p0 + i < parents ? p : parents];
   }
   uint2 q[kChildParents];
 #pragma unroll
@@ -1303,15 +1304,14 @@ __global__ __launch_bounds__(256) void child_table_kernel(const int32_t* __restr
     cell[i] = (q[i].y >> ss) & 1u ? static_cast<int32_t>(q[i].x) + __popc(q[i].y & ((1u << ss) - 1u)) : total;
 #pragma unroll
   for (int i = 0; i < kChildParents; ++i) {
-    const uint32_t b = __builtin_amdgcn_readfirstlane(bits[i]);
+    const uint32_t b = __builtin_amdgcn_readfirstlane(own[i].y);
     if (b == 0) continue;
     uint64_t slots = 0;  // the set slots' cells relative to slot 0's, in order, a byte each
     int n = 0;
 #pragma unroll
     for (int s = 0; s < 8; ++s)
       if ((b >> s) & 1u) slots |= static_cast<uint64_t>((s >> 2) * 16 + ((s >> 1) & 1) * 4 + (s & 1)) << (8 * n++);
-    // a child's own cell: offset 13 of its 27
-    const int64_t first = __builtin_amdgcn_readlane(cell[i], static_cast<int>(slots & 0xff) + 16 + 4 + 1);
+    const int64_t first = __builtin_amdgcn_readfirstlane(own[i].x);
     int32_t* const out = table + first * 27;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {

@@ -251,6 +251,33 @@ def test_child_table_and_coords(cuda, parents, fill):
     assert np.array_equal(out.cpu().numpy(), coords[par] * 2 + bits)
 
 
+def test_child_table_places_rows_by_the_scan(cuda):
+    """A caller's own table whose centre entries are absent, or name another parent: each
+    child's row still lies at the child's own index, and no row past the last child is
+    written (the rows after them keep what they held)."""
+    from hi3d_amd import _lib
+
+    rng = np.random.default_rng(9)
+    p = 203
+    table = rng.integers(0, p + 1, (p, 27)).astype(np.int32)  # any parent or absent, at any offset
+    table[::3, 13] = p
+    mask = (rng.random((p, 8)) < 0.6).astype(np.uint8)
+    mask[:40] = 1
+    ct, par, slot = okmap.child_neighbour_table(table, mask > 0)
+    c = len(par)
+    t, m = torch.as_tensor(table).to(cuda), torch.as_tensor(mask).to(cuda)
+    out = torch.full((8 * p + 16, 27), -7, dtype=torch.int32, device=cuda)
+    parent, child_slot = (torch.empty(8 * p, dtype=torch.int32, device=cuda) for _ in range(2))
+    n = torch.empty(1, dtype=torch.int64, device=cuda)
+    ws = _lib.workspace(_lib.query("hi3d_child_table_workspace", p), t.device)
+    _lib.call("hi3d_child_neighbour_table", _lib.ptr(t), _lib.ptr(m), p, _lib.ptr(ws), ws.numel(), _lib.ptr(out),
+              _lib.ptr(parent), _lib.ptr(child_slot), _lib.ptr(n), _lib.stream(t.device))
+    assert int(n.item()) == c
+    assert np.array_equal(parent[:c].cpu().numpy(), par) and np.array_equal(child_slot[:c].cpu().numpy(), slot)
+    assert np.array_equal(out[:c].cpu().numpy(), ct)
+    assert (out[c:] == -7).all()
+
+
 def test_plan_covers_every_row_once(cuda):
     from hi3d_amd import kmap, workloads
 
