@@ -1296,9 +1296,13 @@ __global__ __launch_bounds__(256) void child_table_kernel(const int32_t* __restr
     np[i] = parent_table[p * 27 + pk];
     own[i] = info[p0 + i < parents ? p : parents];
   }
+  // (every parent's row is read, also one without children, which may hold anything)
   uint2 q[kChildParents];
 #pragma unroll
-  for (int i = 0; i < kChildParents; ++i) q[i] = info[np[i]];
+  for (int i = 0; i < kChildParents; ++i) {
+    const uint32_t at = static_cast<uint32_t>(np[i]), absent = static_cast<uint32_t>(parents);
+    q[i] = info[at < absent ? at : absent];
+  }
 #pragma unroll
   for (int i = 0; i < kChildParents; ++i)
     cell[i] = (q[i].y >> ss) & 1u ? static_cast<int32_t>(q[i].x) + __popc(q[i].y & ((1u << ss) - 1u)) : total;

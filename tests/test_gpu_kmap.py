@@ -252,9 +252,10 @@ def test_child_table_and_coords(cuda, parents, fill):
 
 
 def test_child_table_places_rows_by_the_scan(cuda):
-    """A caller's own table whose centre entries are absent, or name another parent: each
-    child's row still lies at the child's own index, and no row past the last child is
-    written (the rows after them keep what they held)."""
+    """A caller's own table whose centre entries are absent, or name another parent, and
+    whose rows of parents without children hold anything: each child's row still lies at
+    the child's own index, and no row past the last child is written (the rows after them
+    keep what they held)."""
     from hi3d_amd import _lib
 
     rng = np.random.default_rng(9)
@@ -263,8 +264,10 @@ def test_child_table_places_rows_by_the_scan(cuda):
     table[::3, 13] = p
     mask = (rng.random((p, 8)) < 0.6).astype(np.uint8)
     mask[:40] = 1
+    mask[40:60] = 0
     ct, par, slot = okmap.child_neighbour_table(table, mask > 0)
     c = len(par)
+    table[40:50], table[50:60] = 1 << 30, -5  # rows of parents without children are never used
     t, m = torch.as_tensor(table).to(cuda), torch.as_tensor(mask).to(cuda)
     out = torch.full((8 * p + 16, 27), -7, dtype=torch.int32, device=cuda)
     parent, child_slot = (torch.empty(8 * p, dtype=torch.int32, device=cuda) for _ in range(2))
