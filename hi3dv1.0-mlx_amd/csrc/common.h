@@ -66,6 +66,12 @@ struct Workspace {
     used += count * static_cast<int64_t>(sizeof(T));
     return p;
   }
+  // everything that is left
+  void* rest(int64_t* bytes) {
+    void* p = take<char>(0);
+    *bytes = size - used;
+    return p;
+  }
   bool ok() const { return used <= size; }
 };
 

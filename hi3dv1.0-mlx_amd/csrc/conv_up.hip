@@ -363,6 +363,7 @@ int hi3d_stride2_up_plan(const int32_t* down, int64_t n_c, int64_t n_f, int32_t 
   HI3D_REQUIRE(n_f >= 0 && n_f < (int64_t(1) << 31) - 1, "bad fine row count");
   if (n_c == 0) return HI3D_OK;
   HI3D_REQUIRE(down && workspace && order && down_sorted, "null pointer argument");
+  need -= radix::spare_bytes(n_c);
   HI3D_REQUIRE(workspace_bytes >= need, "workspace too small: %lld < %lld bytes", static_cast<long long>(workspace_bytes),
                static_cast<long long>(need));
   const int64_t slab = align_up(n_c * 4, 256);

@@ -1381,9 +1381,9 @@ const char* hi3d_version(void) { return "hi3d_amd 0.1 gfx950"; }
 // Bytes of the cell-order sort that precedes a hash build: keys and rows (two slabs
 // each) and the radix sort's counts.
 static int64_t hash_order_bytes(int64_t n) {
-  // keys, rows (two of each), the radix sort's temporaries, the coordinates in order
-  return 4 * align_up(std::max<int64_t>(n, 1) * 4, 256) + align_up(radix::temp_bytes(std::max<int64_t>(n, 1)), 256) +
-         align_up(std::max<int64_t>(n, 1) * 16, 256);
+  // keys, rows (two of each), the coordinates in order, the radix sort's temporaries
+  const int64_t m = std::max<int64_t>(n, 1);
+  return 4 * align_up(m * 4, 256) + align_up(m * 16, 256) + radix::temp_bytes(m);
 }
 
 // Bytes of a brick table of `cap` buckets: key | mask words, then 8 rows per bucket.
@@ -1445,10 +1445,10 @@ static int kmap_subm_hash(const int32_t* coords, int64_t n, Grid g, int32_t ksiz
   return HI3D_OK;
 }
 
-// Brick-hash build + probe (hi3d_kmap_subm's map) over `cap` buckets at `ws`, with the
-// cell-order sort when the table is large.
+// Brick-hash build + probe (hi3d_kmap_subm's map) over `cap` buckets at `ws` (of ws_bytes),
+// with the cell-order sort when the table is large.
 static int kmap_subm_brick(const int32_t* coords, int64_t n, Grid g, int32_t ksize, int64_t cap, char* ws,
-                           int32_t* nbr, int32_t* counts, int32_t* status, hipStream_t stream) {
+                           int64_t ws_bytes, int32_t* nbr, int32_t* counts, int32_t* status, hipStream_t stream) {
   BrickTable t;
   t.words = reinterpret_cast<unsigned long long*>(ws);
   t.rows = reinterpret_cast<int32_t*>(ws + align_up(cap * 8, 256));
@@ -1479,13 +1479,14 @@ static int kmap_subm_brick(const int32_t* coords, int64_t n, Grid g, int32_t ksi
     const int kb = full ? key_bits + 9 : key_bits - shift;
     hipLaunchKernelGGL(superblock_key_kernel, dim3(blocks), dim3(256), 0, stream, c4, n, g, shift, full, k0, r0,
                        status);
-    HI3D_HIP_CHECK(radix::sort_pairs(order + 4 * slab, radix::temp_bytes(n), k0, k1, r0, r1, n,
-                                     kb > 24 ? kb - 24 : 0, kb, stream));
+    char* const temp = order + 4 * slab + align_up(n * 16, 256);
+    HI3D_HIP_CHECK(radix::sort_pairs(temp, ws + ws_bytes - temp, k0, k1, r0, r1, n, kb > 24 ? kb - 24 : 0, kb,
+                                     stream));
     perm = r0;
     if (full)
       skeys = k0;
     else
-      sorted = reinterpret_cast<int4*>(order + 4 * slab + align_up(radix::temp_bytes(n), 256));
+      sorted = reinterpret_cast<int4*>(order + 4 * slab);
     per = static_cast<int>(ceil_div(probe_blocks, kXcds));
     probe_blocks = static_cast<int64_t>(per) * kXcds;
   }
@@ -1519,10 +1520,11 @@ int hi3d_kmap_subm(const int32_t* coords, int64_t n, int32_t sx, int32_t sy, int
   int64_t need = 0;
   rc = hi3d_kmap_workspace(n, cap, 1, &need);
   if (rc != HI3D_OK) return rc;
+  need -= radix::spare_bytes(n);
   HI3D_REQUIRE(workspace_bytes >= need, "workspace too small: %lld < %lld bytes",
                static_cast<long long>(workspace_bytes), static_cast<long long>(need));
-  return kmap_subm_brick(coords, n, Grid{sx, sy, sz, batch_size}, ksize, cap, static_cast<char*>(workspace), nbr,
-                         counts, status, stream);
+  return kmap_subm_brick(coords, n, Grid{sx, sy, sz, batch_size}, ksize, cap, static_cast<char*>(workspace),
+                         workspace_bytes, nbr, counts, status, stream);
 }
 
 // The same map with the hash table in `scratch`, a device array of this library (no
@@ -1624,6 +1626,7 @@ int kmap_subm_dense(const int32_t* coords, int64_t n, int32_t sx, int32_t sy, in
     int64_t order_need = 0;
     rc = hi3d_kmap_dense_order_workspace(n, &order_need);
     if (rc != HI3D_OK) return rc;
+    order_need -= radix::spare_bytes(n);
     HI3D_REQUIRE(order_bytes >= order_need, "order workspace too small: %lld < %lld bytes",
                  static_cast<long long>(order_bytes), static_cast<long long>(order_need));
     const int64_t slab = align_up(n * 4, 256);
@@ -1740,7 +1743,7 @@ static int resample_structure(const int32_t* coords, int64_t n, int32_t sx, int3
     return HI3D_OK;
   }
   HI3D_REQUIRE(coords && low && inverse && counts && slot && workspace, "null pointer argument");
-  HI3D_REQUIRE(workspace_bytes >= need, "workspace too small");
+  HI3D_REQUIRE(workspace_bytes >= need - radix::spare_bytes(n), "workspace too small");
   HI3D_REQUIRE(sx > 0 && sy > 0 && sz > 0 && batch_size > 0, "spatial_shape and batch_size must be positive");
   const Factor f{fx, fy, fz, (sx + fx - 1) / fx, (sy + fy - 1) / fy, (sz + fz - 1) / fz};
   const uint64_t slots = static_cast<uint64_t>(fx) * fy * fz;
@@ -1750,8 +1753,8 @@ static int resample_structure(const int32_t* coords, int64_t n, int32_t sx, int3
   auto* r0 = ws.take<int32_t>(n);
   auto* r1 = ws.take<int32_t>(n);
   auto* ids = ws.take<int32_t>(n);
-  const int64_t temp_bytes = radix::temp_bytes(n);
-  void* temp = ws.take<char>(temp_bytes);
+  int64_t temp_bytes = 0;
+  void* temp = ws.rest(&temp_bytes);
   const unsigned blocks = static_cast<unsigned>(ceil_div(n, 256));
   const int4* c4 = reinterpret_cast<const int4*>(coords);
   const double space_d = static_cast<double>(batch_size) * f.hx * f.hy * f.hz * static_cast<double>(slots);
@@ -1872,10 +1875,9 @@ int hi3d_child_coords(const int32_t* coords, const int32_t* parent, const int32_
 int hi3d_child_table_workspace(int64_t n_parents, int64_t* bytes) {
   HI3D_REQUIRE(bytes != nullptr, "bytes_host is NULL");
   HI3D_REQUIRE(n_parents >= 0 && n_parents * 8 < (int64_t(1) << 31) - 16, "bad n_parents");
-  // more than the parents' counts, scan and (first child, slots) pairs take: the size stays
-  // the 12 bytes per slot that callers have been given
+  // 12 bytes per slot, more than the parents' counts, scan and (first child, slots) pairs take
   const int64_t m = std::max<int64_t>(n_parents * 8, 1);
-  *bytes = 2 * align_up(m * 4, 256) + align_up((m + 8) * 4, 256) + radix::temp_bytes(m);
+  *bytes = 2 * align_up(m * 4, 256) + align_up((m + 8) * 4, 256) + radix::least_bytes(m);
   return HI3D_OK;
 }
 
@@ -1898,7 +1900,7 @@ int hi3d_child_neighbour_table(const int32_t* parent_table, const uint8_t* mask,
   int32_t* counts = ws.take<int32_t>(n_parents);
   int32_t* excl = ws.take<int32_t>(n_parents);
   uint2* info = ws.take<uint2>(n_parents + 1);
-  const int64_t scan_bytes = radix::temp_bytes(n_parents);
+  const int64_t scan_bytes = radix::least_bytes(n_parents);
   void* temp = ws.take<char>(scan_bytes);
   auto blocks = [](int64_t n) { return dim3(static_cast<unsigned>(ceil_div(n, 256))); };
   hipLaunchKernelGGL(child_count_kernel, blocks(n_parents), dim3(256), 0, stream, mask, n_parents, counts);

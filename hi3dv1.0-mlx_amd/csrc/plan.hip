@@ -383,8 +383,6 @@ __global__ __launch_bounds__(kHaloRows) void halo_tile_kernel(const int32_t* __r
   }
 }
 
-int64_t sort_temp_bytes(int64_t n) { return radix::temp_bytes(std::max<int64_t>(n, 1)); }
-
 // Sorts (keys, rows) on key bits [0, bits) with 32-bit keys when they fit, else 64-bit
 // ones; kbuf0 / kbuf1 hold n 64-bit keys each, rows start in r0. fill(k) launches the
 // kernel that writes the keys into k (uint32_t* or unsigned long long*) and the rows
@@ -422,7 +420,7 @@ int hi3d_conv_plan_workspace(int64_t n_out, int64_t* bytes) {
   HI3D_REQUIRE(bytes != nullptr, "bytes_host is NULL");
   HI3D_REQUIRE(n_out >= 0 && n_out < (int64_t(1) << 31) - 1, "bad n_out");
   const int64_t m = std::max<int64_t>(n_out, 1);
-  *bytes = 2 * align_up(m * 8, 256) + 3 * align_up(m * 4, 256) + sort_temp_bytes(m) + 256;
+  *bytes = 2 * align_up(m * 8, 256) + 3 * align_up(m * 4, 256) + radix::temp_bytes(m) + 256;
   return HI3D_OK;
 }
 
@@ -439,15 +437,15 @@ int hi3d_conv_plan(const int32_t* table, int64_t n_out, int32_t kvol, int64_t n_
                "coord_bits must be in [0, 19] and batch_bits in [0, 7]");
   if (n_out == 0) return HI3D_OK;
   HI3D_REQUIRE(table && rows && gidx && tile_mask && workspace, "null pointer argument");
-  HI3D_REQUIRE(workspace_bytes >= need, "workspace too small");
+  HI3D_REQUIRE(workspace_bytes >= need - radix::spare_bytes(n_out), "workspace too small");
   Workspace ws(workspace, workspace_bytes);
   auto* k0 = ws.take<unsigned long long>(n_out);
   auto* k1 = ws.take<unsigned long long>(n_out);
   auto* r0 = ws.take<int32_t>(n_out);
   auto* r1 = ws.take<int32_t>(n_out);
   auto* masks = ws.take<uint32_t>(n_out);
-  const int64_t temp_bytes = sort_temp_bytes(n_out);
-  void* temp = ws.take<char>(temp_bytes);
+  int64_t temp_bytes = 0;
+  void* temp = ws.rest(&temp_bytes);
   const unsigned blocks = static_cast<unsigned>(ceil_div(n_out, 256));
   const int n = static_cast<int>(n_out);
   const int32_t* order = nullptr;
@@ -531,14 +529,14 @@ int hi3d_halo_plan(const int32_t* table, int64_t n_out, int32_t kvol, int64_t n_
   launch_fill(overflow, 1, int32_t(0), stream);
   if (n_out == 0) return HI3D_OK;
   HI3D_REQUIRE(table && rows && halo && hcount && loff && bmask && workspace, "null pointer argument");
-  HI3D_REQUIRE(workspace_bytes >= need, "workspace too small");
+  HI3D_REQUIRE(workspace_bytes >= need - radix::spare_bytes(n_out), "workspace too small");
   Workspace ws(workspace, workspace_bytes);
   auto* k0 = ws.take<unsigned long long>(n_out);
   auto* k1 = ws.take<unsigned long long>(n_out);
   auto* r0 = ws.take<int32_t>(n_out);
   auto* r1 = ws.take<int32_t>(n_out);
-  const int64_t temp_bytes = sort_temp_bytes(n_out);
-  void* temp = ws.take<char>(temp_bytes);
+  int64_t temp_bytes = 0;
+  void* temp = ws.rest(&temp_bytes);
   const unsigned blocks = static_cast<unsigned>(ceil_div(n_out, 256));
   const int32_t* order = r0;
   if (coords) {

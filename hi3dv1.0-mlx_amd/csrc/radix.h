@@ -35,7 +35,7 @@ static_assert(kBins == kThreads, "one thread per digit in the per-digit steps");
 
 inline int64_t tiles(int64_t n) { return std::max<int64_t>(ceil_div(n, kTile), 1); }
 
-// Keys per thread of a sorting pass: up to 2^20 keys four, so that the tiles fill the CUs
+// Keys per thread of a sorting pass: up to 2^20 keys four (if the workspace has room), so that the tiles fill the CUs
 // (400,003 pairs: downsweep 12.9 -> 6.8 us on 391 tiles instead of 98, upsweep 4.6 -> 4.2;
 // a million pairs about equal), above that sixteen, with longer runs to write.
 constexpr int kFewItems = 4;
@@ -43,12 +43,16 @@ constexpr int64_t kFewKeys = int64_t(1) << 20;
 inline int sort_items(int64_t n) { return n <= kFewKeys ? kFewItems : kItems; }
 inline int64_t sort_tiles(int64_t n) { return std::max<int64_t>(ceil_div(n, kThreads * sort_items(n)), 1); }
 
-// Workspace bytes of sort_pairs and scan for up to n elements (a smaller set may have more
-// tiles): per-tile counts and totals.
+// Workspace bytes: per-tile counts and totals. least_bytes: enough for scan, and for
+// sort_pairs on tiles of kTile keys; every entry point takes a workspace with that much.
+// temp_bytes: what the size queries report, with room for the small tiles of any set of up
+// to n keys (a smaller set may have more of them). spare_bytes: the difference.
+inline int64_t tile_bytes(int64_t ntiles) { return align_up(ntiles * kBins * 4, 256) + align_up(kBins * 4, 256); }
+inline int64_t least_bytes(int64_t n) { return tile_bytes(tiles(n)); }
 inline int64_t temp_bytes(int64_t n) {
-  const int64_t most = std::max(sort_tiles(n), sort_tiles(std::min(n, kFewKeys)));
-  return align_up(most * kBins * 4, 256) + align_up(kBins * 4, 256);
+  return tile_bytes(std::max(sort_tiles(n), sort_tiles(std::min(n, kFewKeys))));
 }
+inline int64_t spare_bytes(int64_t n) { return temp_bytes(n) - least_bytes(n); }
 
 // Exclusive prefix of v over the block's 256 threads; *total gets the sum. part holds
 // kWaves ints of LDS; the function ends with a barrier, so part can be reused.
@@ -305,15 +309,15 @@ __device__ void block_sort_pairs(uint32_t (&keys)[ITEMS], uint32_t (&vals)[ITEMS
 
 // Sorts n (key, value) pairs stably by key bits [begin_bit, end_bit). keys / vals hold
 // the input; on return they point at the sorted pairs, which may be the former
-// keys_alt / vals_alt (swapped with them). temp: temp_bytes(n) bytes.
+// keys_alt / vals_alt (swapped with them). temp: least_bytes(n) bytes or more.
 template <typename K>
 hipError_t sort_pairs(void* temp, int64_t temp_size, K*& keys, K*& keys_alt, int32_t*& vals, int32_t*& vals_alt,
                       int64_t n, int begin_bit, int end_bit, hipStream_t stream) {
   if (n <= 0 || end_bit <= begin_bit) return hipSuccess;
-  if (temp_size < temp_bytes(n) || end_bit > static_cast<int>(8 * sizeof(K)) || begin_bit < 0)
+  if (temp_size < least_bytes(n) || end_bit > static_cast<int>(8 * sizeof(K)) || begin_bit < 0)
     return hipErrorInvalidValue;
-  const int64_t nt = sort_tiles(n);
-  const bool few = sort_items(n) == kFewItems;
+  const bool few = sort_items(n) == kFewItems && temp_size >= tile_bytes(sort_tiles(n));
+  const int64_t nt = few ? sort_tiles(n) : tiles(n);
   auto* counts = static_cast<int32_t*>(temp);
   auto* totals = reinterpret_cast<int32_t*>(static_cast<char*>(temp) + align_up(nt * kBins * 4, 256));
   const dim3 grid(static_cast<unsigned>(nt));
@@ -373,11 +377,11 @@ __global__ __launch_bounds__(kThreads) void tile_scan_kernel(const int32_t* __re
 }
 
 // out[i] = sum of in[0 .. i) (exclusive) or in[0 .. i] (inclusive); out may be in.
-// temp: temp_bytes(n) bytes.
+// temp: least_bytes(n) bytes.
 inline hipError_t scan(void* temp, int64_t temp_size, const int32_t* in, int32_t* out, int64_t n, bool inclusive,
                        hipStream_t stream) {
   if (n <= 0) return hipSuccess;
-  if (temp_size < temp_bytes(n)) return hipErrorInvalidValue;
+  if (temp_size < least_bytes(n)) return hipErrorInvalidValue;
   const int64_t nt = tiles(n);
   auto* sums = static_cast<int32_t*>(temp);
   auto* total = reinterpret_cast<int32_t*>(static_cast<char*>(temp) + align_up(nt * kBins * 4, 256));

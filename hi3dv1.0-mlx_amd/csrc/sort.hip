@@ -26,8 +26,8 @@ int hi3d_sort_pairs(void* keys, void* keys_alt, int32_t* vals, int32_t* vals_alt
   *in_alt = 0;
   if (n == 0 || begin_bit == end_bit) return HI3D_OK;
   HI3D_REQUIRE(keys && keys_alt && vals && vals_alt && workspace, "null pointer argument");
-  HI3D_REQUIRE(workspace_bytes >= radix::temp_bytes(n), "workspace too small: %lld < %lld bytes",
-               static_cast<long long>(workspace_bytes), static_cast<long long>(radix::temp_bytes(n)));
+  HI3D_REQUIRE(workspace_bytes >= radix::least_bytes(n), "workspace too small: %lld < %lld bytes",
+               static_cast<long long>(workspace_bytes), static_cast<long long>(radix::least_bytes(n)));
   int32_t* v = vals;
   int32_t* va = vals_alt;
   if (key_bytes == 4) {
@@ -49,8 +49,8 @@ int hi3d_scan(const int32_t* in, int32_t* out, int64_t n, int32_t inclusive, voi
   HI3D_REQUIRE(n >= 0 && n < (int64_t(1) << 31) - 1, "bad element count");
   if (n == 0) return HI3D_OK;
   HI3D_REQUIRE(in && out && workspace, "null pointer argument");
-  HI3D_REQUIRE(workspace_bytes >= radix::temp_bytes(n), "workspace too small: %lld < %lld bytes",
-               static_cast<long long>(workspace_bytes), static_cast<long long>(radix::temp_bytes(n)));
+  HI3D_REQUIRE(workspace_bytes >= radix::least_bytes(n), "workspace too small: %lld < %lld bytes",
+               static_cast<long long>(workspace_bytes), static_cast<long long>(radix::least_bytes(n)));
   HI3D_HIP_CHECK(radix::scan(workspace, workspace_bytes, in, out, n, inclusive != 0, stream));
   return HI3D_OK;
 }

@@ -158,7 +158,7 @@ extern "C" int hi3d_unique_keys(const int64_t* keys, int64_t n, int32_t key_bits
     return HI3D_OK;
   }
   HI3D_REQUIRE(keys && workspace && uniq && inverse, "null pointer argument");
-  HI3D_REQUIRE(workspace_bytes >= need, "workspace too small");
+  HI3D_REQUIRE(workspace_bytes >= need - radix::spare_bytes(n), "workspace too small");
   Workspace ws(workspace, workspace_bytes);
   auto* k0 = ws.take<unsigned long long>(n);
   auto* k1 = ws.take<unsigned long long>(n);
@@ -167,8 +167,8 @@ extern "C" int hi3d_unique_keys(const int64_t* keys, int64_t n, int32_t key_bits
   auto* head = ws.take<int32_t>(n);
   auto* run = ws.take<int32_t>(n);
   auto* first = ws.take<int32_t>(n);
-  const int64_t temp_bytes = radix::temp_bytes(n);
-  void* temp = ws.take<char>(temp_bytes);
+  int64_t temp_bytes = 0;
+  void* temp = ws.rest(&temp_bytes);
   const unsigned blocks = static_cast<unsigned>(ceil_div(n, 256));
   // keys within [0, 2^key_bits) sort on those bits as they are; any int64 sorts on all
   // 64 bits with the sign bit flipped

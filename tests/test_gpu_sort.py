@@ -81,3 +81,73 @@ def test_scan_matches_cumsum(cuda, n, inclusive):
     c = np.cumsum(x, dtype=np.int64).astype(np.int32)
     ref = c if inclusive else np.concatenate([[0], c[:-1]]).astype(np.int32)
     assert np.array_equal(got, ref)
+
+
+def _al(x: int) -> int:
+    return (x + 255) // 256 * 256
+
+
+def _least(n: int) -> int:
+    """Sort and scan scratch with tiles of 4096 elements."""
+    return 1024 * max((n + 4095) // 4096, 1) + 1024
+
+
+LEAST = {
+    "hi3d_sort_pairs_workspace": _least,
+    "hi3d_unique_keys_workspace": lambda n: 2 * _al(8 * n) + 5 * _al(4 * n) + _least(n) + 256,
+    "hi3d_conv_plan_workspace": lambda n: 2 * _al(8 * n) + 3 * _al(4 * n) + _least(n) + 256,
+    "hi3d_halo_plan_workspace": lambda n: 2 * _al(8 * n) + 3 * _al(4 * n) + _least(n) + 256,
+    "hi3d_downsample_workspace": lambda n: 2 * _al(8 * n) + 3 * _al(4 * n) + _least(n) + 256,
+    "hi3d_stride2_up_plan_workspace": lambda n: 4 * _al(4 * n) + _least(n),
+    "hi3d_child_table_workspace": lambda n: 2 * _al(32 * n) + _al(32 * n + 32) + _least(8 * n),
+    "hi3d_kmap_dense_order_workspace": lambda n: 4 * _al(4 * n) + _least(n),
+    "hi3d_kmap_workspace": lambda n, cap, key64: _al(8 * cap) + _al(32 * cap) + 4 * _al(4 * n) + _least(n) + _al(16 * n),
+}
+
+
+@pytest.mark.parametrize("n", [1, 5000, 150_001, 1_100_000])
+def test_least_workspaces_are_enough(cuda, monkeypatch, n):
+    """Every call that sorts or scans, with the least workspace it takes (tiles of 4096
+    keys, whatever faster tiles the size query leaves room for): the results of the
+    reported size, and nothing written behind the workspace."""
+    from hi3d_amd import _lib, fast_unique, kmap, sort
+
+    rng = np.random.default_rng(n)
+    side = 128
+    cells = torch.as_tensor(rng.permutation(side ** 3)[:n])
+    idx = torch.stack([0 * cells, cells // side ** 2, cells // side % side, cells % side], 1).int().to(cuda)
+    keys = torch.as_tensor(rng.integers(0, 2**31, n).astype(np.int32)).to(cuda)
+    vals = torch.arange(n, dtype=torch.int32, device=cuda)
+    mask = torch.as_tensor(rng.random((n, 8)) < 0.4).to(cuda)
+
+    def run():
+        monkeypatch.setattr(kmap, "KMAP_DENSE_ORDER_MIN_BYTES", 0)
+        m = kmap.build_kernel_map(idx, [side] * 3, 1)
+        far = idx * torch.tensor([1, 16, 16, 16], dtype=torch.int32, device=cuda)
+        hashed = [kmap.build_kernel_map(c, [s] * 3, 1, capacity=1 << 21).table for c, s in ((idx, 512), (far, 2048))]
+        plan = kmap.build_plan(m.table, n, idx)
+        s2 = kmap.stride2_structure(idx, [side] * 3, 1)
+        return [*sort.sort_pairs(keys, vals), sort.scan(vals % 7), m.table, *hashed, plan.rows, plan.gidx, plan.tile_mask,
+                s2.low, s2.inverse, s2.counts, *s2.up_order(), *kmap.child_neighbour_table(m.table, mask),
+                *fast_unique.unique_rows(idx[:, 1:] // 3, True, True)]
+
+    want = run()
+    guards, query = [], _lib.query
+
+    def least(name, *args):
+        if name not in LEAST:
+            return query(name, *args)
+        b = LEAST[name](*args)
+        assert b <= query(name, *args)
+        return b
+
+    def workspace(nbytes, device):
+        t = torch.full((int(nbytes) + 4096,), 0xA5, dtype=torch.uint8, device=device)
+        guards.append(t[int(nbytes):])
+        return t[:int(nbytes)]
+
+    monkeypatch.setattr(_lib, "query", least)
+    monkeypatch.setattr(_lib, "workspace", workspace)
+    for g, w in zip(run(), want, strict=True):
+        assert torch.equal(g, w)
+    assert len(guards) >= 10 and all((g == 0xA5).all() for g in guards)
