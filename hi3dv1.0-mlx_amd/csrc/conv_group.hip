@@ -4,21 +4,24 @@
 //
 //   out[o] = act(bias + sum_k in[gidx[o, k]] . W[:, k, :]^T) (+ residual[o])
 //
-// fp32: x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2), each
-// rounded to nearest: 24 bits, so the three hold every fp32 bit. Of the nine products
-// the kernel keeps w1 x1, w1 x2, w2 x1, w2 x2, w1 x3 and w3 x1; the others are below
-// 2^-25 of the product, under half an fp32 ulp. Products of two bf16 values are exact in
-// fp32 and the MFMA adds them to fp32 accumulators, as the fp32 MFMA does: the result
-// keeps fp32 accuracy at six 32x32x16 bf16 MFMAs in the place of eight 32x32x2 fp32 ones,
-// 192 cycles against 512. Relative error against 64-bit sums: C128, 327,581 voxels
-// 5.8e-7 (fp32 MFMA 6.7e-7), C64 4.2e-7 (5.0e-7), C256 8.5e-7 (9.8e-7): fewer roundings,
-// since one MFMA sums 16 products. What bounds it: the bf16 matrix rate. At C128 and
-// 327,581 voxels the six products of the 64-row tiles' offsets run at 1.06 PFLOP/s (a
-// large bf16 product of the library: 1.19).
+// fp32: 2^16 x = x1 + x2 + x3 with x1 = bf16(2^16 x), x2 = bf16(2^16 x - x1) and x3 the rest,
+// each rounded to nearest. They hold every bit of an fp32 value: 24, and with the scale bf16's
+// smallest step, 2^-133, is the last bit of a subnormal x (without it values below 2^-110 lost
+// bits: at 2^-120 the result had an error of 3.5e-5). Of the nine products the kernel keeps
+// w1 x1, w1 x2, w2 x1, w1 x3, w3 x1 and w2 x2; the other three are together at most about
+// 2^-24 of the product. Products of two bf16 values are exact in fp32 and the MFMA adds them
+// to fp32 accumulators, as the fp32 MFMA does: fp32 accuracy at six 32x32x16 bf16 MFMAs in the
+// place of eight 32x32x2 fp32 ones, 192 cycles against 512. Relative error against 64-bit
+// sums, normal random values: C128, 327,581 voxels 2.3e-7 (fp32 MFMA 6.8e-7), C64, 45,128
+// voxels 1.6e-7 (5.1e-7), C256, 100,000 voxels 3.4e-7 (9.9e-7): one MFMA sums 16 products, and
+// the products of each size (w1 x1, 2^-8 and 2^-16 of it) have a sum of their own (in one sum
+// for all, without the scale, the three errors were 5.9e-7, 4.3e-7, 8.6e-7 and the times about
+// 3 % less). What bounds it: the bf16 matrix rate, at C64 as much the vector operations of the
+// split.
 //
-// Infinities, NaN and values whose bf16 rounding overflows leave a sum that is not
-// finite (a part x2 or x3 of an infinity is NaN); such outputs are summed again in plain
-// fp32 in the epilogue, over the offsets their row has.
+// Infinities, NaN, values from 2^112 and sums from 2^96 on, whose scaled forms overflow,
+// leave a sum that is not finite (a part x2 or x3 of an infinity is NaN); such outputs are
+// summed again in plain fp32 in the epilogue, over the offsets their row has.
 //
 // Reference semantics: subm_conv (src/hi3d_mac/torch_backend/sparse_conv.py:152-195).
 #include <type_traits>
@@ -43,6 +46,8 @@ constexpr int kGroupThreads = 256;
 constexpr int kFewOffsets = 8;
 constexpr int64_t kFewOffsetsWork = 128 * 256;
 
+constexpr float kPartScale = 65536.0f;
+
 // row that absent neighbours read
 __device__ __attribute__((aligned(16))) const uint32_t g_group_zero_row[kGroupMaxRowBytes / 4] = {};
 
@@ -51,7 +56,7 @@ __device__ __forceinline__ void split8(const f32x4 lo, const f32x4 hi, bf16x8 (&
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    float a = j < 2 ? lo[2 * j] : hi[2 * j - 4], b = j < 2 ? lo[2 * j + 1] : hi[2 * j - 3];
+    float a = kPartScale * (j < 2 ? lo[2 * j] : hi[2 * j - 4]), b = kPartScale * (j < 2 ? lo[2 * j + 1] : hi[2 * j - 3]);
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       const bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
@@ -113,7 +118,7 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* __restri
 //    ring of NS slots, one barrier a stage. The next loads go out first, then a stage's
 //    fragments are all read before its first product (fp32 C256 on 100,000 voxels 1.24 ms,
 //    with the loads after the fragments 1.29; C128 on 3,000 voxels 49 against 53 us).
-//  * fp32 rows stay fp32 in LDS and each wave splits its fragments in registers (11 vector
+//  * fp32 rows stay fp32 in LDS and each wave splits its fragments in registers (13 vector
 //    ops per pair of values).
 //  * The gather indices of all offsets reach LDS once, and with them the offsets that each
 //    32-row block has; a wave skips its block's products of the others.
@@ -252,11 +257,14 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
     if (++lks == ksteps) lks = 0;
   };
 
-  f32x16 acc[NB];
+  constexpr int NA = kSplit ? 3 : 1;  // fp32: sums of the products by their size
+  f32x16 acc[NA][NB];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+  for (int l = 0; l < NA; ++l)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[nb][v] = 0.0f;
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[l][nb][v] = 0.0f;
 
   // a stage's fragments: rows x, weights w (fp32: KS steps of 16 inputs, a step's row
   // fragment as two 16-byte chunks and its weights as three parts; 16-bit: 2 KS groups)
@@ -287,20 +295,21 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
       for (int s = 0; s < KS; ++s) {
         bf16x8 xp[3];
         split8(__builtin_bit_cast(f32x4, x[2 * s]), __builtin_bit_cast(f32x4, x[2 * s + 1]), xp);
-        // small products first
-        constexpr int WP[6] = {2, 0, 1, 1, 0, 0}, XP[6] = {0, 2, 1, 0, 1, 0};
+        constexpr int WP[6] = {0, 0, 1, 0, 1, 2}, XP[6] = {0, 1, 0, 2, 1, 0};
 #pragma unroll
         for (int t = 0; t < 6; ++t)
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            acc[nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[nb][3 * s + WP[t]]), xp[XP[t]],
-                                                              acc[nb], 0, 0, 0);
+          for (int nb = 0; nb < NB; ++nb) {
+            f32x16& sum = acc[WP[t] + XP[t]][nb];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[nb][3 * s + WP[t]]), xp[XP[t]], sum,
+                                                          0, 0, 0);
+          }
       }
     } else {
 #pragma unroll
       for (int f = 0; f < XF; ++f)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) Mfma<T>::run(w[nb][f], x[f], acc[nb]);
+        for (int nb = 0; nb < NB; ++nb) Mfma<T>::run(w[nb][f], x[f], acc[0][nb]);
     }
   };
 
@@ -361,7 +370,11 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
         const int chunk = (wn * WN + nb * 32 + 8 * q + 4 * (lane >> 5)) >> 2;
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[nb][4 * q + e];
+        for (int e = 0; e < 4; ++e) {
+          v[e] = acc[0][nb][4 * q + e];
+          if constexpr (kSplit)
+            v[e] = (v[e] + (acc[1][nb][4 * q + e] + acc[2][nb][4 * q + e])) * (1.0f / (kPartScale * kPartScale));
+        }
         *reinterpret_cast<f32x4*>(stg + ((chunk ^ (lane & 15)) << 4)) = v;
       }
     }

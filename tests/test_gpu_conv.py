@@ -351,6 +351,35 @@ def test_16bit_group_kernel(cuda, dtype, cin, cout, density, side, act, res):
     assert torch.equal(y, y2)
 
 
+@pytest.mark.parametrize("cin,cout,side,density", [(64, 64, 20, 0.3), (128, 128, 40, 0.25), (64, 36, 44, 0.25)])
+@pytest.mark.parametrize("ex,ew", [(-100, 0), (-118, 0), (-126, 0), (0, -118), (0, -126), (-135, 40), (40, -135), (-62, -60),
+                                   (-126, 100), (112, -126), (121, -60), (-60, 121), (60, 50)])
+def test_fp32_split_kernel_scales(cuda, cin, cout, side, density, ex, ew):
+    """Features near 2^ex and weights near 2^ew, down to values whose unscaled low parts
+    bf16 cannot hold and to subnormal ones, up to parts and sums that overflow: no larger
+    error than the fp32 matrix cores' on the same inputs (both measured against float64),
+    in the group, the 128-channel and the 64-channel tiles."""
+    from hi3d_amd import _lib, conv, kmap
+
+    rng = np.random.default_rng(side)
+    idx = _rand_indices(rng, side, density)
+    n = len(idx)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    plan = km.plan()
+    x, w, _ = _case(rng, n, cin, cout, torch.float32)
+    xd, wd = (x.double() * 2.0 ** ex).float().to(cuda), (w.double() * 2.0 ** ew).float().to(cuda)
+    y = conv.gather_conv(xd, plan, wd)
+    z = torch.empty_like(y)
+    _lib.call("hi3d_gather_conv", _lib.ptr(xd), n, cin, _lib.ptr(wd), None, cout, 27, _lib.ptr(plan.rows),
+              _lib.ptr(plan.gidx), _lib.ptr(plan.tile_mask), n, None, 0, _lib.DTYPES[torch.float32], _lib.ptr(z),
+              _lib.stream(xd.device))
+    up = 2.0 ** -(ex + ew)  # the sums at an ordinary size, exactly
+    ref = oconv.gather_conv_f64(xd.cpu().double().numpy() * 2.0 ** -ex, km.table.cpu().numpy(),
+                                wd.cpu().double().numpy() * 2.0 ** -ew, np.zeros(cout))
+    ey, ez = (_rel_rms(v.cpu().double().numpy() * up, ref) for v in (y, z))
+    assert ey <= ez, (ey, ez)
+
+
 def test_fp32_split_kernel_not_finite(cuda):
     """Infinities, NaN and values past bf16's largest, in the features and in the weights:
     where the sum over a row's present neighbours is infinite or NaN so is the output,
