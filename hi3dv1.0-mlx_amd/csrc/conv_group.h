@@ -10,7 +10,6 @@ struct GroupConv {
   int64_t n_in;
   int32_t cin;
   const char* weight;   // 16-bit: [cout][kvol][cin]
-  int64_t wn, wk, wc;   // fp32: weight strides (output channel, offset, input channel)
   const char* packed;   // fp32: [kvol][cin / 16][col_blocks][3 parts][64 lanes][16 bytes]
   int32_t col_blocks;   // 32-channel blocks of the packed weights (the last may be padding)
   const char* bias;

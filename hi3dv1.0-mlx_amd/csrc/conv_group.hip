@@ -20,8 +20,11 @@
 // split.
 //
 // Infinities, NaN, values from 2^112 and sums from 2^96 on, whose scaled forms overflow,
-// leave a sum that is not finite (a part x2 or x3 of an infinity is NaN); such outputs are
-// summed again in plain fp32 in the epilogue, over the offsets their row has.
+// leave a sum that is not finite (a part x2 or x3 of an infinity is NaN). A workgroup with
+// such outputs walks its stages once more with the fp32 MFMA, which takes the weights from
+// their parts, and replaces those outputs; a row sums the offsets that it has (C128 on
+// 100,000 voxels, every row NaN: 1.15 ms, fp32 MFMA 0.67, the plain sum of one output after
+// another 40 ms).
 //
 // Reference semantics: subm_conv (src/hi3d_mac/torch_backend/sparse_conv.py:152-195).
 #include <type_traits>
@@ -47,6 +50,7 @@ constexpr int kFewOffsets = 8;
 constexpr int64_t kFewOffsetsWork = 128 * 256;
 
 constexpr float kPartScale = 65536.0f;
+constexpr float kPartMax = 0x1p111f;  // no scaled value below it rounds to infinity
 
 // row that absent neighbours read
 __device__ __attribute__((aligned(16))) const uint32_t g_group_zero_row[kGroupMaxRowBytes / 4] = {};
@@ -70,6 +74,16 @@ __device__ __forceinline__ void split8(const f32x4 lo, const f32x4 hi, bf16x8 (&
       }
     }
   }
+}
+
+// Value e of 8 from their parts as split_weight_kernel stores them.
+__device__ __forceinline__ float joined(const u32x4 (&p)[3], int e) {
+  uint32_t u[3];  // the parts as fp32 bits
+#pragma unroll
+  for (int i = 0; i < 3; ++i) u[i] = e % 2 ? p[i][e / 2] & 0xffff0000u : p[i][e / 2] << 16;
+  const float first = __builtin_bit_cast(float, u[0]);
+  const float sum = first + (__builtin_bit_cast(float, u[1]) + __builtin_bit_cast(float, u[2]));  // exact
+  return first == first ? sum * (1.0f / kPartScale) : __builtin_bit_cast(float, u[1] | u[2] >> 16);
 }
 
 // One thread per 16-byte piece of a part: channel 32 nb + lane % 32, inputs
@@ -104,6 +118,16 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* __restri
   }
   bf16x8 p[3];
   split8(lo, hi, p);
+  // a weight whose scaled form overflows: NaN and the two halves of its bits
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float v = e < 4 ? lo[e] : hi[e - 4];
+    if (fabsf(v) < kPartMax) continue;
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    p[0][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(0x7fc0));
+    p[1][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(u >> 16));
+    p[2][e] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(u));
+  }
 #pragma unroll
   for (int i = 0; i < 3; ++i) *reinterpret_cast<bf16x8*>(packed + block * 3072 + i * 1024 + lane * 16) = p[i];
 }
@@ -116,8 +140,8 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* __restri
 //    and the weights (fp32: BN / 32 x KS x 3 KB of parts, laid out as the fragments are
 //    read; 16-bit: BN rows), by direct-to-LDS 16-byte loads NS - 1 stages ahead into a
 //    ring of NS slots, one barrier a stage. The next loads go out first, then a stage's
-//    fragments are all read before its first product (fp32 C256 on 100,000 voxels 1.24 ms,
-//    with the loads after the fragments 1.29; C128 on 3,000 voxels 49 against 53 us).
+//    fragments are all read before its first product (fp32 C256 on 100,000 voxels 1.23 ms,
+//    with the loads after the fragments 1.29; C128 on 3,000 voxels 51 against 53 us).
 //  * fp32 rows stay fp32 in LDS and each wave splits its fragments in registers (13 vector
 //    ops per pair of values).
 //  * The gather indices of all offsets reach LDS once, and with them the offsets that each
@@ -139,10 +163,11 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
   constexpr int RING = G * NS * STAGE;
   constexpr int SROW = BN * 4;  // staged sums: bytes of a row
   static_assert(G * BM * SROW <= RING, "staged sums");
-  __shared__ __attribute__((aligned(16))) char smem[RING + (KV + 1) * BM * 4 + NW * 8];
+  __shared__ __attribute__((aligned(16))) char smem[RING + (KV + 1) * BM * 4 + NW * 12];
   int32_t* const gl = reinterpret_cast<int32_t*>(smem + RING);
   int32_t* const srow = gl + KV * BM;
   uint32_t* const smask = reinterpret_cast<uint32_t*>(srow + BM);  // [wave][32-row block]
+  uint32_t* const sbad = smask + 2 * NW;  // [wave]: sums that are not finite
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -216,7 +241,7 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
     const int r = load_row(u), c = lane % LPR;
     return (KS == 1 ? (c ^ ((r >> 2) & 3)) : (c ^ ((r >> 1) & 7))) * 16;
   };
-  uint32_t rest = mine;
+  uint32_t rest = 0;
   int lks = 0, lslot = 0;
   const char* src[LA];
   const char* wsrc = nullptr;
@@ -259,12 +284,6 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
 
   constexpr int NA = kSplit ? 3 : 1;  // fp32: sums of the products by their size
   f32x16 acc[NA][NB];
-#pragma unroll
-  for (int l = 0; l < NA; ++l)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[l][nb][v] = 0.0f;
 
   // a stage's fragments: rows x, weights w (fp32: KS steps of 16 inputs, a step's row
   // fragment as two 16-byte chunks and its weights as three parts; 16-bit: 2 KS groups)
@@ -289,13 +308,29 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
       x[f] = *reinterpret_cast<const u32x4*>(st + row_off(wm * 32 + (lane & 31), c));
     }
   };
-  auto products = [&]() __attribute__((always_inline)) {
-    if constexpr (kSplit) {
+  auto products = [&](auto plain) __attribute__((always_inline)) {
+    if constexpr (plain) {
+      // input j of 16 and input 8 + j in one MFMA
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float xj = __builtin_bit_cast(f32x4, x[2 * s + j / 4])[j % 4];
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const u32x4 p[3] = {w[nb][3 * s], w[nb][3 * s + 1], w[nb][3 * s + 2]};
+            acc[1][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(p, j), xj, acc[1][nb], 0, 0, 0);
+          }
+        }
+    } else if constexpr (kSplit) {
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         bf16x8 xp[3];
         split8(__builtin_bit_cast(f32x4, x[2 * s]), __builtin_bit_cast(f32x4, x[2 * s + 1]), xp);
-        constexpr int WP[6] = {0, 0, 1, 0, 1, 2}, XP[6] = {0, 1, 0, 2, 1, 0};
+        // those of x1 first where one group works (C128 on 30,000 voxels 156 -> 152 us; with
+        // four groups a C64 tile's time went 29.4 -> 30.1 us)
+        constexpr int WP[6] = {0, G == 1 ? 1 : 0, G == 1 ? 2 : 1, 0, 1, G == 1 ? 0 : 2};
+        constexpr int XP[6] = {0, G == 1 ? 0 : 1, 0, G == 1 ? 1 : 2, 1, G == 1 ? 2 : 0};
 #pragma unroll
         for (int t = 0; t < 6; ++t)
 #pragma unroll
@@ -313,55 +348,76 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
     }
   };
 
-  // At the barrier of stage s every wave has its share of stage s in LDS and has read
-  // the fragments of stage s - 1, whose slot stage s + NS - 1 takes.
+  // The stages, and the sums to LDS: [group][64 rows][BN] fp32, 16-byte chunk c of row r at
+  // c ^ (r % 16). plain: in acc[0], each offset's products in acc[1] first, which only rows
+  // that have the offset take.
+  auto walk = [&](auto plain) __attribute__((always_inline)) {
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < S) issue();
-  uint32_t crest = mine;
-  int cks = 0, slot = 0;
-  for (int s = 0; s < SMAX; ++s) {
-    constexpr int AHEAD = NS - 2;  // stages that may stay in flight
-    if (s + AHEAD < S) {
-      if (wave < BKB % NWG) wait_vmcnt<AHEAD * (LA + LB)>();
-      else wait_vmcnt<AHEAD * (LA + LBMIN)>();
-    } else {
-      wait_vmcnt<0>();
+    for (int l = 0; l < NA; ++l)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[l][nb][v] = 0.0f;
+    rest = mine;
+    lks = lslot = 0;
+    // At the barrier of stage s every wave has its share of stage s in LDS and has read
+    // the fragments of stage s - 1, whose slot stage s + NS - 1 takes.
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s)
+      if (s < S) issue();
+    uint32_t crest = mine;
+    int cks = 0, slot = 0;
+    for (int s = 0; s < SMAX; ++s) {
+      constexpr int AHEAD = NS - 2;  // stages that may stay in flight
+      if (s + AHEAD < S) {
+        if (wave < BKB % NWG) wait_vmcnt<AHEAD * (LA + LB)>();
+        else wait_vmcnt<AHEAD * (LA + LBMIN)>();
+      } else {
+        wait_vmcnt<0>();
+      }
+      wait_lgkm0();
+      raw_barrier();
+      // this block has the offset (none left: false)
+      const bool have = s < S && (bmask & (crest & (0u - crest))) != 0;
+      if (s + NS - 1 < S) issue();
+      __builtin_amdgcn_sched_barrier(0);
+      if (have) {
+        frags(slot);
+        __builtin_amdgcn_sched_barrier(0);
+        products(plain);
+      }
+      slot = slot == NS - 1 ? 0 : slot + 1;
+      if (++cks == ksteps) {
+        if constexpr (plain) {
+          if (have) {
+            const bool row_has = gl[__builtin_ctz(crest) * BM + wm * 32 + (lane & 31)] >= 0;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+              for (int v = 0; v < 16; ++v) {
+                acc[0][nb][v] += row_has ? acc[1][nb][v] : 0.0f;
+                acc[1][nb][v] = 0.0f;
+              }
+          }
+        }
+        cks = 0;
+        crest &= crest - 1u;
+      }
+    }
+    if constexpr (kSplit && !plain) {
+      float bad = 0.0f;  // NaN if a sum is not finite
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          acc[0][nb][v] = (acc[0][nb][v] + (acc[1][nb][v] + acc[2][nb][v])) * (1.0f / (kPartScale * kPartScale));
+          bad = fmaf(acc[0][nb][v], 0.0f, bad);
+        }
+      const uint64_t b = __builtin_amdgcn_ballot_w64(!(bad == 0.0f));
+      if (lane == 0) sbad[wave_all] = b != 0 ? 1 : 0;
     }
     wait_lgkm0();
     raw_barrier();
-    // this block has the offset (none left: false)
-    const bool have = s < S && (bmask & (crest & (0u - crest))) != 0;
-    if (s + NS - 1 < S) issue();
-    __builtin_amdgcn_sched_barrier(0);
-    if (have) {
-      frags(slot);
-      __builtin_amdgcn_sched_barrier(0);
-      products();
-    }
-    slot = slot == NS - 1 ? 0 : slot + 1;
-    if (++cks == ksteps) {
-      cks = 0;
-      crest &= crest - 1u;
-    }
-  }
-
-  // plain fp32 sum of one output, for fp32 sums that are not finite
-  auto plain = [&](int row, int n) {
-    float s = 0.0f;
-    for (int k = 0; k < kvol; ++k) {
-      const int32_t g = gl[k * BM + row];
-      if (g < 0) continue;
-      const float* xr = reinterpret_cast<const float*>(a.in) + static_cast<int64_t>(g) * a.cin;
-      const float* wr = reinterpret_cast<const float*>(a.weight) + n * a.wn + k * a.wk;
-      for (int c = 0; c < a.cin; ++c) s = fmaf(xr[c], wr[c * a.wc], s);
-    }
-    return s;
-  };
-  // the sums: [group][64 rows][BN] fp32, 16-byte chunk c of row r at c ^ (r % 16)
-  wait_lgkm0();
-  raw_barrier();
-  {
     char* const stg = smem + (group * BM + wm * 32 + (lane & 31)) * SROW;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
@@ -370,21 +426,61 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
         const int chunk = (wn * WN + nb * 32 + 8 * q + 4 * (lane >> 5)) >> 2;
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          v[e] = acc[0][nb][4 * q + e];
-          if constexpr (kSplit)
-            v[e] = (v[e] + (acc[1][nb][4 * q + e] + acc[2][nb][4 * q + e])) * (1.0f / (kPartScale * kPartScale));
-        }
+        for (int e = 0; e < 4; ++e) v[e] = acc[0][nb][4 * q + e];
         *reinterpret_cast<f32x4*>(stg + ((chunk ^ (lane & 15)) << 4)) = v;
       }
     }
-  }
-  wait_lgkm0();
-  raw_barrier();
+    wait_lgkm0();
+    raw_barrier();
+  };
+  walk(std::false_type{});
   constexpr int E = 16 / ES, CPR = BN / E;                 // 16-byte output pieces of a row
   constexpr int TPR = kLN ? 8 : CPR;                       // threads of a row
   constexpr int PASS = (BM * TPR + THREADS - 1) / THREADS;
   static_assert(!kLN || (ES == 2 && BN == 128), "the row norm takes whole 128-channel rows");
+  // the four sums of chunk c of row r
+  auto sums = [&](int r, int c) {
+    f32x4 v = *reinterpret_cast<const f32x4*>(smem + r * SROW + ((c ^ (r & 15)) << 4));
+#pragma unroll
+    for (int g = 1; g < G; ++g) v += *reinterpret_cast<const f32x4*>(smem + (g * BM + r) * SROW + ((c ^ (r & 15)) << 4));
+    return v;
+  };
+  auto biased = [&](float y, int n) {
+    if (a.bias != nullptr) y += static_cast<float>(reinterpret_cast<const T*>(a.bias)[n]);
+    return a.act == HI3D_ACT_SILU ? silu_f32(y) : y;
+  };
+  if constexpr (kSplit) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(sbad[lane % NW] != 0) != 0, 0)) {
+      // finite sums first, an output at a time, then the others from the plain walk
+      static_assert(PASS * E <= 32, "a bit for each of a thread's outputs");
+      uint32_t later = 0;
+      auto finish = [&](bool second) {
+        for (int i = 0; i < PASS; ++i) {
+          const int r = tid / TPR + (THREADS / TPR) * i, n = n0 + tid % CPR * E;
+          const int32_t orow = r < BM ? srow[r] : -1;
+          if (orow < 0 || orow >= a.n_out || n >= a.cout) continue;
+          const f32x4 v = sums(r, tid % CPR);
+#pragma unroll
+          for (int e = 0; e < E; ++e) {
+            const uint32_t bit = 1u << (i * E + e);
+            if (!second && !(fabsf(v[e]) < INFINITY)) later |= bit;
+            if (second != ((later & bit) != 0)) continue;
+            const int64_t at = static_cast<int64_t>(orow) * a.cout + n + e;
+            float y = biased(v[e], n + e);
+            if (a.residual != nullptr) y += reinterpret_cast<const float*>(a.residual)[at];
+            reinterpret_cast<float*>(a.out)[at] = y;
+          }
+        }
+      };
+      finish(false);
+      wait_vmcnt<0>();
+      wait_lgkm0();
+      raw_barrier();
+      walk(std::true_type{});
+      finish(true);
+      return;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < PASS; ++i) {
     // (with the norm eight lanes share a row, lane g its pieces g and g + 8)
@@ -400,27 +496,9 @@ __global__ __launch_bounds__(kGroupThreads * G, 2) void conv_group_kernel(GroupC
       if (!kLN && (!live || n >= a.cout)) continue;  // cout is a multiple of E
 #pragma unroll
       for (int p = 0; p < E / 4; ++p) {
-        const int chunk = piece * (E / 4) + p;
-        f32x4 v = *reinterpret_cast<const f32x4*>(smem + r * SROW + ((chunk ^ (r & 15)) << 4));
+        const f32x4 v = sums(r, piece * (E / 4) + p);
 #pragma unroll
-        for (int g = 1; g < G; ++g)
-          v += *reinterpret_cast<const f32x4*>(smem + (g * BM + r) * SROW + ((chunk ^ (r & 15)) << 4));
-        if constexpr (kSplit) {
-          if (!(fabsf(v[0]) + fabsf(v[1]) + fabsf(v[2]) + fabsf(v[3]) < INFINITY)) {
-#pragma unroll 1
-            for (int e = 0; e < 4; ++e) {
-              const float y = plain(r, n + e);
-              v = f32x4{e == 0 ? y : v[0], e == 1 ? y : v[1], e == 2 ? y : v[2], e == 3 ? y : v[3]};
-            }
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float y = v[e];
-          if (a.bias != nullptr) y += static_cast<float>(reinterpret_cast<const T*>(a.bias)[n + 4 * p + e]);
-          if (a.act == HI3D_ACT_SILU) y = silu_f32(y);
-          h[j][4 * p + e] = static_cast<T>(y);
-        }
+        for (int e = 0; e < 4; ++e) h[j][4 * p + e] = static_cast<T>(biased(v[e], n + 4 * p + e));
       }
     }
     if constexpr (kLN) {
@@ -556,10 +634,6 @@ int hi3d_gather_conv_f32(const float* in, int64_t n_in, int32_t cin, const float
   a.cin = cin;
   a.packed = static_cast<const char*>(workspace);
   a.col_blocks = col_blocks(cout);
-  a.weight = reinterpret_cast<const char*>(weight);
-  a.wn = stride_out;
-  a.wk = stride_offset;
-  a.wc = stride_in;
   a.bias = reinterpret_cast<const char*>(bias);
   a.cout = cout;
   a.kvol = kvol;
@@ -573,14 +647,16 @@ int hi3d_gather_conv_f32(const float* in, int64_t n_in, int32_t cin, const float
   hipLaunchKernelGGL(split_weight_kernel, dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0, s, weight, stride_out,
                      stride_offset, stride_in, vec, cout, cin, a.col_blocks, total, static_cast<char*>(workspace));
   HI3D_LAUNCH_CHECK();
-  // Shapes, against the fp32 MFMA kernels (one box, 3^3 maps): at most one 64 x 64 tile a
-  // CU runs four offset groups a workgroup (3,000 voxels C256: 465 -> 93 us, one group
-  // 141; 8,000 voxels C64: 40 -> 30, one group 43; where a CU has two or three tiles one
-  // group is faster, 20,000 voxels C128: 120 with four, 107 with one). Whole 128-channel
-  // tiles read each gathered row once per 128 channels (327,581 voxels C128: 1307 ->
-  // 805 us, 64-channel tiles 870, 128-row tiles with half the weight reads 808); the
-  // others two stages in 48 KB, so that three workgroups share a CU (45,128 voxels C64:
-  // 78 -> 61 us, three slots and two workgroups 84).
+  // Shapes, against the fp32 MFMA kernels (one box, 3^3 maps, with the weight's split): at
+  // most one 64 x 64 tile a CU runs four offset groups a workgroup (3,000 voxels C256: 463 ->
+  // 102 us, 8,000 voxels C64: 41 -> 31). Whole 128-channel tiles read each gathered row once
+  // per 128 channels (327,581 voxels C128: 1362 -> 814 us; 20,000 voxels 236 -> 131); the
+  // others two stages in 48 KB, so that three workgroups share a CU (45,128 voxels C64: 87 ->
+  // 71 us). The alternatives, timed before the parts were scaled and summed by size: one
+  // group for the two small sets 141 and 43 us for 93 and 30 with four, four groups for 20,000
+  // voxels 120 for 107 (a CU with two or three tiles); 64-channel tiles for C128 870 us for
+  // 805, 128-row tiles with half the weight reads 808; three slots and two workgroups for
+  // C64 84 us for 61.
   if (ceil_div(n_out, 64) * ceil_div(cout, 64) <= compute_units()) return launch_group<float, 64, 1, 2, 4>(a, s);
   if (cout % 128 == 0) return launch_group<float, 128, 2, 2, 1>(a, s);
   return launch_group<float, 64, 2, 2, 1>(a, s);

@@ -301,9 +301,10 @@ int hi3d_gather_conv_f32_workspace(int32_t cin, int32_t cout, int32_t kvol, int6
 /* hi3d_gather_conv in fp32 on the bf16 matrix cores: each operand as the sum of three
  * bf16 values, six of the nine products, fp32 accumulation. The error against 64-bit sums
  * is that of fp32 sums, down to subnormal values; sums that are not finite, or of values
- * too large to scale, are formed in plain fp32. The weight is read through
- * its element strides (output channel, offset, input channel; a dense one 16-byte aligned) and its parts are laid out in the workspace, 16-byte aligned and the
- * call's own until it has run. */
+ * too large to scale, are formed on the fp32 matrix cores. The weight is read through its
+ * element strides (output channel, offset, input channel; a dense one 16-byte aligned)
+ * and its parts are laid out in the workspace, 16-byte aligned and the call's own until
+ * it has run. */
 int hi3d_gather_conv_f32(const float* in_dev, int64_t n_in, int32_t cin, const float* weight_dev,
                          int64_t stride_out, int64_t stride_offset, int64_t stride_in,
                          const float* bias_dev, int32_t cout, int32_t kvol, const int32_t* rows_dev,

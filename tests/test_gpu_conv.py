@@ -409,6 +409,67 @@ def test_fp32_split_kernel_not_finite(cuda):
     assert np.abs(y[fine] - ref[fine]).max() <= 1e-5 * np.sqrt((ref[fine] ** 2).mean())
 
 
+@pytest.mark.parametrize("cin,cout,side,density", [(64, 64, 20, 0.3), (128, 128, 40, 0.2), (96, 36, 44, 0.1)])
+def test_fp32_split_kernel_diverged(cuda, cin, cout, side, density):
+    """Many rows of NaN, infinite and very large features, infinite and very large weights
+    at offsets that rows lack, into the residual's own buffer, in every tile shape: outputs
+    that meet them as the fp32 sums give them, the others the bits that they have without
+    them, and the call at most ten times as long (plain sums of one output after another
+    took over a hundred)."""
+    from hi3d_amd import conv, kmap
+
+    rng = np.random.default_rng(side)
+    idx = _rand_indices(rng, side, density)
+    n = len(idx)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    plan, table = km.plan(), km.table.cpu().numpy()
+    x, w, b = _case(rng, n, cin, cout, torch.float32)
+    r = torch.as_tensor(rng.standard_normal((n, cout), dtype=np.float32))
+    clean = conv.conv(x.to(cuda), plan, w.to(cuda), b.to(cuda), residual=r.to(cuda))
+    hit = np.zeros(n + 1, bool)
+    odd = rng.permutation(n)[: n // 8]
+    hit[odd] = True
+    x2, w2 = x.clone(), w.clone()
+    x2[odd, 3] = torch.as_tensor(rng.choice([np.nan, np.inf, -np.inf, 3e37, -2e36], len(odd)).astype(np.float32))
+    w2[1, 0, 2], w2[2, 5, 0], w2[3, 26, cin - 1] = np.inf, 3e36, np.nan
+    out = r.to(cuda)
+    y = conv.conv(x2.to(cuda), plan, w2.to(cuda), b.to(cuda), residual=out, out=out)
+    assert y.data_ptr() == out.data_ptr()
+    y = y.cpu().numpy()
+    xp = np.concatenate([x2.double().numpy(), np.zeros((1, cin))])
+    with np.errstate(all="ignore"):
+        ref = b.double().numpy() + r.double().numpy()
+        terms = np.abs(ref)
+        for k in range(27):
+            to = np.nonzero(table[:, k] < n)[0]
+            for c in range(cout):
+                # one product at a time: a matrix product may form inf - inf in another order
+                p = xp[table[to, k]] * w2[c, k].double().numpy()
+                ref[to, c] += p.sum(1)
+                terms[to, c] += np.abs(p).sum(1)
+    touched = hit[table].any(1)
+    same = ~touched[:, None] & ~np.isin(np.arange(cout), [1, 2, 3])
+    assert same.sum() > 0 and np.array_equal(y[same], clean.cpu().numpy()[same])
+    assert np.array_equal(np.isnan(y), np.isnan(ref))
+    assert np.array_equal(y[np.isinf(ref)], ref[np.isinf(ref)].astype(np.float32))
+    f = np.isfinite(ref)  # half an ulp of the terms' sum at most for each addition
+    assert (np.abs(y[f] - ref[f]) <= 2.0 ** -24 * (27 * cin + 2) * terms[f]).all()
+
+    def us(xd, wd):
+        a, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = float("inf")
+        for _ in range(3):
+            a.record()
+            conv.conv(xd, plan, wd, None)
+            e.record()
+            e.synchronize()
+            best = min(best, a.elapsed_time(e))
+        return best
+
+    xd, wd = x.to(cuda), w.to(cuda)
+    assert us(torch.full_like(xd, float("nan")), wd) <= 10 * us(xd, wd)
+
+
 @pytest.mark.parametrize("dtype,mode", [
     (torch.float16, "one"), (torch.float16, "mixed"), (torch.bfloat16, "mixed"), (torch.float16, "blocks"),
 ])
