@@ -27,6 +27,7 @@
 // another 40 ms).
 //
 // Reference semantics: subm_conv (src/hi3d_mac/torch_backend/sparse_conv.py:152-195).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -551,9 +552,34 @@ namespace {
 //    24,000 voxels C128 41.5 against 48; C64, two rounds, 19.9 against 20.2).
 //  * From 256 x 256 channels on, two rounds of 64 x 128 tiles (16,000 voxels C256
 //    129 -> 73; three rounds 131 against 131).
-//  * Channel counts that the ring and wide kernels do not take, at any size (96 -> 160 on
-//    1.1M voxels 1503 -> 1094, on 33k 139 -> 63; 32 -> 32 on 1.1M 375 -> 192).
+//  * Channel counts that the ring and wide kernels do not take, where 64 x 64 tiles cost less
+//    than the pipelined kernel's, whose tiles are 256 x 64, 256 x 128 or 128 x 256
+//    (any_pays).
 enum class Group16 { kNone, kFew, kWide, kAny };
+
+// The pipelined kernel pads to its larger tiles and to whole rounds over the CUs (long rows:
+// to one; 1024 -> 128 on 66,001 voxels, two tiles more than a round, 869 us, 947 here); here an
+// input row is read again for every 64 channels. Against its 64-channel tiles these are
+// always faster (two-voxel shells of 240k and 300k voxels: 32 -> 40 1.9 times, 256 -> 40
+// 1.4, 1024 -> 64 1.1). Against the others `per` is the measured time here for an equal
+// area of output there, on two-voxel shells of 240k to 300k voxels, where rows have the most
+// neighbours: it grows with the row length (64 -> 512 1.17, 256 -> 224 1.37, 512 -> 224 1.61,
+// 1024 -> 512 1.69), and rows that are no multiple of 128 bytes, which the pipelined kernel
+// reads in halves, do better here (32 -> 224 0.72, 96 -> 224 0.93, 480 -> 224 1.51). 5 % for
+// what the measurements spread. Of 891 shapes and sizes timed both ways five of those that the
+// rule sends here lose more than 3 %, 6 % at most (64 -> 192 on 30,011 voxels 45 -> 48 us);
+// the gains are 96 -> 160 on 120,007 voxels 283 -> 148 us, 128 -> 320 on 300,007 1253 -> 997.
+// Kept there: 1024 -> 1024 on 30,011 voxels 2.44 ms against 4.31 here, 576 -> 256 on 300,007
+// 3.1 against 4.5, 64 -> 256 on 30,011 47 us against 57.
+bool any_pays(int64_t n_out, int cin, int cout, int64_t cus) {
+  if (cout <= 64) return true;
+  if (cus <= 0) return false;
+  const double per = cin % 64 == 0 ? std::min(1.1 + cin / 900.0, 1.7) : std::min(0.7 + cin / 450.0, 1.5);
+  const int64_t tiles = cout <= 128 ? ceil_div(n_out, 256) : ceil_div(n_out, 128) * ceil_div(cout, 256);
+  const int64_t there = (cin <= 512 ? ceil_div(tiles, cus) * cus : std::max(tiles, cus)) * (128 * 256);
+  const int64_t here = ceil_div(n_out, 64) * 64 * ceil_div(cout, 64) * 64;
+  return per * static_cast<double>(here) <= 0.95 * static_cast<double>(there);
+}
 
 Group16 group16(int64_t n_out, int cin, int cout, int kvol) {
   const int rb = cin * 2;
@@ -565,7 +591,7 @@ Group16 group16(int64_t n_out, int cin, int cout, int kvol) {
   if (cin % 64 == 0 && cin >= 256 && cout % 256 == 0 && row_tiles * (cout / 128) <= 2 * cus) return Group16::kWide;
   const bool ring = (rb % 64 == 0 && rb >= 256 && rb <= 1024 && cout % 128 == 0) ||
                     ((rb == 128 || rb == 256) && (cout == 64 || cout == 128));
-  return ring ? Group16::kNone : Group16::kAny;
+  return !ring && any_pays(n_out, cin, cout, cus) ? Group16::kAny : Group16::kNone;
 }
 
 template <typename T>
@@ -595,6 +621,10 @@ int group_conv16(const GroupConv& c, bool bf16, hipStream_t stream) {
 using namespace hi3d;
 
 extern "C" {
+
+int32_t hi3d_gather_conv_group16(int64_t n_out, int32_t cin, int32_t cout, int32_t kvol) {
+  return n_out > 0 && cin > 0 && cout > 0 ? static_cast<int32_t>(group16(n_out, cin, cout, kvol)) : 0;
+}
 
 int hi3d_gather_conv_f32_workspace(int32_t cin, int32_t cout, int32_t kvol, int64_t* bytes_host) {
   HI3D_REQUIRE(bytes_host != nullptr, "null pointer argument");

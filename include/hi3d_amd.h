@@ -293,6 +293,11 @@ int hi3d_gather_conv(const void* in_dev, int64_t n_in, int32_t cin, const void* 
                      const void* residual_dev, int32_t act, int32_t dtype, void* out_dev,
                      void* stream);
 
+/* Which kernel hi3d_gather_conv runs in 16 bits on the current device: 0 the ring, wide or
+ * pipelined kernels, 1 the group kernel with four offset groups a workgroup, 2 with 64 x 128
+ * tiles, 3 with 64 x 64 tiles. */
+int32_t hi3d_gather_conv_group16(int64_t n_out, int32_t cin, int32_t cout, int32_t kvol);
+
 /* Workspace bytes of hi3d_gather_conv_f32 for these shapes; 0 where it does not take
  * them (use hi3d_gather_conv): it takes Cin a multiple of 32 up to 512, Cout a multiple
  * of 4 and at most 27 offsets, with at most 8 offsets only Cin * Cout >= 32768. */

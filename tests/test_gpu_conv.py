@@ -380,6 +380,55 @@ def test_fp32_split_kernel_scales(cuda, cin, cout, side, density, ex, ew):
     assert ey <= ez, (ey, ez)
 
 
+@pytest.mark.parametrize("dtype,n,cin,cout,kernel", [
+    (torch.float16, 65_000, 64, 96, 0),      # whole rounds of the pipelined 256 x 128 tiles
+    (torch.bfloat16, 32_701, 192, 224, 0),   # of the 128 x 256 tiles
+    (torch.float16, 32_701, 640, 264, 0),    # long rows: the group kernel needs 8 columns of 64
+    (torch.bfloat16, 33_001, 64, 96, 3),     # half a round: the group kernel's 64 x 64 tiles
+    (torch.float16, 33_001, 160, 136, 3),
+    (torch.float16, 40_001, 640, 40, 3),     # up to 64 outputs at any row length
+])
+def test_16bit_other_channel_counts(cuda, dtype, n, cin, cout, kernel):
+    """Channel counts outside the ring and wide kernels', on both sides of the rule between
+    the pipelined kernel and the group kernel, ragged in rows and channels: 600 rows,
+    among them the last tiles', against float64, into memory that held NaN."""
+    from hi3d_amd import _lib, conv, kmap
+
+    assert _lib.lib().hi3d_gather_conv_group16(n, cin, cout, 27) == kernel
+    rng = np.random.default_rng(cin + cout)
+    side = 48
+    cells = rng.permutation(side ** 3)[:n]
+    idx = np.stack([0 * cells, cells // side ** 2, cells // side % side, cells % side], 1).astype(np.int32)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    plan = km.plan()
+    x, w, b = _case(rng, n, cin, cout, dtype)
+    r = torch.as_tensor(rng.standard_normal((n, cout), dtype=np.float32)).to(dtype)
+    out = torch.full((n, cout), float("nan"), dtype=dtype, device=cuda)
+    y = conv.gather_conv(x.to(cuda), plan, w.to(cuda), b.to(cuda), act="silu", residual=r.to(cuda), out=out)
+    assert not y.isnan().any()
+    last = plan.rows[plan.rows >= 0][-300:].cpu().numpy()
+    rows = np.concatenate([last, rng.permutation(n)[:300]])
+    ref = oconv.gather_conv_f64(x.float().numpy(), km.table.cpu().numpy(), w.float().numpy(), b.float().numpy(), rows=rows,
+                                act="silu", residual=r.float().numpy())
+    assert oconv.rel_err(y[torch.as_tensor(rows).to(cuda)].float().cpu().numpy(), ref) <= GATE[dtype]
+
+
+def test_16bit_group_kernel_dispatch(cuda):
+    """The group kernel takes few tiles of any channel counts, and other sets only where it
+    is the faster: not long rows into more than 64 channels, not whole tiles of the
+    pipelined kernel, not the ring and wide kernels' shapes."""
+    from hi3d_amd import _lib
+
+    which = _lib.lib().hi3d_gather_conv_group16
+    for n, cin, cout, kernel in ((1531, 128, 128, 1), (1531, 1024, 1024, 1), (1531, 96, 160, 1), (16_000, 256, 256, 2),
+                                 (17_000, 256, 256, 0), (30_011, 1024, 1024, 0), (300_007, 576, 256, 0),
+                                 (120_007, 768, 768, 0), (30_011, 64, 256, 0), (300_007, 64, 512, 0),
+                                 (120_007, 96, 160, 3), (1_100_000, 96, 160, 3), (1_100_000, 32, 32, 3),
+                                 (300_007, 128, 320, 3), (543_463, 128, 128, 0), (300_007, 200, 40, 0)):
+        assert which(n, cin, cout, 27) == kernel, (n, cin, cout)
+        assert which(n, cin, cout, 8) == 0
+
+
 def test_fp32_split_kernel_not_finite(cuda):
     """Infinities, NaN and values past bf16's largest, in the features and in the weights:
     where the sum over a row's present neighbours is infinite or NaN so is the output,
