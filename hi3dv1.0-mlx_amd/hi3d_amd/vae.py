@@ -209,9 +209,14 @@ def upsample(x: torch.Tensor, level: Level, params: dict, name: str, out: torch.
     table, parent, slot = child_neighbour_table(level.table, mask)
     w = params[f"{name}.proj.weight"]
     y = children(x, parent, slot, w, out=out if out is not None else x.dtype)
-    coords = level.coords.to(table.device, torch.int32).contiguous()
-    if tuple(coords.shape) != (int(level.table.shape[0]), 3):
-        raise ValueError(f"level coordinates must be [{int(level.table.shape[0])}, 3], got {tuple(coords.shape)}")
+    coords = level.coords.to(table.device, torch.int32)
+    if coords.dim() != 2 or int(coords.shape[1]) not in (1, 3):
+        raise ValueError(f"level coordinates must be [rows, 3], got {tuple(coords.shape)}")
+    # more rows than the table has, or none for its last parents where these keep no child
+    rows = int(coords.shape[0])
+    if rows < int(level.table.shape[0]) and parent.numel() and int(parent.max()) >= rows:
+        raise ValueError(f"level coordinates have {rows} rows, a child's parent is row {int(parent.max())}")
+    coords = coords.expand(-1, 3).contiguous()
     child_coords = torch.empty((int(parent.shape[0]), 3), dtype=torch.int32, device=table.device)
     _lib.call("hi3d_child_coords", _lib.ptr(coords), _lib.ptr(parent), _lib.ptr(slot), int(parent.shape[0]),
               _lib.ptr(child_coords), _lib.stream(table.device))

@@ -254,6 +254,33 @@ def test_upsample_with_given_and_empty_masks(cuda):
     assert y.shape == (0, c) and child.n == 0 and child.table.shape == (0, 27)
 
 
+def test_upsample_coordinate_rows(cuda):
+    """Coordinates with rows past the table's, int64 ones, a strided view, one value for
+    all axes, and none for trailing parents that keep no child give the children
+    ``coords[parent] * 2 + bits``; a parent without coordinates is refused."""
+    from hi3d_amd import vae
+
+    coords, level = _level(cuda, side=8)
+    n = len(coords)
+    rng = np.random.default_rng(10)
+    p, gp = _upsample_params(rng, 64, torch.float16)
+    gp = {k: v.to(cuda) for k, v in gp.items()}
+    x = torch.as_tensor(rng.normal(0, 1, (n, 64)).astype(np.float16)).to(cuda)
+    m = rng.random((n, 8)) < 0.3
+    m[n - 3:] = False
+    m[n - 4, 2] = True
+    mask = torch.as_tensor(m).to(cuda)
+    parent, slot = np.nonzero(m)
+    bits = np.stack([slot >> 2 & 1, slot >> 1 & 1, slot & 1], 1)
+    c = level.coords
+    longer = torch.cat([c, torch.full((5, 3), 7, dtype=c.dtype, device=cuda)])
+    for given in (c, longer, longer.long(), torch.cat([c, c], 1)[:, :3], c[:, :1], c[: n - 3]):
+        _, child, _ = vae.upsample(x, vae.Level(given, level.table), gp, "u", mask=mask)
+        assert np.array_equal(child.coords.cpu().numpy(), given.cpu().numpy()[parent] * 2 + bits)
+    with pytest.raises(ValueError, match="rows"):
+        vae.upsample(x, vae.Level(c[: n - 4], level.table), gp, "u", mask=mask)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_resnet_in_place_matches_composed(cuda, dtype):
     """The reference's in-place residual test (tests/test_mlx_kernels.py:124-150): the
