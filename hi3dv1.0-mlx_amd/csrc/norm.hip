@@ -6,6 +6,7 @@
 // 95-102; src/hi3d_mac/mlx_backend/transformer.py:548-549, 570-571, 575-577), the res-block modulation
 // (src/sparc3d/models/transformers/sparc3d_transformer.py:132-144,
 // src/hi3d_mac/mlx_backend/transformer.py:413-424).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -347,54 +348,57 @@ __global__ __launch_bounds__(256) void ln_quant_kernel(const _Float16* __restric
   }
 }
 
-// One wave per output feature and batch element (blockIdx.y): y = W . cond' + b in fp32,
-// then the fp16 (1 + scale) and shift halves. Parameters and cond in their own types
-// (16-bit values convert exactly); a lane's loads go out eight at a time, its sum stays in
-// column order.
+// One wave per output feature and batch element (blockIdx.y, and every gridDim.y-th after
+// it: a grid has at most 65535 rows): y = W . cond' + b in fp32, then the fp16 (1 + scale)
+// and shift halves. Parameters and cond in their own types (16-bit values convert exactly);
+// a lane's loads go out eight at a time, its sum stays in column order.
 template <typename W, typename C>
 __global__ __launch_bounds__(256) void adaln_kernel(const W* __restrict__ w, const W* __restrict__ b,
-                                                    const C* __restrict__ cond, int n_out, int n_in, int apply_silu,
-                                                    _Float16* __restrict__ scale1p, _Float16* __restrict__ shift) {
+                                                    const C* __restrict__ cond, int batches, int n_out, int n_in,
+                                                    int apply_silu, _Float16* __restrict__ scale1p,
+                                                    _Float16* __restrict__ shift) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (j >= n_out) return;
   const W* wr = w + static_cast<int64_t>(j) * n_in;
-  const C* cr = cond + static_cast<int64_t>(blockIdx.y) * n_in;
-  float acc = 0.0f;
-  for (int i0 = lane; i0 < n_in; i0 += 64 * 8) {
-    float wv[8], cv[8];
+  for (int64_t batch = blockIdx.y; batch < batches; batch += gridDim.y) {
+    const C* cr = cond + batch * n_in;
+    float acc = 0.0f;
+    for (int i0 = lane; i0 < n_in; i0 += 64 * 8) {
+      float wv[8], cv[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int i = i0 + 64 * u < n_in ? i0 + 64 * u : i0;
-      wv[u] = static_cast<float>(wr[i]);
-      cv[u] = static_cast<float>(cr[i]);
+      for (int u = 0; u < 8; ++u) {
+        const int i = i0 + 64 * u < n_in ? i0 + 64 * u : i0;
+        wv[u] = static_cast<float>(wr[i]);
+        cv[u] = static_cast<float>(cr[i]);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        float ci = cv[u];
+        if (apply_silu) ci = ci / (1.0f + expf(-ci));
+        if (i0 + 64 * u < n_in) acc += wv[u] * ci;
+      }
     }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      float ci = cv[u];
-      if (apply_silu) ci = ci / (1.0f + expf(-ci));
-      if (i0 + 64 * u < n_in) acc += wv[u] * ci;
+    for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
+    if (lane == 0) {
+      const float y = acc + (b != nullptr ? static_cast<float>(b[j]) : 0.0f);
+      const int half = n_out / 2;
+      const _Float16 yh = static_cast<_Float16>(y);
+      if (j < half) scale1p[batch * half + j] = static_cast<_Float16>(1.0f + static_cast<float>(yh));
+      else shift[batch * half + j - half] = yh;
     }
   }
-  for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
-  if (lane != 0) return;
-  const float y = acc + (b != nullptr ? static_cast<float>(b[j]) : 0.0f);
-  const int half = n_out / 2;
-  const _Float16 yh = static_cast<_Float16>(y);
-  const int64_t row = static_cast<int64_t>(blockIdx.y) * half;
-  if (j < half) scale1p[row + j] = static_cast<_Float16>(1.0f + static_cast<float>(yh));
-  else shift[row + j - half] = yh;
 }
 
 template <typename W>
 void launch_adaln(const void* w, const void* b, const void* cond, int cond_dtype, int batches, int n_out, int n_in,
                   int apply_silu, _Float16* scale1p, _Float16* shift, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4)), static_cast<unsigned>(batches));
+  const dim3 grid(static_cast<unsigned>(ceil_div(n_out, 4)), static_cast<unsigned>(std::min(batches, 65535)));
   auto launch = [&](auto* c) {
     using C = std::remove_const_t<std::remove_pointer_t<decltype(c)>>;
     hipLaunchKernelGGL((adaln_kernel<W, C>), grid, dim3(256), 0, stream, static_cast<const W*>(w), static_cast<const W*>(b),
-                       c, n_out, n_in, apply_silu, scale1p, shift);
+                       c, batches, n_out, n_in, apply_silu, scale1p, shift);
   };
   if (cond_dtype == HI3D_F16) launch(static_cast<const _Float16*>(cond));
   else if (cond_dtype == HI3D_BF16) launch(static_cast<const __bf16*>(cond));
@@ -563,7 +567,7 @@ int hi3d_adaln_modulation(const void* w, const void* b, int32_t param_dtype, con
                           void* stream_) {
   hipStream_t stream = as_stream(stream_);
   HI3D_REQUIRE(n_out > 0 && n_out % 2 == 0 && n_in > 0, "n_out must be even and positive, n_in positive");
-  HI3D_REQUIRE(batches >= 0 && batches <= 65535, "batches must be 0..65535 (got %d)", batches);
+  HI3D_REQUIRE(batches >= 0, "batches must be non-negative (got %d)", batches);
   for (const int32_t d : {param_dtype, cond_dtype})
     HI3D_REQUIRE(d == HI3D_F32 || d == HI3D_F16 || d == HI3D_BF16, "unsupported dtype %d", d);
   if (batches == 0) return HI3D_OK;

@@ -105,6 +105,18 @@ def test_adaln_modulation_equals_projection_of_each_row(cuda, wdt, cdt, batches,
                 assert torch.equal(s1p[i], ws) and torch.equal(sh[i], wh)
 
 
+def test_adaln_modulation_many_batch_elements(cuda):
+    """More batch elements than a grid has rows: each the projection of its own row, exactly
+    (two weights that are powers of two, small whole conditions)."""
+    from hi3d_amd import kernels
+
+    batches = 2 * 65535 + 3
+    cond = torch.arange(batches, dtype=torch.int32, device=cuda).remainder(1021).float()[:, None]
+    w = torch.tensor([[2.0], [0.5]], device=cuda)
+    s1p, sh = kernels.adaln_modulation(w, torch.tensor([1.0, -1.0], device=cuda), cond)
+    assert torch.equal(s1p, (2 * cond + 2).half()) and torch.equal(sh, (0.5 * cond - 1).half())
+
+
 @pytest.mark.parametrize("c", [32, 128, 256, 2112, 20])
 def test_layer_norm_fp16_parameters(cuda, c):
     """fp16 weight and bias as they are (aligned, or in a view that is not): the bits of
