@@ -75,6 +75,8 @@ def adaln_projection(
     if c.numel() != n_in:
         raise ValueError(f"cond must have {n_in} entries")
     b = None if bias is None else bias.to(torch.float32).reshape(-1).contiguous()
+    if b is not None and b.numel() < n_out:
+        raise ValueError(f"bias has {b.numel()} entries for {n_out} features")
     scale1p = torch.empty(n_out // 2, dtype=torch.float16, device=device)
     shift = torch.empty(n_out // 2, dtype=torch.float16, device=device)
     _lib.call(
@@ -102,6 +104,8 @@ def adaln_modulation(
         raise ValueError("the projection must produce an even number of features")
     if c.dim() != 2 or int(c.shape[1]) != n_in:
         raise ValueError(f"cond must have {n_in} entries")
+    if b is not None and b.numel() < n_out:
+        raise ValueError(f"bias has {b.numel()} entries for {n_out} features")
     batches = int(c.shape[0])
     scale1p = torch.empty((batches, n_out // 2), dtype=torch.float16, device=device)
     shift = torch.empty((batches, n_out // 2), dtype=torch.float16, device=device)

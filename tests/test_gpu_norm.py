@@ -117,6 +117,18 @@ def test_adaln_modulation_many_batch_elements(cuda):
     assert torch.equal(s1p, (2 * cond + 2).half()) and torch.equal(sh, (0.5 * cond - 1).half())
 
 
+def test_adaln_refuses_a_short_bias(cuda):
+    from hi3d_amd import kernels
+
+    w, bias = torch.zeros((8, 4), device=cuda), torch.ones(9, device=cuda)
+    for f, cond in ((kernels.adaln_projection, torch.zeros(4, device=cuda)),
+                    (kernels.adaln_modulation, torch.zeros((2, 4), device=cuda))):
+        for b in (bias[:7], bias[:0]):
+            with pytest.raises(ValueError, match="bias has"):
+                f(w, b, cond)
+        assert (f(w, bias, cond)[0] == 2).all()  # entries past the features are not used
+
+
 @pytest.mark.parametrize("c", [32, 128, 256, 2112, 20])
 def test_layer_norm_fp16_parameters(cuda, c):
     """fp16 weight and bias as they are (aligned, or in a view that is not): the bits of
