@@ -458,8 +458,8 @@ __global__ __launch_bounds__(256, 1) void w8a8_gemm_kernel(const int8_t* __restr
   }
 }
 
-// Few tiles: 16 waves share a BM x BN tile in G groups of WM x WN waves, group g taking the
-// K stages s = g mod G, each through its own ring of NS stages of 128 bytes of K; the
+// Few tiles: G groups of WM x WN waves share a BM x BN tile, group g taking the K stages
+// s = g mod G, each through its own ring of NS stages of KB bytes of K; the
 // groups' int32 sums meet in LDS (exact in any order). A launch whose 256 x 256 tiles
 // leave CUs idle spends its time in one tile's chain of K stages: smaller tiles fill the
 // CUs and the groups shorten the chain.
@@ -1601,11 +1601,12 @@ int pp_groups(int64_t mt, int nt, int k) {
 // 1030 x 8448 x 2112 went 71 -> 42 us, 16 x 8448 x 2112 66 -> 16, 500 x 2112 x 6336 36 -> 18.
 // What bounds the 128 x 128 tile: LDS traffic, 80 KB per 128 bytes of K against 512
 // cycles of MFMA.
-enum class FewTile { kNone, k64, k128x64, k128 };
+enum class GemmPath : int32_t { kTile, kFew64, kFew128x64, kFew128, kPingPongList, kPingPong, kList };
 
-FewTile few_tile(int64_t m, int n, int k, int64_t tiles256) {
+// kTile: none of them.
+GemmPath few_path(int64_t m, int n, int k, int64_t tiles256) {
   const int64_t cus = compute_units();
-  if (cus <= 0 || tiles256 > cus) return FewTile::kNone;
+  if (k % 64 != 0 || n % 8 != 0 || cus <= 0 || tiles256 > cus) return GemmPath::kTile;
   auto time = [&](int bm, int bn, double a, double b) {
     return static_cast<double>(ceil_div(ceil_div(m, bm) * ceil_div(n, bn), cus)) * (a + b * k);
   };
@@ -1613,8 +1614,31 @@ FewTile few_tile(int64_t m, int n, int k, int64_t tiles256) {
   const double load = static_cast<double>(tiles256) / static_cast<double>(cus);
   const double t256 = 9.0 + 7.4e-3 * static_cast<double>(align_up(k, 256)) + 9.0 * load;
   const double least = std::min(t64, std::min(t128x64, t128));
-  if (least >= t256) return FewTile::kNone;
-  return least == t64 ? FewTile::k64 : least == t128x64 ? FewTile::k128x64 : FewTile::k128;
+  if (least >= t256) return GemmPath::kTile;
+  return least == t64 ? GemmPath::kFew64 : least == t128x64 ? GemmPath::kFew128x64 : GemmPath::kFew128;
+}
+
+// The kernel of a GEMM; acc: its int32 sums are stored too, aligned: the scales and the bias
+// are 4-byte and acc_out is 16-byte aligned.
+//  * Few 256 x 256 tiles: few_path.
+//  * kPingPongList, the ping-pong kernel over lists of tiles: K a multiple of 64 from 512 on
+//    with n % 8 == 0 (up to three stages of zeros where K is not a multiple of 256, still
+//    faster than the 4-wave kernels: 20011 x 2112 x 6336 342 -> 311 us, 20011 x 704 x 4096
+//    104 -> 84, and 95 -> 83 us at K 576, where a quarter of the stages are zeros) and 32-bit
+//    byte offsets within a tile of the output and of acc_out.
+//  * kPingPong, one tile a workgroup: a multiple of 256 that the lists do not take (K = 256,
+//    or offsets past 32 bits).
+//  * kList, the 4-wave kernel over lists of tiles: K of 256 to 448 at whole tiles' sizes.
+//  * kTile: the rest.
+GemmPath gemm_path(int64_t m, int n, int k, bool acc, bool aligned) {
+  const int64_t mtiles = ceil_div(m, kGemmBM), blocks = mtiles * ceil_div(n, kGemmBN);
+  if (const GemmPath few = few_path(m, n, k, blocks); few != GemmPath::kTile) return few;
+  if (k % 64 != 0 || n % 8 != 0 || !aligned) return GemmPath::kTile;
+  const bool k31 = static_cast<int64_t>(k) * 256 < (int64_t(1) << 31);
+  if (k >= 512 && k31 && m < (int64_t(1) << 29) && static_cast<int64_t>(n) * (acc ? 1024 : 512) < (int64_t(1) << 31) - 4096)
+    return GemmPath::kPingPongList;
+  if (k % 256 == 0 && k31) return GemmPath::kPingPong;
+  return k >= 4 * 64 && k < 8 * 64 && m >= kGemmBM && n >= kGemmBN ? GemmPath::kList : GemmPath::kTile;
 }
 
 template <int BM, int BN, int WM, int WN, int NS, int G, int KB>
@@ -1674,6 +1698,10 @@ int hi3d_w8a8_quantize(const void* x, int64_t m, int32_t k, const float* signs, 
   return HI3D_OK;
 }
 
+int32_t hi3d_w8a8_gemm_kernel(int64_t m, int32_t n, int32_t k, int32_t with_acc) {
+  return m > 0 && n > 0 && k > 0 ? static_cast<int32_t>(gemm_path(m, n, k, with_acc != 0, true)) : 0;
+}
+
 int hi3d_w8a8_gemm(const int8_t* q, const float* sa, const int8_t* w, const float* sw, const void* bias, int64_t m,
                    int32_t n, int32_t k, void* out, int32_t* acc_out, void* stream_) {
   hipStream_t stream = as_stream(stream_);
@@ -1689,77 +1717,43 @@ int hi3d_w8a8_gemm(const int8_t* q, const float* sa, const int8_t* w, const floa
   HI3D_REQUIRE(blocks < (int64_t(1) << 31), "problem too large");
   const _Float16* b = static_cast<const _Float16*>(bias);
   _Float16* o = static_cast<_Float16*>(out);
-  if (k % 64 == 0 && n % 8 == 0) {
-    const FewTile t = few_tile(m, n, k, blocks);
-    if (t != FewTile::kNone) {
-      if (t == FewTile::k64) launch_few<64, 64, 2, 2, 2, 4, 128>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
-      else if (t == FewTile::k128x64) launch_few<128, 64, 2, 2, 3, 4, 64>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
-      else launch_few<128, 128, 2, 2, 3, 3, 64>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
-      HI3D_LAUNCH_CHECK();
-      return HI3D_OK;
-    }
+  const bool aligned = ((reinterpret_cast<uintptr_t>(sa) | reinterpret_cast<uintptr_t>(sw) |
+                         reinterpret_cast<uintptr_t>(bias)) & 3) == 0 &&
+                       (reinterpret_cast<uintptr_t>(acc_out) & 15) == 0;
+  const GemmPath path = gemm_path(m, n, k, acc_out != nullptr, aligned);
+  if (path == GemmPath::kFew64 || path == GemmPath::kFew128x64 || path == GemmPath::kFew128) {
+    if (path == GemmPath::kFew64) launch_few<64, 64, 2, 2, 2, 4, 128>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
+    else if (path == GemmPath::kFew128x64) launch_few<128, 64, 2, 2, 3, 4, 64>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
+    else launch_few<128, 128, 2, 2, 3, 3, 64>(q, sa, w, sw, b, m, n, k, o, acc_out, stream);
+    HI3D_LAUNCH_CHECK();
+    return HI3D_OK;
   }
-  // per-lane source offsets within a 256-row tile are 32-bit
-  // The persistent ping-pong kernel takes K a multiple of 64 from 512 on with n % 8 == 0
-  // (up to three stages of zeros where K is not a multiple of 256, still faster than the
-  // 4-wave kernels: 20011 x 2112 x 6336 342 -> 311 us, 20011 x 704 x 4096 104 -> 84, and
-  // 95 -> 83 us at K 576, where a quarter of the stages are zeros)
-  // and 32-bit byte offsets within a tile of the output (and of acc_out, 16-byte aligned,
-  // whose int32 accumulators it also stores).
-  const bool aligned4 = ((reinterpret_cast<uintptr_t>(sa) | reinterpret_cast<uintptr_t>(sw) |
-                          reinterpret_cast<uintptr_t>(bias)) & 3) == 0 &&
-                        (reinterpret_cast<uintptr_t>(acc_out) & 15) == 0;
-  if (k % 64 == 0 && k >= 512 && n % 8 == 0 && static_cast<int64_t>(k) * 256 < (int64_t(1) << 31) &&
-      m < (int64_t(1) << 29) &&
-      static_cast<int64_t>(n) * (acc_out ? 1024 : 512) < (int64_t(1) << 31) - 4096 && aligned4) {
+  const int cus = compute_units();
+  if (path == GemmPath::kPingPongList || path == GemmPath::kPingPong) {
     const int gr = pp_groups(mtiles, ntiles, k);
     const int parts = 8 / gr;
     const int64_t per_xcd = static_cast<int64_t>((ntiles + gr - 1) / gr) * ((mtiles + parts - 1) / parts);
-    const int cus = compute_units();
-    HI3D_REQUIRE(cus > 0, "cannot query the compute unit count");
-    const int64_t wpx = std::min<int64_t>(per_xcd, std::max(1, cus / 8));
-    const dim3 grid(static_cast<unsigned>(wpx * 8));
-    auto launch = [&](auto* kernel) {
-      hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out, mtiles, ntiles, gr);
+    auto launch = [&](auto* kernel, int64_t workgroups) {
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(workgroups)), dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o,
+                         acc_out, mtiles, ntiles, gr);
     };
-    if (k % 256 == 0) launch(acc_out ? w8a8_gemm_pq_kernel<true, false> : w8a8_gemm_pq_kernel<false, false>);
-    else launch(acc_out ? w8a8_gemm_pq_kernel<true, true> : w8a8_gemm_pq_kernel<false, true>);
+    if (path == GemmPath::kPingPongList) {
+      HI3D_REQUIRE(cus > 0, "cannot query the compute unit count");
+      const int64_t workgroups = std::min<int64_t>(per_xcd, std::max(1, cus / 8)) * 8;
+      if (k % 256 == 0) launch(acc_out ? w8a8_gemm_pq_kernel<true, false> : w8a8_gemm_pq_kernel<false, false>, workgroups);
+      else launch(acc_out ? w8a8_gemm_pq_kernel<true, true> : w8a8_gemm_pq_kernel<false, true>, workgroups);
+    } else {
+      HI3D_REQUIRE(per_xcd * 8 < (int64_t(1) << 31), "problem too large");
+      launch(acc_out ? w8a8_gemm_pp_kernel<true> : w8a8_gemm_pp_kernel<false>, per_xcd * 8);
+    }
     HI3D_LAUNCH_CHECK();
     return HI3D_OK;
   }
-  // The ping-pong kernel takes K a multiple of 256 with n % 8 == 0 (with
-  // acc_out it also stores the int32 accumulators, 16-byte aligned).
-  if (k % 256 == 0 && n % 8 == 0 && static_cast<int64_t>(k) * 256 < (int64_t(1) << 31) &&
-      (reinterpret_cast<uintptr_t>(sa) & 3) == 0 && (reinterpret_cast<uintptr_t>(sw) & 3) == 0 &&
-      (reinterpret_cast<uintptr_t>(bias) & 3) == 0 && (reinterpret_cast<uintptr_t>(acc_out) & 15) == 0) {
-    const int gr = pp_groups(mtiles, ntiles, k);
-    const int parts = 8 / gr;
-    const int64_t per_xcd = static_cast<int64_t>((ntiles + gr - 1) / gr) * ((mtiles + parts - 1) / parts);
-    HI3D_REQUIRE(per_xcd * 8 < (int64_t(1) << 31), "problem too large");
-    const dim3 grid(static_cast<unsigned>(per_xcd * 8));
-    if (acc_out)
-      hipLaunchKernelGGL(w8a8_gemm_pp_kernel<true>, grid, dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out,
-                         mtiles, ntiles, gr);
-    else
-      hipLaunchKernelGGL(w8a8_gemm_pp_kernel<false>, grid, dim3(512), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out,
-                         mtiles, ntiles, gr);
-    HI3D_LAUNCH_CHECK();
-    return HI3D_OK;
-  }
-  // With acc_out the same kernel also stores the int32 accumulators (16-byte aligned).
-  if (k % 64 == 0 && k >= 4 * 64 && k < 8 * 64 && m >= kGemmBM && n >= kGemmBN && n % 8 == 0 &&
-      static_cast<int64_t>(kGemmBM) * k < (int64_t(1) << 32) && (reinterpret_cast<uintptr_t>(sa) & 3) == 0 &&
-      (reinterpret_cast<uintptr_t>(sw) & 3) == 0 && (reinterpret_cast<uintptr_t>(bias) & 3) == 0 &&
-      (reinterpret_cast<uintptr_t>(acc_out) & 15) == 0) {
-    const int cus = compute_units();
+  if (path == GemmPath::kList) {
     HI3D_REQUIRE(cus > 0, "cannot query the compute unit count");
-    const int64_t workers = blocks < cus ? blocks : cus;
-    if (acc_out)
-      hipLaunchKernelGGL(w8a8_gemm_persistent_kernel<true>, dim3(static_cast<unsigned>(workers)), dim3(256), 0, stream,
-                         q, sa, w, sw, b, m, n, k, o, acc_out, ntiles, blocks);
-    else
-      hipLaunchKernelGGL(w8a8_gemm_persistent_kernel<false>, dim3(static_cast<unsigned>(workers)), dim3(256), 0, stream,
-                         q, sa, w, sw, b, m, n, k, o, acc_out, ntiles, blocks);
+    hipLaunchKernelGGL(acc_out ? w8a8_gemm_persistent_kernel<true> : w8a8_gemm_persistent_kernel<false>,
+                       dim3(static_cast<unsigned>(std::min<int64_t>(blocks, cus))), dim3(256), 0, stream, q, sa, w, sw, b, m,
+                       n, k, o, acc_out, ntiles, blocks);
     HI3D_LAUNCH_CHECK();
     return HI3D_OK;
   }

@@ -489,6 +489,12 @@ int hi3d_w8a8_gemm(const int8_t* q_dev, const float* sa_dev, const int8_t* w_dev
                    const float* sw_dev, const void* bias_dev, int64_t m, int32_t n, int32_t k,
                    void* out_dev, int32_t* acc_dev, void* stream);
 
+/* Which kernel hi3d_w8a8_gemm runs on the current device (with_acc: acc_dev given; scales and
+ * bias 4-byte, acc_dev 16-byte aligned): 1, 2, 3 the K-group kernel with 64 x 64, 128 x 64 and
+ * 128 x 128 tiles, 4 the persistent ping-pong kernel, 5 the ping-pong kernel, 6 the persistent
+ * four-wave kernel, 0 the one-tile kernel. */
+int32_t hi3d_w8a8_gemm_kernel(int64_t m, int32_t n, int32_t k, int32_t with_acc);
+
 /* ------------------------------------------------- VAE GroupNorm + swish -- */
 
 /* Workspace bytes of hi3d_group_stats (per-block partial column sums). */

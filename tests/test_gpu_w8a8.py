@@ -228,13 +228,11 @@ def test_gemm_non_contiguous_operands_and_scale_checks(cuda):
                                              (600, 300, 2112, False), (200, 264, 512, True), (513, 8, 768, False),
                                              (777, 1800, 2560, True)])
 def test_gemm_full_output_bit_exact(cuda, m, n, k, with_bias):
-    """Every output bit-equal to the oracle on every fused-output path: the persistent
-    ping-pong kernel (k % 256 == 0, k >= 512, n % 8 == 0: ragged rows and channel tiles
-    through its store descriptors, one tile per workgroup or several, k = 512 and 768
-    with no middle stage loop), the ping-pong kernel (k = 256), the persistent four-wave
-    kernel (k % 64 == 0, k < 2048, m, n >= 256: its edge tiles move back to overlap their
-    neighbours) and the one-tile kernel (the rest), with and without bias; each also
-    equals its accumulator-dump variant's output."""
+    """Every output bit-equal to the oracle, with and without bias, and equal to the
+    accumulator-dump variant's output: the K-group kernel's tiles (all but two shapes, with
+    ragged rows and channel tiles), the persistent ping-pong kernel on whole tiles
+    (4096 x 4096 x 1024) and the one-tile kernel (n = 300). test_large_gemm_kernels has the
+    kernels for more 256 x 256 tiles than CUs on ragged sizes."""
     from hi3d_amd import w8a8
 
     rng = np.random.default_rng(m * 7 + n * 3 + k)
@@ -252,6 +250,50 @@ def test_gemm_full_output_bit_exact(cuda, m, n, k, with_bias):
     assert np.array_equal(got, ref), int((got != ref).sum())
     out2, _ = w8a8.gemm(dev[0], dev[1], dev[2], dev[3], bias_t, return_acc=True)
     assert torch.equal(out, out2)
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (4200, 4104, 256, 5),    # ping-pong: one tile a workgroup
+    (4200, 4104, 320, 6), (4105, 4360, 384, 6), (4200, 4104, 448, 6),  # edge tiles overlap their neighbours
+    (4200, 4104, 512, 4),    # persistent ping-pong with no middle stages
+    (4105, 4360, 768, 4), (4200, 4104, 1024, 4),
+    (4200, 4104, 1088, 4),   # 64 mod 256: three stages of zeros
+    (9000, 2120, 512, 4),    # 324 tiles on a narrow output: workgroups with one tile and with two
+    (4200, 4104, 192, 0), (4200, 4104, 272, 0), (4200, 4100, 512, 0),  # one tile a workgroup, four waves
+])
+def test_large_gemm_kernels(cuda, m, n, k, kernel):
+    """More 256 x 256 tiles than CUs, ragged in rows and channels, on every kernel for them:
+    accumulators exact and outputs bit-equal to the float32 epilogue, with and without bias
+    and accumulators."""
+    from hi3d_amd import _lib, w8a8
+
+    for acc in (0, 1):
+        assert _lib.lib().hi3d_w8a8_gemm_kernel(m, n, k, acc) == kernel
+    rng = np.random.default_rng(m + 3 * n + k)
+    q, w = rng.integers(-127, 128, (m, k), dtype=np.int8), rng.integers(-127, 128, (n, k), dtype=np.int8)
+    q[m - 1], w[n - 1] = 127, -127
+    sa, sw = rng.uniform(1e-3, 1e-2, m).astype(np.float32), rng.uniform(1e-5, 1e-4, n).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float16)
+    acc = (torch.from_numpy(q).double() @ torch.from_numpy(w).double().T).numpy().astype(np.int32)
+    args = [torch.from_numpy(t).to(cuda) for t in (q, sa, w, sw, bias)]
+    for b in (args[4], None):
+        out, got = w8a8.gemm(*args[:4], b, return_acc=True)
+        assert np.array_equal(got.cpu().numpy(), acc)
+        assert np.array_equal(out.cpu().numpy(), ow8a8.epilogue(acc, sa, sw, np.zeros(n, np.float16) if b is None else bias))
+        assert torch.equal(w8a8.gemm(*args[:4], b), out)
+
+
+def test_gemm_kernel_choice(cuda):
+    """Which kernel the shapes of the tests above take."""
+    from hi3d_amd import _lib
+
+    which = _lib.lib().hi3d_w8a8_gemm_kernel
+    for m, n, k, kernel in ((1, 8, 64, 1), (64, 1024, 8448, 1), (129, 520, 2112, 1), (897, 1032, 1088, 1),
+                            (1030, 1024, 1024, 2), (777, 1800, 2560, 2),
+                            (1030, 2112, 512, 3), (1025, 2120, 704, 3), (500, 6336, 2112, 3),
+                            (1030, 2112, 8448, 3), (2600, 1032, 1536, 3), (4096, 4096, 1024, 4), (600, 300, 2112, 0),
+                            (4200, 4104, 576, 4), (2900, 6000, 1152, 4), (65536, 4096, 1024, 4), (20011, 6336, 2112, 4)):
+        assert which(m, n, k, 0) == kernel, (m, n, k)
 
 
 def test_checkpoint_round_trip(cuda, tmp_path):
@@ -308,15 +350,17 @@ def _norm_params(rng, c, affine, modulate):
 
 
 @pytest.mark.parametrize("c,rotation", [(64, "h64"), (128, "none"), (1024, "h64"), (1024, "none"), (2112, "h64"),
-                                        (4096, "h64"), (1000, "none"), (4160, "h64")])
+                                        (4096, "h64"), (1000, "none"), (4160, "h64"), (2560, "h64"), (2568, "none"),
+                                        (3072, "h64"), (3080, "none")])
 def test_norm_quantize_bitwise_equals_norm_then_quantiser(cuda, c, rotation):
     """LayerNorm (plain, affine, modulate, both) fused with the quantiser: codes and
     scales bitwise equal to ``layer_norm_modulate`` then ``quantize_activation``, and to
     the oracle's quantiser on the norm's fp16 rows. One lane per 8 columns from 8 to 64
-    lanes per row, two to eight chunks per lane, widths that leave lanes idle (1000,
-    2112), and the composed path above 4096. Rows include all-equal rows (a zero
-    norm), rows whose modulated values overflow fp16 (an infinite scale, compared with
-    the composition only) and tiny and huge magnitudes."""
+    lanes per row, two to eight chunks per lane (five up to 2560 columns, six up to 3072),
+    widths that leave lanes idle (1000, 2112, 2568, 3080), and the composed path above
+    4096. Rows include all-equal rows (a zero norm), rows whose modulated values overflow
+    fp16 (an infinite scale, compared with the composition only) and tiny and huge
+    magnitudes."""
     from hi3d_amd import kernels, w8a8
 
     rng = np.random.default_rng(c + len(rotation))
@@ -385,7 +429,7 @@ def test_norm_linear_workload4_shape_a(cuda):
 
 @pytest.mark.parametrize("m,n,k", [
     (1, 8, 64), (63, 72, 128), (65, 64, 192), (64, 1024, 8448), (129, 520, 2112),   # 64 x 64 tiles, K = 64 mod 128
-    (1030, 1024, 1024), (897, 1032, 1088),                                         # 128 x 64
+    (1030, 1024, 1024), (897, 1032, 1088),                                         # 128 x 64, 64 x 64
     (1030, 2112, 512), (1025, 2120, 704), (500, 6336, 2112),                       # 128 x 128, three K groups
     (4200, 4104, 576), (4200, 4104, 704), (2900, 6000, 1152),                      # 256 x 256, K = 64, 192, 128 mod 256
 ])
