@@ -149,7 +149,9 @@ def test_ring_kernel_variants(cuda, dtype, cin, cout, density, act, res):
     multiple of 128, rows up to 2 KB), on 128-row tiles (fp32: four 32x32x2 MFMAs per
     fragment);
     several output-column tiles, two to sixteen K steps per offset, SiLU and residual in
-    the epilogue, and isolated voxels (tiles whose only offset is the centre)."""
+    the epilogue, and isolated voxels (tiles whose only offset is the centre). The 16-bit
+    sets are small enough for the group kernel, and fp32 but 80 -> 128 has a kernel of its
+    own: test_ring_kernels_large_sets runs the ring kernels themselves."""
     from hi3d_amd import conv, kmap
 
     rng = np.random.default_rng(cin * 7 + cout + int(density * 1000))
@@ -165,6 +167,80 @@ def test_ring_kernel_variants(cuda, dtype, cin, cout, density, act, res):
     # accumulation alone reaches 1.2-1.5e-5 of the RMS (the pipelined kernel's as well)
     gate = 2e-5 if dtype == torch.float32 and cin > 256 else GATE[dtype]
     assert oconv.rel_err(y.float().cpu().numpy(), ref) <= gate
+
+
+@pytest.mark.parametrize("dtype,n,limit,cin,cout,side,act,res", [
+    (torch.float16, 16_513, 16_384, 256, 256, 48, "silu", True),     # 256 x 256 tiles, 128-byte K steps
+    (torch.bfloat16, 16_385, 16_384, 256, 256, 160, None, False),    # one row more than the limit, isolated voxels
+    (torch.float16, 8_321, 8_192, 512, 512, 32, None, True),         # two column tiles
+    (torch.bfloat16, 4_225, 4_096, 192, 512, 24, "silu", True),
+    (torch.float16, 8_301, 8_192, 160, 256, 32, "silu", False),      # 256 x 256 tiles, 64-byte K steps
+    (torch.bfloat16, 8_193, 8_192, 160, 256, 128, None, True),
+    (torch.float16, 16_449, 16_384, 256, 128, 40, None, True),       # 256 x 128 tiles, 128-byte K steps
+    (torch.bfloat16, 16_387, 16_384, 128, 128, 160, "silu", False),
+    (torch.float16, 5_500, 5_440, 128, 384, 32, None, False),        # three column tiles
+    (torch.float16, 16_450, 16_384, 160, 128, 48, "silu", True),     # 384 x 128 tiles, 64-byte K steps
+    (torch.bfloat16, 16_385, 16_384, 224, 128, 160, None, False),
+    (torch.float16, 16_400, 16_384, 64, 64, 48, "silu", True),       # 128 x 64 tiles
+    (torch.bfloat16, 32_801, 32_768, 128, 64, 160, None, False),
+    (torch.float16, 16_385, 16_384, 64, 128, 48, None, True),        # 128 x 128 tiles
+    (torch.bfloat16, 16_513, 16_384, 64, 128, 160, "silu", False),
+])
+def test_ring_kernels_large_sets(cuda, dtype, n, limit, cin, cout, side, act, res):
+    """16-bit sets just past the most rows that the group kernel takes, so that the ring and
+    wide kernels run, ragged in rows: 600 rows, among them the last tiles', against float64,
+    into memory that held NaN, and the same bits under another tile plan."""
+    from hi3d_amd import _lib, conv, kmap
+
+    which = _lib.lib().hi3d_gather_conv_group16
+    assert which(limit, cin, cout, 27) in (1, 2) and which(n, cin, cout, 27) == 0
+    rng = np.random.default_rng(cin + 5 * cout + side)
+    cells = rng.choice(side ** 3, n, replace=False)
+    idx = np.stack([0 * cells, cells // side ** 2, cells // side % side, cells % side], 1).astype(np.int32)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    plan = km.plan()
+    x, w, b = _case(rng, n, cin, cout, dtype)
+    r = torch.as_tensor(rng.standard_normal((n, cout), dtype=np.float32)).to(dtype) if res else None
+    xd, wd, bd = x.to(cuda), w.to(cuda), b.to(cuda)
+    rd = None if r is None else r.to(cuda)
+    out = torch.full((n, cout), float("nan"), dtype=dtype, device=cuda)
+    y = conv.gather_conv(xd, plan, wd, bd, act=act, residual=rd, out=out)
+    assert not y.isnan().any()
+    rows = np.concatenate([plan.rows[plan.rows >= 0][-300:].cpu().numpy(), rng.permutation(n)[:300]])
+    ref = oconv.gather_conv_f64(x.float().numpy(), km.table.cpu().numpy(), w.float().numpy(), b.float().numpy(), rows=rows,
+                                act=act, residual=None if r is None else r.float().numpy())
+    assert oconv.rel_err(y[torch.as_tensor(rows).to(cuda)].float().cpu().numpy(), ref) <= GATE[dtype]
+    assert torch.equal(conv.gather_conv(xd, kmap.build_plan(km.table, n, window_rows=512), wd, bd, act=act, residual=rd), y)
+
+
+@pytest.mark.parametrize("cin,cout,n,side,act,res", [
+    (64, 64, 3_001, 24, "silu", True),     # 16-row blocks that skip offsets
+    (64, 64, 2_000, 100, None, False),
+    (128, 64, 2_501, 24, None, True), (64, 256, 1_300, 24, "silu", False), (256, 256, 2_049, 20, "silu", True),
+    (512, 128, 1_025, 20, None, False), (80, 128, 2_000, 20, None, True),
+])
+def test_fp32_tile_kernels(cuda, cin, cout, n, side, act, res):
+    """``hi3d_gather_conv`` in fp32 (the fp32 matrix cores; the module takes them where the
+    split kernel does not take the shape), every output against float64."""
+    from hi3d_amd import _lib, conv, kmap
+
+    rng = np.random.default_rng(cin + 3 * cout + side)
+    cells = rng.choice(side ** 3, n, replace=False)
+    idx = np.stack([0 * cells, cells // side ** 2, cells // side % side, cells % side], 1).astype(np.int32)
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
+    plan = km.plan()
+    x, w, b = _case(rng, n, cin, cout, torch.float32)
+    r = torch.as_tensor(rng.standard_normal((n, cout), dtype=np.float32)) if res else None
+    xd, wd, bd = x.to(cuda), w.to(cuda), b.to(cuda)
+    rd = None if r is None else r.to(cuda)
+    y = torch.full((n, cout), float("nan"), device=cuda)
+    _lib.call("hi3d_gather_conv", _lib.ptr(xd), n, cin, _lib.ptr(wd), _lib.ptr(bd), cout, 27, _lib.ptr(plan.rows),
+              _lib.ptr(plan.gidx), _lib.ptr(plan.tile_mask), n, _lib.ptr(rd), conv.ACTIVATIONS[act],
+              _lib.DTYPES[torch.float32], _lib.ptr(y), _lib.stream(xd.device))
+    ref = oconv.gather_conv_f64(x.numpy(), km.table.cpu().numpy(), w.numpy(), b.numpy(), act=act,
+                                residual=None if r is None else r.numpy())
+    # 2e-5 above 256 input channels: see test_ring_kernel_variants
+    assert oconv.rel_err(y.cpu().numpy(), ref) <= (2e-5 if cin > 256 else GATE[torch.float32])
 
 
 def test_halo_plan_resolves_the_table(cuda):
@@ -581,18 +657,21 @@ def test_plan_choice_does_not_change_results(cuda):
     assert oconv.rel_err(halo_outs[0].float().cpu().numpy(), outs[0].float().cpu().numpy().astype(np.float64)) <= 1e-2
 
 
+@pytest.mark.parametrize("side,radius,kernel", [(96, 38.0, 0), (64, 27.0, 2)])
 @pytest.mark.parametrize("dtype,act,res", [(torch.float16, None, False), (torch.float16, "silu", True),
                                            (torch.bfloat16, "silu", False)])
-def test_wide2_offset_skips_are_exact(cuda, dtype, act, res):
+def test_wide2_offset_skips_are_exact(cuda, dtype, act, res, side, radius, kernel):
     """The 256 x 256 kernel's waves skip the MFMAs of offsets that none of their 64 rows
     has. On a sphere shell (structured masks, so many 64-row blocks lack offsets of their
     256-row tile) the output is bitwise the same under plans that skip different
-    (block, offset) pairs, and within the fp16 gate of float64."""
-    from hi3d_amd import conv, kmap, workloads
+    (block, offset) pairs, and within the fp16 gate of float64. The smaller shell runs the
+    group kernel's 64 x 128 tiles, whose waves skip by 32 rows."""
+    from hi3d_amd import _lib, conv, kmap, workloads
 
     rng = np.random.default_rng(31)
-    idx = workloads.sphere_shell(64, 27.0, seed=3)
-    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [64] * 3, 1)
+    idx = workloads.sphere_shell(side, radius, seed=3)
+    assert _lib.lib().hi3d_gather_conv_group16(len(idx), 256, 256, 27) == kernel
+    km = kmap.build_kernel_map(torch.as_tensor(idx).to(cuda), [side] * 3, 1)
     x, w, b = _case(rng, len(idx), 256, 256, dtype)
     r = torch.as_tensor(rng.standard_normal((len(idx), 256), dtype=np.float32)).to(dtype) if res else None
     xd, wd, bd = x.to(cuda), w.to(cuda), b.to(cuda)

@@ -193,17 +193,22 @@ def test_dense_linear_refuses_unsupported_shapes(cuda):
         conv.dense_linear(x[:, :32], torch.zeros((96, 32), dtype=torch.float16, device=cuda))
 
 
-@pytest.mark.parametrize("cin,batches,side", [(256, 1, 18), (128, 3, 14), (512, 2, 12), (192, 2, 16)])
-def test_conv_ln_silu_bitwise_equals_conv_then_norm(cuda, cin, batches, side):
+@pytest.mark.parametrize("cin,batches,side,kernel", [
+    (256, 1, 18, 1), (128, 3, 14, 1), (512, 2, 12, 1), (192, 2, 16, 1),    # few tiles: the group kernel
+    (256, 1, 46, 0), (128, 3, 32, 0), (512, 2, 36, 0), (192, 2, 38, 0),    # the wide kernel
+])
+def test_conv_ln_silu_bitwise_equals_conv_then_norm(cuda, cin, batches, side, kernel):
     """conv1 with norm2, each row's batch modulation and SiLU in its epilogue against the
     convolution followed by the LayerNorm + modulate + SiLU kernel on each batch's rows:
-    bitwise equal (rows of several batch elements interleaved, so tiles mix batches)."""
-    from hi3d_amd import conv, kernels, kmap
+    bitwise equal (rows of several batch elements interleaved, so tiles mix batches), in
+    the kernels of small and of large sets."""
+    from hi3d_amd import _lib, conv, kernels, kmap
 
     rng = np.random.default_rng(cin + batches)
     idx = _indices(rng, side, 0.2, batches)
     idx = idx[rng.permutation(len(idx))]  # interleave the batch elements' rows
     n = len(idx)
+    assert _lib.lib().hi3d_gather_conv_group16(n, cin, 128, 27) == kernel
     coords = torch.as_tensor(idx).to(cuda)
     km = kmap.build_kernel_map(coords, [side] * 3, batches)
     plan = km.plan()
