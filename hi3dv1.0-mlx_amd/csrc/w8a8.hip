@@ -29,14 +29,14 @@ namespace {
 // so that a row stays in registers and a set of few rows spreads over four times the waves.
 constexpr int kQuantCols = 1024;  // columns per pass
 
-template <int NP, bool kRotate, bool kFull, bool kBlock>
+template <int NP, bool kRotate, bool kFull, bool kBlock, bool kPrefetch>
 __global__ __launch_bounds__(256) void quant_kernel(const _Float16* __restrict__ x, int64_t m, int k,
                                                     const float* __restrict__ signs, int8_t* __restrict__ q,
                                                     float* __restrict__ scale) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) float mult[];  // k multipliers when rotating
   static_assert(!kBlock || !kFull, "a wave's last pass may lie past the row");
-  constexpr bool kPrefetch = !kBlock;  // the next row's loads in flight while one is computed
+  // kPrefetch: the next row's loads in flight while one is computed
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t first = kBlock ? static_cast<int64_t>(blockIdx.x) : static_cast<int64_t>(blockIdx.x) * 4 + wave;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * (kBlock ? 1 : 4);
@@ -1649,19 +1649,29 @@ void launch_few(const int8_t* q, const float* sa, const int8_t* w, const float* 
                      dim3(64 * WM * WN * G), 0, stream, q, sa, w, sw, b, m, n, k, o, acc_out, ntiles);
 }
 
-template <int NP, bool kFull, bool kBlock>
-void launch_quant_as(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, hipStream_t stream) {
-  const int64_t most = int64_t(compute_units()) * 8;
+template <int NP, bool kFull, bool kBlock, bool kPrefetch>
+void launch_quant_as(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, int64_t most,
+                     hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(std::min<int64_t>(kBlock ? m : ceil_div(m, 4), most)));
   const size_t lds = static_cast<size_t>(k) * sizeof(float);
-  if (signs) hipLaunchKernelGGL((quant_kernel<NP, true, kFull, kBlock>), grid, dim3(256), lds, stream, x, m, k, signs, q, s);
-  else hipLaunchKernelGGL((quant_kernel<NP, false, kFull, kBlock>), grid, dim3(256), 0, stream, x, m, k, signs, q, s);
+  if (signs) hipLaunchKernelGGL((quant_kernel<NP, true, kFull, kBlock, kPrefetch>), grid, dim3(256), lds, stream, x, m, k, signs, q, s);
+  else hipLaunchKernelGGL((quant_kernel<NP, false, kFull, kBlock, kPrefetch>), grid, dim3(256), 0, stream, x, m, k, signs, q, s);
 }
 
+// A wave per row, NP passes: the row's.
 template <int NP>
-void launch_quant(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, hipStream_t stream) {
-  if (k % kQuantCols == 0) launch_quant_as<NP, true, false>(x, m, k, signs, q, s, stream);
-  else launch_quant_as<NP, false, false>(x, m, k, signs, q, s, stream);
+void launch_quant(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, int64_t most,
+                  hipStream_t stream) {
+  if (k == NP * kQuantCols) launch_quant_as<NP, true, false, true>(x, m, k, signs, q, s, most, stream);
+  else launch_quant_as<NP, false, false, true>(x, m, k, signs, q, s, most, stream);
+}
+
+// A workgroup per row, NP passes a wave.
+template <int NP>
+void launch_quant_row(const _Float16* x, int64_t m, int k, const float* signs, int8_t* q, float* s, int64_t most,
+                      hipStream_t stream) {
+  if (NP <= 2 && m >= 8 * most) launch_quant_as<NP, false, true, true>(x, m, k, signs, q, s, most, stream);
+  else launch_quant_as<NP, false, true, false>(x, m, k, signs, q, s, most, stream);
 }
 
 }  // namespace
@@ -1686,14 +1696,22 @@ int hi3d_w8a8_quantize(const void* x, int64_t m, int32_t k, const float* signs, 
   if (signs) HI3D_REQUIRE((reinterpret_cast<uintptr_t>(signs) & 15) == 0, "multipliers must be 16-byte aligned");
   const int passes = (k + kQuantCols - 1) / kQuantCols;
   // From three passes on a row per workgroup, NP passes a wave: kernel time 7.6 -> 6.5 us on
-  // 1030 x 2112, 53 -> 50 us on 20011 x 2112, 72 -> 69 us on 24000 x 4096; rows past 8192
-  // columns used to be read twice by one wave (1030 x 8448: 36 -> 14 us).
-  if (passes <= 1) launch_quant<1>(xh, m, k, signs, q, scale, stream);
-  else if (passes <= 2) launch_quant<2>(xh, m, k, signs, q, scale, stream);
-  else if (passes <= 4) launch_quant_as<1, false, true>(xh, m, k, signs, q, scale, stream);
-  else if (passes <= 8) launch_quant_as<2, false, true>(xh, m, k, signs, q, scale, stream);
-  else if (passes <= 12) launch_quant_as<3, false, true>(xh, m, k, signs, q, scale, stream);
-  else launch_quant_as<4, false, true>(xh, m, k, signs, q, scale, stream);
+  // 1030 x 2112, 53 -> 50 us on 20011 x 2112; rows past 8192 columns used to be read twice by
+  // one wave (1030 x 8448: 36 -> 14 us). With eight rows a workgroup and more the next row is
+  // loaded ahead (65536 x 8192 rotated 356 -> 332 us, 65536 x 2112 152 -> 145; with two rows a
+  // workgroup the last, useless loads cost as much, 4000 x 8192 18.4 -> 19.4). Many rows
+  // without the rotation, where the barrier of each row shows, stay with a wave each up to
+  // 4096 columns.
+  const int64_t most = int64_t(compute_units()) * 8;  // workgroups that fill the CUs
+  const bool many = signs == nullptr && m >= 2 * most;
+  if (passes <= 1) launch_quant<1>(xh, m, k, signs, q, scale, most, stream);
+  else if (passes <= 2) launch_quant<2>(xh, m, k, signs, q, scale, most, stream);
+  else if (passes == 3 && many) launch_quant<3>(xh, m, k, signs, q, scale, most, stream);
+  else if (passes == 4 && many) launch_quant<4>(xh, m, k, signs, q, scale, most, stream);
+  else if (passes <= 4) launch_quant_row<1>(xh, m, k, signs, q, scale, most, stream);
+  else if (passes <= 8) launch_quant_row<2>(xh, m, k, signs, q, scale, most, stream);
+  else if (passes <= 12) launch_quant_row<3>(xh, m, k, signs, q, scale, most, stream);
+  else launch_quant_row<4>(xh, m, k, signs, q, scale, most, stream);
   HI3D_LAUNCH_CHECK();
   return HI3D_OK;
 }

@@ -456,12 +456,14 @@ def test_few_tile_gemm(cuda, m, n, k):
     assert np.array_equal(w8a8.gemm(*args[:4], None).cpu().numpy(), plain)
 
 
-@pytest.mark.parametrize("m,k", [(1, 2112), (5, 4096), (3, 8192), (2, 8256), (7, 12352), (9000, 2112), (2, 16384)])
+@pytest.mark.parametrize("m,k", [(1, 2112), (5, 4096), (3, 8192), (2, 8256), (7, 12352), (9000, 2112), (2, 16384),
+                                 (3, 3072), (2, 5120), (5, 12288), (4099, 3072), (4099, 4096), (16389, 4096), (16391, 4160)])
 @pytest.mark.parametrize("rotation", ["h64", "none"])
 def test_wide_row_quantiser(cuda, m, k, rotation):
     """Rows of a workgroup each (more than 2048 columns): waves with no columns in their
     last pass, more rows than workgroups, zero rows and rows whose scale is not finite,
-    against the oracle's codes and scales."""
+    against the oracle's codes and scales; so many rows that the next one is loaded ahead or,
+    without the rotation, that a wave takes one: the bits of 1000 rows at a time."""
     from hi3d_amd import w8a8
 
     rng = np.random.default_rng(m + k)
@@ -477,6 +479,9 @@ def test_wide_row_quantiser(cuda, m, k, rotation):
     fine = np.isfinite(want_s)
     assert np.array_equal(s[:8].cpu().numpy()[fine], want_s[fine])
     assert np.array_equal(q[:8].cpu().numpy()[fine], want_q[fine])
+    if m > 4096:
+        parts = [w8a8.quantize_activation(torch.from_numpy(x[i:i + 1000]).to(cuda), None, rotation) for i in range(0, m, 1000)]
+        assert torch.equal(torch.cat([p[0] for p in parts]), q) and torch.equal(torch.cat([p[1] for p in parts]), s)
     # rows one at a time give the same bits as together
     for i in ([m - 1, m // 2] if m > 8 else []):
         q1, s1 = w8a8.quantize_activation(torch.from_numpy(x[i:i + 1]).to(cuda), None, rotation)
