@@ -258,7 +258,9 @@ def test_gemm_full_output_bit_exact(cuda, m, n, k, with_bias):
     (4200, 4104, 512, 4),    # persistent ping-pong with no middle stages
     (4105, 4360, 768, 4), (4200, 4104, 1024, 4),
     (4200, 4104, 1088, 4),   # 64 mod 256: three stages of zeros
-    (9000, 2120, 512, 4),    # 324 tiles on a narrow output: workgroups with one tile and with two
+    (9000, 2120, 512, 4),    # one channel group; workgroups with one tile and with two
+    (4200, 6344, 576, 4),    # four groups of 7, 7, 7 and 4 channel tiles over 9 and 8 token tiles
+    (2000, 8456, 2112, 4),   # eight groups, one of them empty and one short
     (4200, 4104, 192, 0), (4200, 4104, 272, 0), (4200, 4100, 512, 0),  # one tile a workgroup, four waves
 ])
 def test_large_gemm_kernels(cuda, m, n, k, kernel):
